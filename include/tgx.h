@@ -109,8 +109,10 @@ int tgx_ringfilter_dev(double *f, int nk, int nlon, int nlat, int ld, int order,
  * k1..k2 (0-based, inclusive) are solved. */
 
 /* scheme: TGX_SCHEME_THOMAS (thread per column, reference operation order),
- * TGX_SCHEME_PCR (one wavefront per column, cyclic reduction in registers,
- * at most 256 rows), TGX_SCHEME_AUTO (timed once per shape, cached). */
+ * TGX_SCHEME_PCR (4 to 32 lanes per column, each lane eliminating its rows in
+ * registers, cyclic reduction across the lanes; at most 256 rows; a column
+ * whose segments are badly pivoted on their own is solved in the reference
+ * order), TGX_SCHEME_AUTO (timed once per shape, cached). */
 int tgx_trsolv_dev_f64(const double *a, const double *b, const double *c, const double *f,
                        double *x, int ldk, int k1, int k2, int col0, int ncol, int scheme,
                        void *stream);
@@ -141,12 +143,14 @@ int tgx_trsolv_dev_mixed(const double *a, const double *b, const double *c, cons
                          double *x, int ldk, int k1, int k2, int col0, int ncol, int nsweep,
                          void *stream);
 
-/* 2x2 block Thomas (duv.F:830-906): a,b,c (2,2,ldk,·), f,x (2,ldk,·);
- * rows 0..nrow-1. */
+/* 2x2 block rows (duv.F:830-906): a,b,c (2,2,ldk,·), f,x (2,ldk,·);
+ * rows 0..nrow-1.  Up to 256 rows by the partitioned elimination of
+ * TGX_SCHEME_PCR, block form; beyond, thread per column in reference order. */
 int tgx_blktri2_dev_f64(const double *a, const double *b, const double *c, const double *f,
                         double *x, int ldk, int nrow, int col0, int ncol, void *stream);
 
-/* 3x3 block elimination of comp: p,q,r (3,3,ldk,·), f,x (3,ldk,·); rows 0..nrow-1. */
+/* 3x3 block elimination of comp: p,q,r (3,3,ldk,·), f,x (3,ldk,·); rows
+ * 0..nrow-1, solved as the 2x2 rows are. */
 int tgx_blktri3_dev_f64(const double *p, const double *q, const double *r, const double *f,
                         double *x, int ldk, int nrow, int col0, int ncol, void *stream);
 

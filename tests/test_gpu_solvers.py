@@ -220,3 +220,105 @@ def test_solvers_from_two_host_threads_and_two_streams(pkg):
     for got in (out, [o1, o2]):
         for (rx, ry), (gx, gy) in zip(ref, got):
             assert torch.equal(rx, gx) and torch.equal(ry, gy)
+
+
+SEG_ROWS = (1, 2, 3, 31, 32, 33, 57, 64, 65, 112, 113, 128, 129, 255, 256, 257)
+
+
+def _segment_solve(pkg, nblk, sys_, x, n, col0=0):
+    if nblk == 1:
+        return pkg.tgx.trsolv_dev(*sys_, x, 0, n - 1, scheme=2, col0=col0, ncol=x.shape[0] - col0)
+    a, b, c, f = (v[col0:] for v in sys_)
+    return (pkg.tgx.blktri2_dev if nblk == 2 else pkg.tgx.blktri3_dev)(a, b, c, f, x[col0:], n)
+
+
+@pytest.mark.parametrize("nblk", [1, 2, 3])
+def test_partitioned_solver_row_counts(pkg, oracle, nblk):
+    """Row counts at every edge of the segment sizes, column counts that leave
+    a wavefront's last columns empty, rows beyond n and the unused couplings
+    NaN (neither may be read into the solution), columns before col0
+    untouched.  Diagonally dominant rows: each of the few dozen operations
+    behind an unknown is an ulp at most, inside the block solvers' 1e-14."""
+    import torch
+    from test_oracle_solvers import to_colmajor
+    for n in SEG_ROWS:
+        for ncol, col0 in ((1, 0), (37, 0), (70, 5)):
+            rng = np.random.default_rng(1000 * n + ncol)
+            nk = n + (n + ncol) % 3
+            A = rng.uniform(-1, 1, (ncol, nk, nblk, nblk))
+            C = rng.uniform(-1, 1, (ncol, nk, nblk, nblk))
+            B = rng.uniform(-1, 1, (ncol, nk, nblk, nblk))
+            dom = np.abs(A).sum((2, 3)) + np.abs(B).sum((2, 3)) + np.abs(C).sum((2, 3))
+            B = B + np.eye(nblk) * (dom + rng.uniform(.1, 1., (ncol, nk)))[..., None, None]
+            F = rng.normal(size=(ncol, nk, nblk))
+            y = np.zeros((ncol, nk, nblk))
+            A[:, 0] = 0.
+            C[:, n - 1] = 0.
+            if nblk == 1:
+                oracle.trsolv_ng(A[..., 0, 0], B[..., 0, 0], C[..., 0, 0], F[..., 0], y[..., 0], nk, ncol, n)
+            elif nblk == 2:
+                # blktri solves rows lev0..lev1-1: one level more than the rows
+                ext = [np.concatenate([v[:, :n], v[:, :1]], axis=1) for v in (A, B, C, F)]
+                z = np.zeros((ncol, n + 1, 2))
+                oracle.blktri(*[to_colmajor(v) for v in ext[:3]], np.ascontiguousarray(ext[3]), z, 1, n + 1, 5,
+                              5 + ncol - 1, 100000)
+                y[:, :n] = z[:, :n]
+            else:
+                oracle.blktri3(to_colmajor(A), to_colmajor(B), to_colmajor(C), np.ascontiguousarray(F), y, nk, ncol, n)
+            for v in (A, B, C, F):
+                v[:, n:] = np.nan
+            A[:, 0] = np.nan if nblk < 3 else 0.
+            C[:, n - 1] = np.nan if nblk < 3 else 0.
+            sys_ = [torch_dev(to_colmajor(v) if nblk > 1 else v[..., 0, 0]) for v in (A, B, C)]
+            sys_.append(torch_dev(F if nblk > 1 else F[..., 0]))
+            x = torch.full(sys_[3].shape, -5.0, dtype=torch.float64, device="cuda")
+            print("case nblk=%d n=%d ncol=%d col0=%d" % (nblk, n, ncol, col0), flush=True)
+            _segment_solve(pkg, nblk, sys_, x, n, col0)
+            got = x.cpu().numpy().reshape(ncol, nk, nblk)
+            assert np.all(got[:, n:] == -5.0) and np.all(got[:col0] == -5.0)
+            assert relerr(got[col0:, :n], y[col0:, :n]) <= 1e-14, (n, ncol)
+
+
+@pytest.mark.parametrize("nblk", [1, 2, 3])
+@pytest.mark.parametrize("n", [24, 56, 112, 200])
+def test_partitioned_solver_bad_segments(pkg, nblk, n):
+    """Zero diagonal blocks where a segment starts: unsolvable segment by
+    segment, well conditioned as a whole and for Thomas.  The other columns of
+    the wavefront hold ordinary rows, one of them a NaN, which stays in its
+    column.  Against a dense solve; the pattern (4, ..., 4, 0) with unit
+    couplings has a condition number below 100, so 1e-12."""
+    import torch
+    ncol = 9
+    eye = np.eye(nblk)
+    B = np.tile(4. * eye, (ncol, n, 1, 1))
+    A = np.tile(eye, (ncol, n, 1, 1))
+    C = np.tile(eye, (ncol, n, 1, 1))
+    rng = np.random.default_rng(n + nblk)
+    F = rng.normal(size=(ncol, n, nblk))
+    B[2::3, 8::8] = 0.        # a multiple of every segment length
+    F[4, n // 2, 0] = np.nan
+    A[:, 0] = 0.
+    C[:, n - 1] = 0.
+    sys_ = [torch_dev(v if nblk > 1 else v[..., 0, 0]) for v in (A, B, C)] + [torch_dev(F if nblk > 1 else F[..., 0])]
+    x = torch.zeros(sys_[3].shape, dtype=torch.float64, device="cuda")
+    _segment_solve(pkg, nblk, sys_, x, n)
+    got = x.cpu().numpy().reshape(ncol, n, nblk)
+    assert np.isnan(got[4]).any()
+    for col in range(ncol):
+        if col == 4:
+            continue
+        M = np.zeros((n * nblk, n * nblk))
+        for k in range(n):
+            s = slice(k * nblk, (k + 1) * nblk)
+            M[s, s] = B[col, k]
+            if k:
+                M[s, (k - 1) * nblk:k * nblk] = A[col, k]
+            if k < n - 1:
+                M[s, (k + 1) * nblk:(k + 2) * nblk] = C[col, k]
+        assert np.linalg.cond(M) < 100.
+        ref = np.linalg.solve(M, F[col].ravel()).reshape(n, nblk)
+        assert relerr(got[col], ref) <= 1e-12, (col, relerr(got[col], ref))
+    if nblk == 1:  # solved again in the reference's order: bit for bit the Thomas scheme
+        y = torch.zeros_like(x)
+        pkg.tgx.trsolv_dev(*sys_, y, 0, n - 1, scheme=1)
+        assert torch.equal(x[2::3], y[2::3])

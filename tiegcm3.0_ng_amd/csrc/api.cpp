@@ -43,8 +43,11 @@ bool tgx_on_main_thread() { return (pid_t)syscall(SYS_gettid) == getpid(); }
 // ---- launchers (solvers.hip) -------------------------------------------------
 extern "C" int tgx_launch_thomas_f64(const double *, const double *, const double *, const double *,
                                      double *, double *, int, int, int, int, int, hipStream_t);
-extern "C" int tgx_launch_pcr(const double *, const double *, const double *, const double *,
-                              double *, int, int, int, int, int, int, int, hipStream_t);
+extern "C" int tgx_launch_mixed(const double *, const double *, const double *, const double *,
+                                double *, int, int, int, int, int, int, hipStream_t);
+// segsolve.hip
+extern "C" int tgx_launch_segment(int, const double *, const double *, const double *, const double *, double *, int,
+                                  int, int, hipStream_t);
 extern "C" int tgx_launch_blktri2_f64(const double *, const double *, const double *, const double *,
                                       double *, double *, int, int, int, int, hipStream_t);
 extern "C" int tgx_launch_ringfilter(double *, int, long, int, const long *, const int *, int, int, int,
@@ -171,7 +174,10 @@ int col_bucket(int ncol) {
 
 int run_scalar(int scheme, const double *a, const double *b, const double *c, const double *f,
                double *x, int ldk, int k1, int k2, int col0, int ncol, hipStream_t s) {
-  if (scheme == TGX_SCHEME_PCR) return tgx_launch_pcr(a, b, c, f, x, ldk, k1, k2, col0, ncol, 0, 0, s);
+  if (scheme == TGX_SCHEME_PCR) {
+    const size_t o = (size_t)col0 * ldk + k1;
+    return tgx_launch_segment(1, a + o, b + o, c + o, f + o, x + o, ldk, k2 - k1 + 1, ncol, s);
+  }
   void *w2 = nullptr;
   size_t need = sizeof(double) * (size_t)ldk * (size_t)ncol;
   if (int rc = get_scratch(need, s, &w2)) return rc;
@@ -212,6 +218,12 @@ extern "C" int tgx_autotune_choice(int ldk, int k1, int k2, int ncol) {
 }
 
 // ---- device entry points ----------------------------------------------------
+namespace {
+// Rows up to which a column stays on chip (segsolve.hip); beyond, a thread
+// per column keeps its block gammas in HBM.
+constexpr int kSegRows = 256;
+}  // namespace
+
 extern "C" int tgx_trsolv_dev_f64(const double *a, const double *b, const double *c,
                                   const double *f, double *x, int ldk, int k1, int k2, int col0,
                                   int ncol, int scheme, void *stream) {
@@ -251,7 +263,7 @@ extern "C" int tgx_trsolv_dev_mixed(const double *a, const double *b, const doub
   if (ldk <= 0 || k1 < 0 || k2 >= ldk || col0 < 0 || ncol < 0 || nsweep < 0 || nsweep > 8)
     return tgx_set_error(1, "tgx_trsolv_dev_mixed: bad arguments");
   if (k2 - k1 + 1 > 256) return tgx_set_error(1, "tgx_trsolv_dev_mixed: at most 256 rows");
-  return tgx_launch_pcr(a, b, c, f, x, ldk, k1, k2, col0, ncol, nsweep, 1, (hipStream_t)stream);
+  return tgx_launch_mixed(a, b, c, f, x, ldk, k1, k2, col0, ncol, nsweep, (hipStream_t)stream);
 }
 
 extern "C" int tgx_blktri2_dev_f64(const double *a, const double *b, const double *c,
@@ -259,6 +271,11 @@ extern "C" int tgx_blktri2_dev_f64(const double *a, const double *b, const doubl
                                    int ncol, void *stream) {
   if (ldk <= 0 || nrow < 1 || nrow > ldk || col0 < 0 || ncol < 0)
     return tgx_set_error(1, "tgx_blktri2_dev_f64: bad shape");
+  if (nrow <= kSegRows) {
+    const size_t o = (size_t)col0 * ldk;
+    return tgx_launch_segment(2, a + 4 * o, b + 4 * o, c + 4 * o, f + 2 * o, x + 2 * o, ldk, nrow, ncol,
+                              (hipStream_t)stream);
+  }
   void *gs = nullptr;
   if (int rc = get_scratch(sizeof(double) * 4 * (size_t)ldk * (size_t)(col0 + ncol), (hipStream_t)stream, &gs)) return rc;
   return tgx_launch_blktri2_f64(a, b, c, f, x, (double *)gs, ldk, nrow, col0, ncol, (hipStream_t)stream);
@@ -269,6 +286,11 @@ extern "C" int tgx_blktri3_dev_f64(const double *p, const double *q, const doubl
                                    int ncol, void *stream) {
   if (ldk <= 0 || nrow < 1 || nrow > ldk || col0 < 0 || ncol < 0)
     return tgx_set_error(1, "tgx_blktri3_dev_f64: bad shape");
+  if (nrow <= kSegRows) {
+    const size_t o = (size_t)col0 * ldk;
+    return tgx_launch_segment(3, p + 9 * o, q + 9 * o, r + 9 * o, f + 3 * o, x + 3 * o, ldk, nrow, ncol,
+                              (hipStream_t)stream);
+  }
   void *gs = nullptr;
   if (int rc = get_scratch(sizeof(double) * 9 * (size_t)ldk * (size_t)(col0 + ncol), (hipStream_t)stream, &gs)) return rc;
   return tgx_launch_blktri3_f64(p, q, r, f, x, (double *)gs, ldk, nrow, col0, ncol, (hipStream_t)stream);

@@ -11,8 +11,8 @@
 
 extern "C" int tgx_launch_thomas_f64(const double *, const double *, const double *, const double *,
                                      double *, double *, int, int, int, int, int, hipStream_t);
-extern "C" int tgx_launch_pcr(const double *, const double *, const double *, const double *,
-                              double *, int, int, int, int, int, int, int, hipStream_t);
+extern "C" int tgx_launch_segment(int, const double *, const double *, const double *, const double *, double *, int,
+                                  int, int, hipStream_t);
 
 // One copy per GPU, held until the process ends.  Only device code may name
 // it: host code uses the address hipGetSymbolAddress returns for the current
@@ -62,7 +62,10 @@ extern "C" int tgx_trsolv_dev_f64_noalloc(const double *a, const double *b, cons
     if (scheme == TGX_SCHEME_AUTO) scheme = TGX_SCHEME_THOMAS;
   }
   if (scheme == TGX_SCHEME_PCR && nrow > 256) scheme = TGX_SCHEME_THOMAS;
-  if (scheme == TGX_SCHEME_PCR) return tgx_launch_pcr(a, b, c, f, x, ldk, k1, k2, col0, ncol, 0, 0, s);
+  if (scheme == TGX_SCHEME_PCR) {
+    const size_t o = (size_t)col0 * ldk + k1;
+    return tgx_launch_segment(1, a + o, b + o, c + o, f + o, x + o, ldk, nrow, ncol, s);
+  }
   const unsigned long long need = (unsigned long long)ldk * (unsigned long long)ncol;
   if (need > (unsigned long long)TGX_NOALLOC_SCRATCH_DOUBLES)
     return tgx_set_error(TGX_ERR_ARG,

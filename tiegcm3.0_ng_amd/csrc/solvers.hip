@@ -3,12 +3,12 @@
 //   blktri              (2x2 block tridiagonal, duv.F:801-908)
 //   comp 3x3 elimination (comp_ng.F90:281-326 on pre-assembled blocks)
 //
-// Two schemes for the scalar system:
-//   * Thomas, one thread per column, in the reference's operation order
-//     (bit-compatible with the Fortran when FP contraction is off);
-//   * parallel cyclic reduction (PCR), one wavefront (or half) per column,
-//     coefficients held in registers and exchanged with cross-lane shuffles.
-// and a mixed-precision PCR: FP32 reduction, FP64 residual r = f - A x,
+// Thread per column in the reference's operation order (bit-compatible with
+// the Fortran when FP contraction is off): the scalar Thomas scheme, and block
+// columns beyond 256 rows.  segsolve.hip holds the partitioned solver the
+// other calls take.
+// Beside them a mixed-precision PCR, one wavefront (or half) per column: FP32
+// reduction in registers with cross-lane shuffles, FP64 residual r = f - A x,
 // iterative refinement sweeps that reuse the FP32 reduction multipliers.
 #include "tgx_common.h"
 
@@ -133,38 +133,6 @@ constexpr int pcr_nsteps() {
   int n = SEG * NPL, s = 0;
   while ((1 << s) < n) ++s;
   return s;
-}
-
-// FP64 PCR: the whole column in registers, coalesced loads (a column is
-// contiguous in the level-fastest layout).
-template <int SEG, int NPL>
-__global__ void __launch_bounds__(256) pcr_kfast_f64(
-    const double *__restrict__ a, const double *__restrict__ b, const double *__restrict__ c,
-    const double *__restrict__ f, double *__restrict__ x, int ldk, int k1, int k2, int col0,
-    int ncol) {
-  const int lane = threadIdx.x % SEG;
-  const int col = (blockIdx.x * blockDim.x + threadIdx.x) / SEG;
-  const bool live = col < ncol;
-  const int n = k2 - k1 + 1;
-  size_t o = (size_t)(col0 + (live ? col : 0)) * (size_t)ldk + k1;
-  PcrRows<double, SEG, NPL> R;
-#pragma unroll
-  for (int e = 0; e < NPL; ++e) {
-    int r = lane * NPL + e;
-    bool in = live && r < n;
-    R.a[e] = (in && r > 0) ? a[o + r] : 0.;
-    R.b[e] = in ? b[o + r] : 1.;
-    R.c[e] = (in && r < n - 1) ? c[o + r] : 0.;
-    R.d[e] = in ? f[o + r] : 0.;
-  }
-  constexpr int NS = pcr_nsteps<SEG, NPL>();
-#pragma unroll
-  for (int st = 0; st < NS; ++st) pcr_step<double, SEG, NPL>(R, 1 << st, lane, nullptr, nullptr);
-#pragma unroll
-  for (int e = 0; e < NPL; ++e) {
-    int r = lane * NPL + e;
-    if (live && r < n) x[o + r] = R.d[e] / R.b[e];
-  }
 }
 
 // Mixed precision: FP32 PCR reduction of the FP64 system, FP64 residual with
@@ -503,30 +471,24 @@ extern "C" int tgx_launch_thomas_f64(const double *a, const double *b, const dou
 }
 
 template <int SEG, int NPL>
-static int launch_pcr(const double *a, const double *b, const double *c, const double *f,
-                      double *x, int ldk, int k1, int k2, int col0, int ncol, int nsweep,
-                      bool mixed, hipStream_t s) {
+static int launch_mixed(const double *a, const double *b, const double *c, const double *f, double *x, int ldk, int k1,
+                        int k2, int col0, int ncol, int nsweep, hipStream_t s) {
   int cols_per_block = 256 / SEG;
   int nb = (ncol + cols_per_block - 1) / cols_per_block;
-  if (mixed)
-    hipLaunchKernelGGL((tgx::pcr_kfast_mixed<SEG, NPL>), dim3(nb), dim3(256), 0, s, a, b, c, f,
-                       x, ldk, k1, k2, col0, ncol, nsweep);
-  else
-    hipLaunchKernelGGL((tgx::pcr_kfast_f64<SEG, NPL>), dim3(nb), dim3(256), 0, s, a, b, c, f, x,
-                       ldk, k1, k2, col0, ncol);
+  hipLaunchKernelGGL((tgx::pcr_kfast_mixed<SEG, NPL>), dim3(nb), dim3(256), 0, s, a, b, c, f, x, ldk, k1, k2, col0,
+                     ncol, nsweep);
   TGX_HIP(hipGetLastError());
   return 0;
 }
 
-extern "C" int tgx_launch_pcr(const double *a, const double *b, const double *c,
-                              const double *f, double *x, int ldk, int k1, int k2, int col0,
-                              int ncol, int nsweep, int mixed, hipStream_t s) {
+extern "C" int tgx_launch_mixed(const double *a, const double *b, const double *c, const double *f, double *x, int ldk,
+                                int k1, int k2, int col0, int ncol, int nsweep, hipStream_t s) {
   if (ncol <= 0 || k2 < k1) return 0;
   int n = k2 - k1 + 1;
-  if (n <= 32) return launch_pcr<32, 1>(a, b, c, f, x, ldk, k1, k2, col0, ncol, nsweep, mixed, s);
-  if (n <= 64) return launch_pcr<64, 1>(a, b, c, f, x, ldk, k1, k2, col0, ncol, nsweep, mixed, s);
-  if (n <= 128) return launch_pcr<64, 2>(a, b, c, f, x, ldk, k1, k2, col0, ncol, nsweep, mixed, s);
-  if (n <= 256) return launch_pcr<64, 4>(a, b, c, f, x, ldk, k1, k2, col0, ncol, nsweep, mixed, s);
+  if (n <= 32) return launch_mixed<32, 1>(a, b, c, f, x, ldk, k1, k2, col0, ncol, nsweep, s);
+  if (n <= 64) return launch_mixed<64, 1>(a, b, c, f, x, ldk, k1, k2, col0, ncol, nsweep, s);
+  if (n <= 128) return launch_mixed<64, 2>(a, b, c, f, x, ldk, k1, k2, col0, ncol, nsweep, s);
+  if (n <= 256) return launch_mixed<64, 4>(a, b, c, f, x, ldk, k1, k2, col0, ncol, nsweep, s);
   return tgx_set_error(1, "PCR supports at most 256 rows per column (got %d)", n);
 }
 
