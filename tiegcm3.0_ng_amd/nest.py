@@ -224,7 +224,7 @@ class CoupledNests:
         self.graphs = []
         while True:
             graph = torch.cuda.CUDAGraph()
-            with torch.cuda.graph(graph):
+            with _step.no_collection(), torch.cuda.graph(graph):
                 self.run()
             self.graphs.append((graph, self._phases()))
             if self._phases() == start or len(self.graphs) == 2:

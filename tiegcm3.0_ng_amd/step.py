@@ -7,7 +7,9 @@ routines: oplus_ng (with its nstep_sub sub-cycles), the minor species,
 dt_ng, duv_ng and comp_o2o_ng + comp_ng, or the whole step in the
 reference's order (dynamics_ng.F90:99-233).
 """
+import contextlib
 import ctypes as C
+import gc
 
 import torch
 
@@ -91,6 +93,20 @@ _SIGS = {
 
 ROUTINES = ("oplus", "minors", "dt", "duv", "comp")
 SCHEMES = {"auto": 0, "thomas": 1, "pcr": 2}
+
+
+@contextlib.contextmanager
+def no_collection():
+    """Holds Python's cyclic garbage collector off during a graph capture: the
+    destructor of a collected CUDAGraph synchronises the device, which fails
+    while a stream is capturing and ends the process."""
+    on = gc.isenabled()
+    gc.disable()
+    try:
+        yield
+    finally:
+        if on:
+            gc.enable()
 
 
 def profile_begin(max_calls):
@@ -339,14 +355,15 @@ class NestedStep:
         self.nstep_ng = list(nstep_ng)
         self.forked = forked
         self.graph = None
-        self.order = []  # domain index of each sub-step, in launch order
+        self.order = self._order(0)  # domain index of each sub-step, in launch order
 
-        def visit(level):
-            for _ in range(self.nstep_ng[level]):
-                self.order.append(level)
-                if level + 1 < len(self.states):
-                    visit(level + 1)
-        visit(0)
+    def _order(self, level):
+        order = []
+        for _ in range(self.nstep_ng[level]):
+            order.append(level)
+            if level + 1 < len(self.states):
+                order += self._order(level + 1)
+        return order
 
     def substeps(self):
         return {i: self.order.count(i) for i in range(len(self.states))}
@@ -376,7 +393,7 @@ class NestedStep:
         self.graphs = []
         for _ in range(2 if odd else 1):   # nothing runs while capturing
             graph = torch.cuda.CUDAGraph()
-            with torch.cuda.graph(graph):
+            with no_collection(), torch.cuda.graph(graph):
                 self.run()
             self.graphs.append((graph, self._phases()))
         self._set_phases(start)             # the data is still where the warm-up left it
