@@ -482,3 +482,44 @@ def test_oplus_kept_factorisation_equals_full_assembly(pkg, name, nsub):
     torch.cuda.synchronize()
     for n in a.out:
         assert torch.equal(a.out[n], b.out[n]), n
+
+
+@pytest.mark.parametrize("shape", [(8, 6, 4), (13, 9, 5), (16, 12, 17), (31, 7, 29), (32, 8, 57), (33, 10, 64),
+                                   (47, 11, 65), (18, 9, 113), (20, 8, 128), (150, 120, 12)],
+                         ids=lambda s: "%dx%dx%d" % s)
+@pytest.mark.parametrize("glb", [False, True], ids=["nest", "global"])
+def test_block_kernels_equal_thread_per_column(pkg, monkeypatch, shape, glb):
+    """The block kernels of the Thomas scheme (16 threads per column) give every
+    output of every routine bit for bit as the thread-per-column kernels do:
+    grids whose rows end inside a block, levels at the edges of a thread's run
+    (one level, none) and of the LDS split (64/65, 128), one and several O+
+    sub-cycles, with and without N2 extrapolation above an O-dominated top, a
+    grid beyond comp's block form.  On a global grid the interior rows (the
+    others are not defined) and, for O+, the rows across the poles."""
+    import torch
+    nlon, nlat, nk = shape
+    if glb:
+        nlon = (nlon + 11) // 12 * 12
+        nlat = max(nlat, 8)
+    name = "blk%dx%dx%d" % (nlon, nlat, nk)
+    monkeypatch.setitem(pkg.synth.CONFIGS, name, (nlon, nlat, nk, 14. / (nk - 1), 10., 10., None))
+    if glb:
+        monkeypatch.setitem(pkg.tgx.RING_CHUNKS, (nlon, nlat), [3, 6, 12][:nlat // 3])
+    for nsub, n2_top in ((1, None), (3, 2e-3)):
+        g = pkg.synth.make_grid(name, nstep_sub=nsub, glb=glb, n2_top=n2_top)
+        F = pkg.synth.make_global_state(g) if glb else pkg.synth.make_state(g)
+        print("case %s glb=%d nsub=%d" % (name, glb, nsub), flush=True)
+        states = []
+        for large in ("0", "1"):
+            monkeypatch.setenv("TGX_LARGE_GRID_FORMS", large)
+            st = pkg.step.GlobalState(g, F) if glb else pkg.step.NestState(g, F, scheme="thomas")
+            st.step()
+            whole = {n: t.clone() for n, t in st.out.items()}
+            for r in pkg.step.ROUTINES:  # each routine on its own (its own sources)
+                getattr(st, r)()
+            torch.cuda.synchronize()
+            states.append((whole, st.out))
+        for a, b in zip(*states):
+            for n in a:
+                rows = slice(2, nlat + 2) if glb and n not in ("op", "op_nm") else slice(None)
+                assert torch.equal(a[n][..., rows, :], b[n][..., rows, :]), n

@@ -1,11 +1,11 @@
-// The global grid's passes around the column kernels: comp's post pass
-// after its ring filter (the time smoothing, N2 and the normalisation) on the
-// latitudes the filter reaches (the column kernels apply the post passes
-// themselves on the others, and the ring filter launch applies those of dt,
-// duv, the minor species and O+), the periodic points of the outputs
-// (mp_periodic_f3d) and the halos of an input field (mk_polelat.F,
-// mp_periodic_f4d).  Level planes as in tgx_step.h; the elementwise passes
-// take one thread per (point, level), the longitudes fastest.
+// The global grid's passes around the column kernels of the larger grids: the
+// periodic points of the outputs (mp_periodic_f3d), the rows across the poles
+// of O+ between sub-cycles, and the halos of an input field (mk_polelat.F,
+// mp_periodic_f4d).  The post passes are the column kernels', the ring filter
+// launch's and comp_post_block's; the block kernels of the smaller grids write
+// the periodic points themselves.  Level planes as in tgx_step.h; the
+// elementwise passes take one thread per (point, level), the longitudes
+// fastest.
 #include <hip/hip_runtime.h>
 
 #include "../../include/tgx.h"
@@ -15,80 +15,10 @@
 namespace tgx {
 namespace glb {
 
-constexpr double DTSMOOTH = 0.95, DTSMOOTH_DIV2 = 0.5 * (1. - DTSMOOTH);
-
 struct Dims {
   int nk, nlon, nlat, ld;
-  int nfilt;     // latitudes the ring filter reaches next to each pole
   size_t plane;  // ld * (nlat + 4)
 };
-
-// Row j of the r-th filtered latitude (r < 2 nfilt): the nfilt next to the
-// south pole, then the nfilt next to the north pole.
-__device__ __forceinline__ int filtered_row(const Dims &D, int r) {
-  return r < D.nfilt ? 2 + r : D.nlat + 2 - 2 * D.nfilt + r;
-}
-
-// comp.F:936-1022 on one column per thread: the time smoothing of the
-// filtered O2, O, He, N2 above its lowest level under 0.01 extrapolated in
-// log(N2 n) (:975-990), the floors and the normalisation.
-struct CompIO {
-  double *o2, *o1, *he, *o2nm, *o1nm, *henm;
-  const double *o2i, *o1i, *hei, *o2nmi, *o1nmi, *henmi, *xnmbar;
-  const double *zpmid;
-  double dz;
-};
-
-__global__ void __launch_bounds__(256) comp_post_kernel(Dims D, CompIO C) {
-  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (long)D.nlon * 2 * D.nfilt) return;
-  const int row = (int)(t / D.nlon);
-  const int j = filtered_row(D, row), i = 2 + (int)(t - (long)row * D.nlon);
-  const size_t c = (size_t)j * D.ld + i;
-  const int nk = D.nk;
-  const double small = 1.e-9;
-  // the lowest level with N2 < 0.01 and the level below it
-  int ktop = nk;
-  for (int k = 0; k < nk; ++k) {
-    const size_t p = (size_t)k * D.plane + c;
-    const double n2 = 1. - C.o2[p] - C.o1[p] - C.he[p];
-    if (n2 < 0.01) {
-      ktop = k;
-      break;
-    }
-  }
-  const bool extrap = ktop + 1 < nk && ktop >= 1;
-  double n2top = 0., dn2dz = 0., zmtop = 0.;
-  if (extrap) {
-    const size_t pt = (size_t)ktop * D.plane + c, pb = pt - D.plane;
-    zmtop = C.zpmid[ktop];
-    n2top = log((1. - C.o2[pt] - C.o1[pt] - C.he[pt]) * C.xnmbar[pt]);
-    const double n2top1 = log((1. - C.o2[pb] - C.o1[pb] - C.he[pb]) * C.xnmbar[pb]);
-    dn2dz = (n2top - n2top1) / C.dz;
-  }
-  for (int k = 0; k < nk; ++k) {
-    const size_t p = (size_t)k * D.plane + c;
-    const double o2 = C.o2[p], o1 = C.o1[p], he = C.he[p];
-    const double o2nm = DTSMOOTH_DIV2 * (C.o2nmi[p] + o2) + DTSMOOTH * C.o2i[p];
-    const double o1nm = DTSMOOTH_DIV2 * (C.o1nmi[p] + o1) + DTSMOOTH * C.o1i[p];
-    const double henm = DTSMOOTH_DIV2 * (C.henmi[p] + he) + DTSMOOTH * C.hei[p];
-    double n2 = 1. - o2 - o1 - he;
-    if (extrap && k > ktop) n2 = exp(n2top + dn2dz * (C.zpmid[k] - zmtop)) / C.xnmbar[p];
-    const double a = o2 > small ? o2 : small, b = o1 > small ? o1 : small;
-    const double cc = he > small ? he : small, d = n2 > small ? n2 : small;
-    const double norm = a + b + cc + d;
-    C.o2[p] = a / norm;
-    C.o1[p] = b / norm;
-    C.he[p] = cc / norm;
-    const double n2nm = 1. - o2nm - o1nm - henm;
-    const double an = o2nm > small ? o2nm : small, bn = o1nm > small ? o1nm : small;
-    const double cn = henm > small ? henm : small, dn = n2nm > small ? n2nm : small;
-    const double normn = an + bn + cn + dn;
-    C.o2nm[p] = an / normn;
-    C.o1nm[p] = bn / normn;
-    C.henm[p] = cn / normn;
-  }
-}
 
 // mp_periodic_f3d on the interior latitudes of up to eight fields: thread
 // per (periodic point, interior latitude, level, field).
@@ -157,9 +87,8 @@ __global__ void __launch_bounds__(256) halos_kernel(Dims D, double *__restrict__
 
 inline unsigned nblocks(long n) { return (unsigned)((n + 255) / 256); }
 
-Dims dims_of(const tgx_ng_grid *g, int nfilt) {
+Dims dims_of(const tgx_ng_grid *g) {
   Dims D;
-  D.nfilt = nfilt;
   D.nk = g->nk;
   D.nlon = g->nlon;
   D.nlat = g->nlat;
@@ -183,31 +112,16 @@ int periodic(const Dims &D, double *const *f, int n, int nk, hipStream_t s) {
 
 using namespace tgx::glb;
 
-// What remains of a global routine after its ring filter launch
-// (step_api.cpp), which has applied the post pass of dt, duv, the minor
-// species and O+ on the filtered latitudes: which 0 dt, 1 duv, 2 minor
-// species N2D and Ar, 3 minor species NO and N4S, 4 O+ sub-step (op_in,
-// nm_in: the sub-step's inputs, op_o, nm_o: its outputs, whose rows across
-// the poles take those of in->op / in->op_nm), 5 comp (its post pass on the
-// nfilt filtered latitudes next to each pole, which needs whole columns).
-// Then the periodic points of the outputs on every interior latitude.
-extern "C" int tgx_glb_post(int which, int nfilt, const tgx_ng_grid *g, const tgx_ng_fields *in,
-                            const tgx_ng_out *out, const double *op_in, const double *nm_in, double *op_o,
-                            double *nm_o, hipStream_t s) {
+// What remains of a global routine's larger-grid form after its post pass
+// (the column kernel's, the ring filter launch's and, for comp,
+// comp_post_block's): which 0 dt, 1 duv, 2 minor species N2D and Ar, 3 minor
+// species NO and N4S, 4 O+ sub-step (op_o, nm_o: its outputs, whose rows
+// across the poles take those of in->op / in->op_nm), 5 comp.  The periodic
+// points of the outputs on every interior latitude.
+extern "C" int tgx_glb_post(int which, const tgx_ng_grid *g, const tgx_ng_fields *in, const tgx_ng_out *out,
+                            double *op_o, double *nm_o, hipStream_t s) {
   if (which < 0 || which > 5) return tgx_set_error(TGX_ERR_ARG, "tgx_glb_post: unknown pass %d", which);
-  const Dims D = dims_of(g, nfilt);
-  if (which == 5 && nfilt > 0) {
-    CompIO C;
-    C.o2 = out->o2; C.o1 = out->o1; C.he = out->he;
-    C.o2nm = out->o2_nm; C.o1nm = out->o1_nm; C.henm = out->he_nm;
-    C.o2i = in->o2; C.o1i = in->o1; C.hei = in->he;
-    C.o2nmi = in->o2_nm; C.o1nmi = in->o1_nm; C.henmi = in->he_nm;
-    C.xnmbar = in->xnmbar;
-    C.zpmid = g->zpmid;
-    C.dz = g->dz;
-    hipLaunchKernelGGL(comp_post_kernel, dim3(nblocks((long)D.nlon * 2 * nfilt)), dim3(256), 0, s, D, C);
-  }
-  TGX_HIP(hipGetLastError());
+  const Dims D = dims_of(g);
   // mp_periodic_f3d of every output the pass wrote
   double *per[8];
   int n = 0;
@@ -240,7 +154,6 @@ extern "C" int tgx_glb_halos(double *f, int nk, int nlon, int nlat, int ld, doub
     return tgx_set_error(TGX_ERR_ARG, "tgx_glb_halos: bad arguments (nk %d nlon %d (even) nlat %d ld %d)", nk, nlon,
                          nlat, ld);
   Dims D;
-  D.nfilt = 0;
   D.nk = nk;
   D.nlon = nlon;
   D.nlat = nlat;

@@ -4730,6 +4730,1499 @@ __global__ void __launch_bounds__(256) duv_wave_stage2(tgx_ng_grid g, Geo G, tgx
   }
 }
 
+// =============================================================================
+// Thomas columns, one block per BC columns of a latitude row.
+//
+// On a grid whose columns do not fill the chip one to a thread, a tile kernel
+// spends its time on one memory round trip after another, twice per level
+// (2.5 deg, 57 levels: 190-320 us per kernel for 10-25 us of traffic).  Here
+// 16 threads share a column: each assembles the rows of a run of levels, as
+// the tile kernels do, from the planes of the stencil preludes, and puts them
+// into LDS; one thread per column then eliminates and substitutes there in the
+// reference's order, and all threads apply the output stage to their own
+// levels.  The arithmetic is that of the tile kernels operation by operation,
+// so the results are theirs bit for bit, while the assembly runs with 16 times
+// the threads and the ratios, gammas and forward solutions never leave the CU.
+// A wavefront's load takes 64/BC levels of BC neighbouring columns: whole
+// 128-byte lines at BC = 16 (the PCR kernels' loads take 8 bytes of each of
+// 64 lines).
+constexpr int BSEG = 16;  // threads per column
+constexpr size_t BLOCK_LDS = 64 * 1024;  // LDS of one block
+
+template <int BC>
+struct BlockCol {
+  int c, s, i, j;
+  bool active, lat, ghost, solve;  // ghost: a global grid's periodic points and rows across the poles
+  __device__ __forceinline__ BlockCol(const Geo &G) {
+    const int ntx = (G.nlond + BC - 1) / BC;
+    const int b = tgx_xcd_block(gridDim.x);
+    c = threadIdx.x % BC;
+    s = threadIdx.x / BC;
+    i = (b % ntx) * BC + c;
+    j = b / ntx;
+    active = i < G.nlond && j < G.nlatd;
+    lat = active && !G.glb && (j == 0 || j == G.nlatd - 1 || i == 0 || i == G.nlond - 1);
+    ghost = G.glb && (i < 2 || i >= G.nlon + 2 || j < 2 || j >= G.nlat + 2);
+    solve = active && !lat && !ghost;
+  }
+  // f(k, i, j) = v, at the periodic point that repeats it too (mp_periodic_f3d)
+  __device__ __forceinline__ void put(const Geo &G, double *f, size_t p, double v) const {
+    f[p] = v;
+    if (!G.glb) return;
+    if (i < 4) f[p + G.nlon] = v;
+    else if (i >= G.nlon) f[p - G.nlon] = v;
+  }
+  // this thread's run of n levels
+  __device__ __forceinline__ void run(int n, int &k0, int &k1) const {
+    const int m = (n + BSEG - 1) / BSEG;
+    k0 = min(s * m, n);
+    k1 = min(k0 + m, n);
+  }
+};
+
+// The back substitution x(k) = F(k) - R(k) x(k+1) on one column in LDS, F
+// becoming the solution, CH rows read ahead (a row's LDS latency is several
+// times its arithmetic).
+template <int BC>
+__device__ __forceinline__ void block_back(const double *R, double *F, int n, double xn) {
+  constexpr int CH = 8;
+  double f[CH], r[CH];
+  auto load = [&](int k) {
+#pragma unroll
+    for (int q = 0; q < CH; ++q) {
+      const int o = max(k - q, 0) * BC;
+      f[q] = F[o];
+      r[q] = R[o];
+    }
+  };
+  load(n - 2);
+  for (int k = n - 2; k >= 0; k -= CH) {
+    double fc[CH], rc[CH];
+#pragma unroll
+    for (int q = 0; q < CH; ++q) {
+      fc[q] = f[q];
+      rc[q] = r[q];
+    }
+    load(k - CH);
+#pragma unroll
+    for (int q = 0; q < CH; ++q) {
+      const double x = fc[q] - rc[q] * xn;
+      if (k - q >= 0) {
+        F[(k - q) * BC] = x;
+        xn = x;
+      }
+    }
+  }
+}
+// Thomas (trsolv_ng.F90:14-26) on the n rows of one column in LDS, row k of
+// an array at k*BC: R becomes the ratios, Q the pivots, F the solution.  A row
+// is read ahead of the chain of divisions.
+template <int BC>
+__device__ __forceinline__ void block_thomas(const double *P, double *Q, double *R, double *F, int n) {
+  double w1 = Q[0], w3 = F[0] / w1, r = R[0];
+  F[0] = w3;
+  double p1 = P[BC], q1 = Q[BC], r1 = R[BC], f1 = F[BC];
+  for (int k = 1; k < n; ++k) {
+    const int kn = min(k + 1, n - 1) * BC;
+    const double p2 = P[kn], q2 = Q[kn], r2 = R[kn], f2 = F[kn];
+    const double w2 = r / w1;
+    R[(k - 1) * BC] = w2;
+    w1 = q1 - p1 * w2;
+    w3 = (f1 - p1 * w3) / w1;
+    Q[k * BC] = w1;
+    F[k * BC] = w3;
+    r = r1;
+    p1 = p2; q1 = q2; r1 = r2; f1 = f2;
+  }
+  block_back<BC>(R, F, n, w3);
+}
+// The two sweeps with kept pivots Q and ratios R.
+template <int BC>
+__device__ __forceinline__ void block_thomas_kept(const double *P, const double *Q, const double *R, double *F, int n) {
+  double w3 = F[0] / Q[0];
+  F[0] = w3;
+  double p1 = P[BC], q1 = Q[BC], f1 = F[BC];
+  for (int k = 1; k < n; ++k) {
+    const int kn = min(k + 1, n - 1) * BC;
+    const double p2 = P[kn], q2 = Q[kn], f2 = F[kn];
+    w3 = (f1 - p1 * w3) / q1;
+    F[k * BC] = w3;
+    p1 = p2; q1 = q2; f1 = f2;
+  }
+  block_back<BC>(R, F, n, w3);
+}
+
+// dt_ng.F90:54-213 (dt_tile_kernel's arithmetic).
+template <int BC>
+__global__ void __launch_bounds__(BC * BSEG) dt_block_kernel(tgx_ng_grid g, Geo G, tgx_ng_fields in, tgx_ng_out out,
+                                                             const double *__restrict__ hadv_tn,
+                                                             const double *__restrict__ smooth_tn_nm) {
+  extern __shared__ double smem[];
+  const BlockCol<BC> B(G);
+  const int nk = G.nk, i = B.i, j = B.j;
+  double *P = smem + B.c, *Q = P + BC * nk, *R = Q + BC * nk, *F = R + BC * nk;
+  const double dz = g.dz, dtx2inv = g.dtx2inv;
+  const int ic = B.active ? i : 0, jc = B.active ? j : 0;
+  const size_t c2 = G.a2(ic, jc);
+  const double t_lbc = in.t_lbc[c2], tl = in.tlbc[c2];
+  if (B.active && B.s == 0) {
+    out.tlbc_nm[c2] = tl;
+    out.tlbc[c2] = t_lbc;
+  }
+  int k0, k1;
+  B.run(nk - 1, k0, k1);
+#define F3(f, k) (f)[G.a3((k), ic, jc)]
+  if (B.solve && k0 < k1) {
+    struct DL { double w, cp, km, qtotal, schti, kt, un, vn; };
+    struct DS { double xn, o1, rkm12, mbar, scht, hdt, qji, cool_imp, cool_exp, hadv, tsm; };
+    auto load_dl = [&](int L, DL &D) {
+      size_t p = G.a3(L, ic, jc);
+      D.w = in.w_upd[p]; D.cp = in.cp[p]; D.km = in.km[p]; D.qtotal = in.qtotal[p];
+      D.schti = in.schti[p]; D.kt = in.kt[p]; D.un = in.un[p]; D.vn = in.vn[p];
+    };
+    auto load_ds = [&](int L, DS &S) {
+      size_t p = G.a3(L, ic, jc);
+      S.xn = in.xnmbar[p]; S.o1 = in.o1[p];
+      S.rkm12 = in.rkm12[p]; S.mbar = in.mbar[p]; S.scht = in.scht[p]; S.hdt = in.hdt[p];
+      S.qji = in.qji_tn[p]; S.cool_imp = in.cool_imp[p]; S.cool_exp = in.cool_exp[p];
+      S.hadv = hadv_tn[p]; S.tsm = smooth_tn_nm[p];
+    };
+    auto gf = [&](const DL &D, double expzL, double diftL, double tni, double &gg, double &ff) {
+      double h = D.schti;
+      double rho = P0 * g.expzmid_inv / (h * GRAV);
+      rho = rho * expzL;
+      double gpart = h * h * rho * D.cp;
+      double gpart_a = gpart * diftL;
+      gg = GRAV * (D.kt + gpart_a) / (P0 * h * (dz * dz));
+      ff = GRAV * GRAV * (h * h) * rho / (tni * P0 * 2. * dz);
+      ff = ff * diftL;
+    };
+    const double ulbc = in.ulbc[c2], vlbc = in.vlbc[c2];
+    DL dc, dn;
+    load_dl(k0, dc);
+    const int km = max(k0 - 1, 0);
+    double tn_m = F3(in.tn, km), tn_c = F3(in.tn, k0), tn_p = F3(in.tn, k0 + 1);
+    double un_m = F3(in.un, km), vn_m = F3(in.vn, km);
+    double gk, fk, dudz_prev = 0., dvdz_prev = 0.;
+    gf(dc, g.expz[k0], g.dift[k0], k0 == 0 ? tl : .5 * (tn_m + tn_c), gk, fk);
+    if (k0 == nk - 2) {  // the shear of level nk - 3, which the top row takes a third of
+      dudz_prev = (dc.un - F3(in.un, nk - 4)) / (2. * dz);
+      dvdz_prev = (dc.vn - F3(in.vn, nk - 4)) / (2. * dz);
+    }
+    for (int k = k0; k < k1; ++k) {
+      DS ds;
+      load_dl(k + 1, dn);
+      load_ds(k, ds);
+      const double tn_pp = k + 2 <= nk - 1 ? F3(in.tn, k + 2) : 0.;
+      const double expzk = g.expz[k], expzk1 = g.expz[k + 1], dift1 = g.dift[k + 1];
+      const double w_k = dc.w, w_k1 = dn.w;
+      // veradv (:57-65)
+      double raw_k = k == 0 ? (tn_c - t_lbc) * w_k * 2. : (tn_c - tn_m) * w_k;
+      double raw_k1 = (k + 1 <= nk - 2) ? (tn_p - tn_c) * w_k1 : 0.;
+      double veradv = (raw_k + raw_k1) * .5;
+      veradv = veradv / dz;
+      // interface means (:71-78)
+      double cpi = .5 * (dc.cp + dn.cp);
+      double kmi = .5 * (dc.km + dn.km);
+      double wi = .5 * (w_k + w_k1);
+      // cptn (:67, :80-83)
+      double advec_tn = ds.hadv + veradv;
+      double cptn = cpi * (advec_tn - dtx2inv * ds.tsm);
+      cptn = cptn * expzk;
+      // dudz (:85-94)
+      double dudz, dvdz;
+      if (k == 0) {
+        dudz = (dc.un + 1. / 3. * dn.un - 4. / 3. * ulbc) / dz;
+        dvdz = (dc.vn + 1. / 3. * dn.vn - 4. / 3. * vlbc) / dz;
+      } else if (k <= nk - 3) {
+        dudz = (dn.un - un_m) / (2. * dz);
+        dvdz = (dn.vn - vn_m) / (2. * dz);
+      } else {
+        dudz = dudz_prev / 3.;
+        dvdz = dvdz_prev / 3.;
+      }
+      dudz_prev = dudz;
+      dvdz_prev = dvdz;
+      // heating (:96-113)
+      double qsolar = .5 * (dc.qtotal + dn.qtotal);
+      double t = ds.xn * ds.o1 * RIO1;
+      double qrecomb = TSURPLUS * ds.rkm12 * (t * t) * AVO / ds.mbar;
+      double qm = GRAV * kmi / (P0 * ds.scht) * (dudz * dudz + dvdz * dvdz);
+      qm = qm / expzk;
+      double total_heat = qsolar + ds.hdt + qrecomb + ds.qji + qm;
+      double total_heat_a = total_heat * expzk;
+      cptn = cptn - total_heat_a;
+      // coefficients (:141-163)
+      double p = gk - fk, q, r;
+      double g1 = 0., f1 = 0.;
+      if (k <= nk - 3) {
+        double tni1 = .5 * (tn_c + tn_p);
+        gf(dn, expzk1, dift1, tni1, g1, f1);
+        q = -(g1 - f1 + gk + fk);
+        r = g1 + f1;
+      } else {
+        q = -gk - fk;
+        r = 0.;
+      }
+      double rhs = cptn;
+      double qpart = cpi * (dtx2inv + ds.cool_imp) + wi * GASK / ds.mbar;
+      rhs = rhs + ds.cool_exp;
+      double qpart_a = qpart * expzk;
+      q = q - qpart_a;
+      if (k == 0) {
+        q = q - p;
+        rhs = rhs - 2. * p * t_lbc;
+        p = 0.;
+      }
+      P[k * BC] = p;
+      Q[k * BC] = q;
+      R[k * BC] = r;
+      F[k * BC] = rhs;
+      gk = g1; fk = f1;
+      tn_m = tn_c; tn_c = tn_p; tn_p = tn_pp;
+      un_m = dc.un; vn_m = dc.vn;
+      dc = dn;
+    }
+  }
+  __syncthreads();
+  if (B.s == 0 && B.solve) block_thomas<BC>(P, Q, R, F, nk - 1);
+  __syncthreads();
+  if (!B.active || B.ghost) return;
+  if (B.lat) {
+    for (int k = B.s; k < nk; k += BSEG) {
+      double v;
+      lateral_value(G, in.lonb_tn, in.latb_tn, k, i, j, v);
+      size_t p = G.a3(k, i, j);
+      out.tn_nm[p] = DTSMOOTH_DIV2 * (in.tn_nm[p] + v) + DTSMOOTH * in.tn[p];
+      out.tn[p] = v > 100. ? v : 100.;
+    }
+    return;
+  }
+  // outputs (:167, :208-213)
+  const bool raw = G.raw_row(j);
+  for (int k = B.s; k < nk; k += BSEG) {
+    const size_t p = G.a3(k, i, j);
+    if (raw) {  // the raw solution; filter_tn and the post pass follow (dt.F:389-424)
+      if (k < nk - 1) out.tn[p] = F[k * BC];
+      continue;
+    }
+    if (G.glb && k == nk - 1) {  // spval at the top level (dt.F:407-408)
+      B.put(G, out.tn, p, SPVAL);
+      B.put(G, out.tn_nm, p, SPVAL);
+      continue;
+    }
+    const double x = k < nk - 1 ? F[k * BC] : F[(nk - 2) * BC] * F[(nk - 2) * BC] / F[(nk - 3) * BC];
+    B.put(G, out.tn_nm, p, DTSMOOTH_DIV2 * (in.tn_nm[p] + x) + DTSMOOTH * in.tn[p]);
+    B.put(G, out.tn, p, x > 100. ? x : 100.);
+  }
+#undef F3
+}
+
+// duv_ng.F90:73-80, the vertical integral ztmp: the increments of all levels
+// at once, one thread per column adding them up in the order of the loop.
+template <int BC>
+__global__ void __launch_bounds__(BC * BSEG) duv_stage1_block(tgx_ng_grid g, Geo G, tgx_ng_fields in, tgx_ng_out out,
+                                                              double *__restrict__ ztmp) {
+  extern __shared__ double smem[];
+  const BlockCol<BC> B(G);
+  const int nk = G.nk, i = B.active ? B.i : 0, j = B.active ? B.j : 0;
+  double *Z = smem + B.c;
+  const double dz = g.dz, wt = 0.225;
+#pragma unroll 4
+  for (int k = B.s; k < nk; k += BSEG) {
+    if (k == nk - 1) {  // its place holds level 0 of z
+      Z[k * BC] = in.z[G.a2(i, j)];
+      continue;
+    }
+    const size_t p = G.a3(k, i, j);
+    double tbar = (in.tn[p] * (-2.) + in.tn_nm[p] + out.tn[p]) * wt + in.tn[p];
+    Z[k * BC] = dz / DZGRAV * tbar / in.mbar[p];
+  }
+  __syncthreads();
+  if (B.s == 0) {
+    double zt = Z[(nk - 1) * BC], d = Z[0];
+    Z[0] = zt;
+    for (int k = 0; k < nk - 1; ++k) {
+      const double dn = Z[(k + 1) * BC];
+      zt = d + zt;
+      Z[(k + 1) * BC] = zt;
+      d = dn;
+    }
+  }
+  __syncthreads();
+  if (B.active)
+    for (int k = B.s; k < nk; k += BSEG) ztmp[G.a3(k, i, j)] = Z[k * BC];
+}
+
+// A value from the lane of this group of four that the quad permutation CTRL
+// names.
+template <int CTRL>
+__device__ __forceinline__ double quad(double v) {
+  union { double d; int w[2]; } a, b;
+  a.d = v;
+  b.w[0] = __builtin_amdgcn_mov_dpp(a.w[0], CTRL, 0xf, 0xf, true);
+  b.w[1] = __builtin_amdgcn_mov_dpp(a.w[1], CTRL, 0xf, 0xf, true);
+  return b.d;
+}
+
+// 2x2 block Thomas of the wind rows (duv.F:830-906; the couplings p and r are
+// multiples of the unit block) on one column in LDS, by four lanes: lane e
+// holds element e (11, 12, 21, 22) of the inverse, gamma and pivot blocks, so
+// the four divisions of a row are one instruction sequence.  The B elements
+// become the gammas of the row, S the solution.
+template <int BC>
+__device__ __forceinline__ void block_thomas_uv(const double *P, const double *R, double *Bm, double *S1, int rows, int n,
+                                                int e) {
+  // element arrays: Bm + e*rows; right-hand sides S1, S1 + rows
+  double *Be = Bm + e * rows, *Sx = S1 + (e & 1) * rows, *Sy = S1 + (e >> 1) * rows;
+  // be(e) = {h22, -h12, -h21, h11}(e) / det
+  auto invert = [&](double h) {
+    const double t = h * quad<0x1b>(h);                      // h11 h22 in lanes 0, 3; h12 h21 in 1, 2
+    const double det = quad<0x00>(t) - quad<0x55>(t);
+    const double a = quad<0x1b>(h);
+    return (e == 0 || e == 3 ? a : -h) / det;
+  };
+  // y of row e>>1: be(row,1) x1 + be(row,2) x2, x(e&1) in this lane
+  auto apply = [&](double be, double x) {
+    const double t = be * x;
+    return quad<0xa0>(t) + quad<0xf5>(t);                    // lanes 0,1: t0 + t1; lanes 2,3: t2 + t3
+  };
+  double be = invert(Be[0]);
+  double y = apply(be, Sx[0]);                               // y1 in lanes 0, 1; y2 in 2, 3
+  if ((e & 1) == 0) Sy[0] = y;
+  double rp = R[0], p = P[BC], r = R[BC], b = Be[BC], x0 = Sx[BC];
+  for (int k = 1; k < n; ++k) {
+    const int o = k * BC, on = min(k + 1, n - 1) * BC;
+    const double pn = P[on], rn = R[on], bn = Be[on], xn = Sx[on];
+    const double g = be * rp;
+    Be[o - BC] = g;
+    be = invert(b - p * g);
+    const double yx = quad<0x88>(y);                         // y(e & 1)
+    y = apply(be, x0 - p * yx);
+    if ((e & 1) == 0) Sy[o] = y;
+    rp = r;
+    p = pn; r = rn; b = bn; x0 = xn;
+  }
+  // back substitution, row e>>1 in this lane: (S - g(row,1) x1) - g(row,2) x2
+  const double *G1 = Bm + (e & 2) * rows, *G2 = G1 + rows;
+  double s = Sy[max(n - 2, 0) * BC], g1 = G1[max(n - 2, 0) * BC], g2 = G2[max(n - 2, 0) * BC];
+  for (int k = n - 2; k >= 0; --k) {
+    const int on = max(k - 1, 0) * BC;
+    const double sn = Sy[on], g1n = G1[on], g2n = G2[on];
+    const double x = s - g1 * quad<0x00>(y) - g2 * quad<0xaa>(y);
+    if ((e & 1) == 0) Sy[k * BC] = x;
+    y = x;
+    s = sn; g1 = g1n; g2 = g2n;
+  }
+}
+
+// duv_ng.F90:83-321 (duv_tile_kernel's arithmetic).
+template <int BC>
+__global__ void __launch_bounds__(BC * BSEG) duv_block_kernel(tgx_ng_grid g, Geo G, tgx_ng_fields in, tgx_ng_out out,
+                                                              UvTerms UT) {
+  extern __shared__ double smem[];
+  const BlockCol<BC> B(G);
+  const int nk = G.nk, i = B.i, j = B.j;
+  double *P = smem + B.c, *R = P + BC * nk, *B11 = R + BC * nk, *B12 = B11 + BC * nk, *B21 = B12 + BC * nk,
+         *B22 = B21 + BC * nk, *S1 = B22 + BC * nk, *S2 = S1 + BC * nk;
+  const double dz = g.dz, dtx2inv = g.dtx2inv;
+  const int ic = B.active ? i : 0, jc = B.active ? j : 0;
+  const size_t c2 = G.a2(ic, jc);
+  if (B.active && B.s == 0) {
+    if (B.solve) {
+      B.put(G, out.ulbc_nm, c2, in.ulbc[c2]);
+      B.put(G, out.vlbc_nm, c2, in.vlbc[c2]);
+      B.put(G, out.ulbc, c2, in.u_lbc[c2]);
+      B.put(G, out.vlbc, c2, in.v_lbc[c2]);
+    } else if (B.lat) {
+      out.ulbc_nm[c2] = in.ulbc[c2];
+      out.vlbc_nm[c2] = in.vlbc[c2];
+      out.ulbc[c2] = in.u_lbc[c2];
+      out.vlbc[c2] = in.v_lbc[c2];
+    }
+  }
+  int k0, k1;
+  B.run(nk - 1, k0, k1);
+  if (B.solve && k0 < k1) {
+    const double racs = g.racs[jc], cor = g.cor[jc], tanphi = g.tanphi[jc];
+    const double ulbc = in.u_lbc[c2], vlbc = in.v_lbc[c2];
+    struct UL { double w, lxx, lyy, lxy, lyx, ui, vi, km, schti, scht, divx, divy; };
+    struct US { double Fe, Fn, hdu, hdv, unms, vnms, advu, advv, un; };
+    auto load_ul = [&](int L, UL &U) {
+      size_t p = G.a3(L, ic, jc);
+      U.w = in.w_upd[p]; U.lxx = in.lxx[p]; U.lyy = in.lyy[p]; U.lxy = in.lxy[p]; U.lyx = in.lyx[p];
+      U.ui = in.ui[p]; U.vi = in.vi[p]; U.km = in.km[p]; U.schti = in.schti[p]; U.scht = in.scht[p];
+      U.divx = UT.divx_ztmp[p]; U.divy = UT.divy_z[p];
+    };
+    auto load_us = [&](int L, US &S) {
+      size_t p = G.a3(L, ic, jc);
+      S.Fe = out.Fe[p]; S.Fn = out.Fn[p]; S.hdu = in.hdu[p]; S.hdv = in.hdv[p];
+      S.unms = UT.unms[p]; S.vnms = UT.vnms[p]; S.advu = UT.advu[p]; S.advv = UT.advv[p]; S.un = in.un[p];
+    };
+    auto e1b = [&](double scht, int L) -> double {
+      double e = P0 * scht / GRAV;
+      return e * g.expz[L] * g.xmue[L];
+    };
+    auto gg = [&](const UL &U, double evf) { return GRAV * (U.km + evf) / (P0 * U.schti * (dz * dz)); };
+    UL ua, ub;
+    load_ul(k0, ua);
+    load_ul(k0 + 1, ub);
+    double e1_c = e1b(ua.scht, k0), e1_m, gk;
+    if (k0 == 0) {
+      e1_m = 0.;
+      const double e1_1 = e1b(ub.scht, 1);
+      gk = gg(ua, e1_c * e1_c / sqrt(e1_c * e1_1));
+    } else {
+      e1_m = e1b(in.scht[G.a3(k0 - 1, ic, jc)], k0 - 1);
+      gk = gg(ua, sqrt(e1_m * e1_c));
+    }
+    for (int k = k0; k < k1; ++k) {
+      US us;
+      if (k > k0) load_ul(k + 1, ub);
+      load_us(k, us);
+      double e1_n = k + 1 <= nk - 2 ? e1b(ub.scht, k + 1) : sqrt(e1_c * e1_c * e1_c / e1_m);
+      double gk1 = gg(ub, sqrt(e1_c * e1_n));
+      double g_1 = gk1;
+      const double expzk = g.expz[k];
+      double wi = .5 * (ua.w + ub.w);
+      double dwdz = wi / (2. * dz);
+      dwdz = dwdz * expzk;
+      double lxxi = .5 * (ua.lxx + ub.lxx), lyyi = .5 * (ua.lyy + ub.lyy);
+      double lxyi = .5 * (ua.lxy + ub.lxy), lyxi = .5 * (ua.lyx + ub.lyx);
+      double uii = .5 * (ua.ui + ub.ui), vii = .5 * (ua.vi + ub.vi);
+      double udc = us.Fe + lxxi * uii + lxyi * vii;
+      double vdc = us.Fn + lyyi * vii - lyxi * uii;
+      double zl = (ua.divx + ub.divx) * .5;
+      zl = zl * racs;
+      zl = zl * GRAV / g.dlamda;
+      double zp = (ua.divy + ub.divy) * .5;
+      zp = zp * GRAV * RE_INV / g.dphi;
+      double s1 = dtx2inv * us.unms + us.hdu + udc - us.advu - zl;
+      double s2 = dtx2inv * us.vnms + us.hdv + vdc - us.advv - zp;
+      s1 = s1 * expzk;
+      s2 = s2 * expzk;
+      double p11 = -(gk + dwdz);
+      double r11 = -(g_1 - dwdz);
+      double q11 = gk + g_1;
+      double qa = dtx2inv + lxxi;
+      qa = qa * expzk;
+      double qq11 = q11 + qa;
+      qa = dtx2inv + lyyi;
+      qa = qa * expzk;
+      double qq22 = q11 + qa;
+      double q12 = cor + us.un / RE * tanphi;
+      double q21 = q12;
+      qa = q12 - lxyi;
+      qa = qa * expzk;
+      double qq12 = -qa;
+      qa = q21 - lyxi;
+      qa = qa * expzk;
+      double qq21 = qa;
+      if (k == 0) {  // :207-212
+        qq11 = qq11 - p11;
+        qq22 = qq22 - p11;
+        s1 = s1 - 2. * (p11 * ulbc);
+        s2 = s2 - 2. * (p11 * vlbc);
+        p11 = 0.;
+      }
+      if (k == nk - 2) {  // :214-215
+        qq11 = qq11 + r11;
+        qq22 = qq22 + r11;
+        r11 = 0.;
+      }
+      const int o = k * BC;
+      P[o] = p11; R[o] = r11;
+      B11[o] = qq11; B12[o] = qq12; B21[o] = qq21; B22[o] = qq22;
+      S1[o] = s1; S2[o] = s2;
+      gk = gk1;
+      e1_m = e1_c;
+      e1_c = e1_n;
+      ua = ub;
+    }
+  }
+  __syncthreads();
+  if ((int)threadIdx.x < 4 * BC) {  // every column of the block (one that is not solved holds no rows and is not read)
+    const int cc = (int)threadIdx.x >> 2;
+    const int ci = i - B.c + cc;
+    const int edge = G.glb ? 2 : 1;
+    if (j >= edge && j < G.nlatd - edge && ci >= edge && ci < G.nlond - edge)
+      block_thomas_uv<BC>(P - B.c + cc, R - B.c + cc, B11 - B.c + cc, S1 - B.c + cc, BC * nk, nk - 1,
+                          (int)threadIdx.x & 3);
+  }
+  __syncthreads();
+  if (!B.active || B.ghost) return;
+  const bool raw = G.raw_row(j);
+  for (int k = B.s; k < nk; k += BSEG) {
+    const size_t p = G.a3(k, i, j);
+    double u, v;
+    if (B.lat) {
+      lateral_value(G, in.lonb_un, in.latb_un, k, i, j, u);
+      lateral_value(G, in.lonb_vn, in.latb_vn, k, i, j, v);
+    } else if (raw) {  // the raw solution; filter_uv and the post pass follow (duv.F:490-514)
+      if (k < nk - 1) {
+        out.un[p] = S1[k * BC];
+        out.vn[p] = S2[k * BC];
+      }
+      continue;
+    } else if (k < nk - 1) {
+      u = S1[k * BC];
+      v = S2[k * BC];
+    } else if (G.glb) {  // spval at the top level (duv.F:385-386, :512-513)
+      B.put(G, out.un, p, SPVAL);
+      B.put(G, out.vn, p, SPVAL);
+      B.put(G, out.un_nm, p, SPVAL);
+      B.put(G, out.vn_nm, p, SPVAL);
+      continue;
+    } else {  // :250
+      u = 2 * S1[(nk - 2) * BC] - S1[(nk - 3) * BC];
+      v = 2 * S2[(nk - 2) * BC] - S2[(nk - 3) * BC];
+    }
+    B.put(G, out.un, p, u);
+    B.put(G, out.vn, p, v);
+    B.put(G, out.un_nm, p, DTSMOOTH_DIV2 * (in.un_nm[p] + u) + DTSMOOTH * in.un[p]);
+    B.put(G, out.vn_nm, p, DTSMOOTH_DIV2 * (in.vn_nm[p] + v) + DTSMOOTH * in.vn[p]);
+  }
+}
+
+// One O+ sub-step (oplus_tile_kernel's arithmetic and MODEs).  The kept
+// factorisation lies in 64-column groups: W.fac holds the sub-diagonal, the
+// pivot and the boundary terms, value 0 of W.w2 the ratio.
+template <int BC, int MODE>
+__device__ __forceinline__ void oplus_block(const tgx_ng_grid &g, const Geo &G, const tgx_ng_fields &in,
+                                            const double *op, const double *optm1, const double *lonb,
+                                            const double *latb, const OpWork &W, const OpTerms &OT,
+                                            const double *oploss_p, const double *opprod_p, double *opout,
+                                            double *optm1out) {
+  extern __shared__ double smem[];
+  const BlockCol<BC> B(G);
+  const int nk = G.nk, i = B.i, j = B.j, nsub = g.nstep_sub;
+  double *P = smem + B.c, *Q = P + BC * nk, *R = Q + BC * nk, *F = R + BC * nk;
+  const double dz = g.dz, dtx2inv = g.dtx2inv;
+  const int ic = B.active ? i : 0, jc = B.active ? j : 0;
+  const size_t c2 = G.a2(ic, jc);
+  int k0, k1;
+  B.run(nk - 1, k0, k1);
+#define F3(f, k) (f)[G.a3((k), ic, jc)]
+  if (B.solve && k0 < k1) {
+    const double bz = in.bz[c2], cs = g.cs[jc];
+    double opflux = 0., dvb;
+    const double pi = 4.0 * atan(1.0), rtd = 180. / pi;
+    if (MODE != 2 && k1 == nk - 1) {  // :77-91, the top row's
+      const double phid = 2.0e8, phin = -2.0e8, ppolar = 0.;
+      double rl = in.rlatm[c2], a = 0.;
+      if (fabs(rl) >= pi / 4.5) a = 1.;
+      if (fabs(rl) < pi / 4.5 && fabs(rl) > pi / 18) a = .5 * (1. + cos(fabs(rl) * 6. - pi * 4. / 3.));
+      if (fabs(rl) <= pi / 18) a = 0.;
+      double fed = phid * a, fen = phin * a, chi = in.chi[c2];
+      if (chi >= 0.5 * pi) opflux = fen; else opflux = fed;
+      if ((chi * rtd - 80.) * (chi * rtd - 100.) < 0.)
+        opflux = .5 * (fed + fen) + .5 * (fed - fen) * cos(pi * (chi * rtd - 80.) / 20.);
+      if (fabs(rl) >= pi / 3.) opflux = opflux + ppolar;
+    }
+    {  // :94-104 (df_2d of bx and of cs*by)
+      double dbxdx = dflon1(in.bx, G, i, j);
+      auto csby = [&](int jj) { return g.cs[jj] * in.by[G.a2(i, jj)]; };
+      int J1 = G.nlatd - 1;
+      double dcsbydy;
+      if (j == 0) dcsbydy = csby(1) - csby(0);
+      else if (j == J1) dcsbydy = csby(J1) - csby(J1 - 1);
+      else dcsbydy = (csby(j + 1) - csby(j - 1)) / 2.;
+      double vv = dbxdx / g.dlamda + dcsbydy / g.dphi;
+      vv = vv / cs;
+      dvb = (vv + 2. * bz) / RE;
+    }
+    const double dvbz = dvb / bz;
+    const double gmr = GRAV * RMOP / (2. * GASK);
+    struct OL { double scht, hdz, tp1, dj, bdotu, bdopj, wi; };
+    struct OS { double oploss, opprod, djbz, bd_diff, bd_diffj, bd_bvel, bd_djbz, vdotn, opts2, pcf, w1, w2; };
+    auto load_ol = [&](int L, OL &q) {
+      size_t p = G.a3(L, ic, jc);
+      q.scht = in.scht[p];
+      q.bdopj = W.bdopj[p];
+      if (MODE == 2) return;  // the right-hand side needs no more
+      q.hdz = 1. / (q.scht * dz);
+      q.tp1 = 0.5 * (in.ti[p] + in.te[p]);
+      q.dj = W.dj[p]; q.bdotu = W.bdotu[p]; q.wi = in.wi[p];
+    };
+    auto load_os = [&](int L, OS &q) {
+      size_t p = G.a3(L, ic, jc);
+      q.opprod = opprod_p[p];
+      q.djbz = W.djbz[p];
+      q.bd_diff = OT.bd_diff[p]; q.bd_diffj = OT.bd_diffj[p]; q.bd_bvel = OT.bd_bvel[p];
+      q.vdotn = OT.vdotn[p]; q.opts2 = OT.opts2[p];
+      if (MODE != 2) {
+        q.oploss = oploss_p[p];
+        q.bd_djbz = OT.bd_djbz[p];
+      } else {
+        const size_t t = G.tile(L, ic, jc, 0, OF_NV);
+        q.pcf = L > 0 ? W.fac[t] : 0.;
+        q.w1 = W.fac[t + 64];
+        q.w2 = L < nk - 2 ? W.w2[G.tile(L, ic, jc, 0, OW_NV)] : 0.;
+      }
+    };
+    OL qa = {}, qb = {}, qc = {};
+    if (k0 > 0) load_ol(k0 - 1, qa);
+    load_ol(k0, qb);
+    for (int k = k0; k < k1; ++k) {
+      OS os;
+      load_ol(k + 1, qc);
+      load_os(k, os);
+      const bool top = k == nk - 2;
+      // explicit terms (:181-211, :250)
+      double dbd;
+      if (k == 0) dbd = qc.bdopj - qb.bdopj;
+      else if (k <= nk - 3) dbd = (qc.bdopj - qa.bdopj) / 2.;
+      else dbd = qb.bdopj - qa.bdopj;
+      double bdzdvb = bz / (qb.scht * dz) * dbd + dvb * qb.bdopj;
+      double bd_op = os.djbz * os.bd_diffj;
+      double diffexp = bdzdvb + os.bd_diff + bd_op;
+      double expl = -1. * diffexp;
+      expl = expl + os.vdotn + os.bd_bvel;
+      expl = expl - os.opts2 * dtx2inv * nsub;
+      const int o = k * BC;
+      if (MODE == 2) {  // the kept factorisation and boundary terms
+        if (top) expl = expl - W.fac[G.tile(k, ic, jc, 2, OF_NV)];
+        expl = expl - os.opprod;
+        if (k == 0) expl = expl - W.fac[G.tile(0, ic, jc, 2, OF_NV)];
+        P[o] = os.pcf; Q[o] = os.w1; R[o] = os.w2; F[o] = expl;
+      } else {
+        // diffusion, drift and wind coefficients (:239-278)
+        double divbz = dvbz + os.bd_djbz / (qb.dj * (bz * bz));
+        double hm = qb.hdz - 0.5 * divbz, hp = qb.hdz + 0.5 * divbz;
+        hm = hm * (bz * bz);
+        hp = hp * (bz * bz);
+        double hdzi_k = k == 0 ? 1.5 * qb.hdz - 0.5 * qc.hdz : 0.5 * (qa.hdz + qb.hdz);
+        double hdzi_k1 = top ? 1.5 * qb.hdz - 0.5 * qa.hdz : 0.5 * (qb.hdz + qc.hdz);
+        double dji = k == 0 ? 1.5 * qb.dj - 0.5 * qc.dj : 0.5 * (qa.dj + qb.dj);
+        double dji1 = top ? 1.5 * qb.dj - 0.5 * qa.dj : 0.5 * (qb.dj + qc.dj);
+        double t0 = k == 0 ? 2. * (2. * qb.tp1 - qc.tp1) * hdzi_k - gmr : 2. * qa.tp1 * hdzi_k - gmr;
+        double t01 = 2. * qb.tp1 * hdzi_k1 - gmr;
+        double t1 = 2. * qb.tp1 * hdzi_k + gmr;
+        double t11 = top ? 2. * (2. * qb.tp1 - qa.tp1) * hdzi_k1 + gmr : 2. * qc.tp1 * hdzi_k1 + gmr;
+        double diffp = hm * dji * t0;
+        double diffq = -(hp * dji1 * t01 + hm * dji * t1);
+        double diffr = hp * dji1 * t11;
+        double hdzk = qb.hdz;
+        double wii = .5 * (qb.wi + qc.wi);
+        double driftp = wii * 0.5 * hdzk;
+        double driftq = -wii * 6. / RE;
+        double driftr = -wii * 0.5 * hdzk;
+        double windp = k == 0 ? bz * (2. * qb.bdotu - qc.bdotu) * 0.5 * hdzk : bz * qa.bdotu * 0.5 * hdzk;
+        double windq = -qb.bdotu * dvbz * bz;
+        double windr = !top ? -bz * qc.bdotu * 0.5 * hdzk : bz * (2. * qb.bdotu - qa.bdotu) * 0.5 * hdzk;
+        double pcf = diffp + driftp + windp;
+        double qcf = diffq + driftq + windq - dtx2inv * nsub;
+        double rcf = diffr + driftr + windr;
+        if (top) {  // upper boundary (:280-286)
+          double djn = dji1;
+          double ubcb = -(bz * bz) * djn * t01;
+          double ubca = -(bz * bz) * djn * t11;
+          qcf = qcf + ubcb / ubca * rcf;
+          const double ub = opflux * rcf / ubca;
+          if (MODE == 1) W.fac[G.tile(k, ic, jc, 2, OF_NV)] = ub;
+          expl = expl - ub;
+          rcf = 0.;
+        }
+        qcf = qcf - os.oploss;
+        expl = expl - os.opprod;
+        if (k == 0) {  // lower boundary (:301-303)
+          qcf = qcf - pcf;
+          const double lb = 2. * pcf * F3(in.qop, 0) / (1.5 * os.oploss - 0.5 * F3(oploss_p, 1));
+          if (MODE == 1) W.fac[G.tile(0, ic, jc, 2, OF_NV)] = lb;
+          expl = expl - lb;
+          pcf = 0.;
+        }
+        P[o] = pcf; Q[o] = qcf; R[o] = rcf; F[o] = expl;
+      }
+      qa = qb;
+      qb = qc;
+    }
+  }
+  __syncthreads();
+  if (B.s == 0 && B.solve) {
+    if (MODE == 2) block_thomas_kept<BC>(P, Q, R, F, nk - 1);
+    else block_thomas<BC>(P, Q, R, F, nk - 1);
+  }
+  __syncthreads();
+  if (!B.active) return;
+  if (B.ghost) {  // the rows across the poles keep the step input's between sub-cycles (oplus.F:942)
+    if (j < 2 || j >= G.nlat + 2)
+      for (int k = B.s; k < nk; k += BSEG) {
+        const size_t p = G.a3(k, i, j);
+        opout[p] = in.op[p];
+        optm1out[p] = in.op_nm[p];
+      }
+    return;
+  }
+  const bool raw = G.raw_row(j);
+  for (int k = B.s; k < nk; k += BSEG) {
+    const size_t p = G.a3(k, i, j);
+    if (MODE == 1 && B.solve && k < nk - 1) {
+      const size_t t = G.tile(k, i, j, 0, OF_NV);
+      W.fac[t] = P[k * BC];
+      W.fac[t + 64] = Q[k * BC];
+      if (k < nk - 2) W.w2[G.tile(k, i, j, 0, OW_NV)] = R[k * BC];
+    }
+    double x;
+    if (B.lat) {
+      lateral_value(G, lonb, latb, k, i, j, x);
+    } else if (raw) {  // the raw solution; filter_op and the post pass follow (oplus.F:896-941)
+      if (k < nk - 1) opout[p] = F[k * BC];
+      continue;
+    } else if (k < nk - 1) {
+      x = F[k * BC];
+    } else if (G.glb) {  // zero at the top level (oplus.F:922-923)
+      B.put(G, opout, p, 0.);
+      B.put(G, optm1out, p, 0.);
+      continue;
+    } else {
+      x = F[(nk - 2) * BC] * F[(nk - 2) * BC] / F[(nk - 3) * BC];
+    }
+    const double nm = DTSMOOTH * op[p] + DTSMOOTH_DIV2 * (optm1[p] + x);
+    B.put(G, opout, p, x > 0. ? x : 0.);
+    B.put(G, optm1out, p, nm > 0. ? nm : 0.);
+  }
+#undef F3
+}
+#define OPLUS_BLOCK_KERNEL(name, MODE)                                                                                \
+  template <int BC>                                                                                                   \
+  __global__ void __launch_bounds__(BC * BSEG)                                                                        \
+  name(tgx_ng_grid g, Geo G, tgx_ng_fields in, tgx_ng_out, const double *__restrict__ op,                             \
+       const double *__restrict__ optm1, const double *__restrict__ lonb, const double *__restrict__ latb, OpWork W,  \
+       OpTerms OT, const double *__restrict__ loss, const double *__restrict__ prod, double *__restrict__ opout,      \
+       double *__restrict__ optm1out) {                                                                               \
+    oplus_block<BC, MODE>(g, G, in, op, optm1, lonb, latb, W, OT, loss, prod, opout, optm1out);                       \
+  }
+OPLUS_BLOCK_KERNEL(oplus_block_kernel, 0)
+OPLUS_BLOCK_KERNEL(oplus_block_keep_kernel, 1)
+OPLUS_BLOCK_KERNEL(oplus_block_reuse_kernel, 2)
+#undef OPLUS_BLOCK_KERNEL
+
+// minor_ng.F90:60-237 for a pair of species (minor_kernel's arithmetic).
+template <int BC, int SA, int SB, bool LIN>
+__device__ __forceinline__ void minor_block(const tgx_ng_grid &g, const Geo &G, const tgx_ng_fields &in,
+                                            const tgx_ng_out &out, const MinorTerms &MT) {
+  extern __shared__ double smem[];
+  const BlockCol<BC> B(G);
+  const int nk = G.nk;
+  const int i = B.active ? B.i : 0, j = B.active ? B.j : 0;
+  // species q: P, Q, R, F at smem + 4*q*BC*nk
+  double *P = smem + B.c;
+  const int rows = BC * nk;
+  const double dzp = g.dz, dtx2inv = g.dtx2inv, rdz = 1. / g.dz;
+  const size_t c2 = G.a2(i, j);
+  const int SP[2] = {SA, SB};
+  double *outs[2], *outs_nm[2];
+  const double *fc[2], *fctm1[2], *lonb[2], *latb[2];
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    int s = SP[q];
+    outs[q] = s == 0 ? out.no : s == 1 ? out.n4s : s == 2 ? out.n2d : out.ar;
+    outs_nm[q] = s == 0 ? out.no_nm : s == 1 ? out.n4s_nm : s == 2 ? out.n2d_nm : out.ar_nm;
+    fc[q] = s == 0 ? in.no : s == 1 ? in.n4s : s == 2 ? in.n2d : in.ar;
+    fctm1[q] = s == 0 ? in.no_nm : s == 1 ? in.n4s_nm : s == 2 ? in.n2d_nm : in.ar_nm;
+    lonb[q] = s == 0 ? in.lonb_no : s == 1 ? in.lonb_n4s : s == 2 ? in.lonb_n2d : in.lonb_ar;
+    latb[q] = s == 0 ? in.latb_no : s == 1 ? in.latb_n4s : s == 2 ? in.latb_n2d : in.latb_ar;
+  }
+  const double small = 1.e-12;
+  int k0, k1;
+  B.run(nk, k0, k1);
+#define F3(f, k) (f)[G.a3((k), i, j)]
+  if (B.solve && k0 < k1) {
+    const double pi = 4.0 * atan(1.0);
+    double dfac;
+    {  // minor_ng.F90:145-154
+      const double hor = .25, dtr = pi / 180.;
+      if (!(g.difhor > 0)) dfac = 1.;
+      else {
+        double rlat = g.glat[j] * dtr;
+        if (fabs(rlat) >= pi / 4.5) dfac = hor + 1.;
+        else dfac = hor + .5 * (1. + sin(pi * (fabs(rlat) - pi / 9.) / (pi / 4.5)));
+      }
+    }
+    const double racs = g.racs[j];
+    SpeciesConst sc[2] = {species_const(SA), species_const(SB)};
+    const double *n2d_upd = out.n2d;  // the N2D of this step (used by NO and N4S)
+
+    // lower boundary of the major species (:66-69)
+    const double o2_0 = F3(in.o2, 0), o1_0 = F3(in.o1, 0), he_0 = F3(in.he, 0);
+    const double bo2 = g.b[0] * o2_0 + g.b[1] * o1_0 + g.b[2] * he_0 + g.fb[0];
+    const double bo1 = g.b[3] * o2_0 + g.b[4] * o1_0 + g.b[5] * he_0 + g.fb[1];
+    const double bhe = g.b[6] * o2_0 + g.b[7] * o1_0 + g.b[8] * he_0 + g.fb[2];
+    const double xmbari = 1. / (bo2 * RIO2 + bo1 * RIO1 + (1. - bo2 - bo1 - bhe) * RIN2 + bhe * RIHE);
+
+    struct MR { double o1, o2, he, mbar, tn, barm, w; };  // shared fields at one level
+    struct SR { double rhs, sloss, s0prod, la, lb, n2d; };  // one species at one level
+    auto load_mr = [&](int L, MR &R) {
+      size_t p = G.a3(L, i, j);
+      R.o1 = in.o1[p]; R.o2 = in.o2[p]; R.he = in.he[p]; R.mbar = in.mbar[p]; R.tn = in.tn[p];
+      R.barm = in.barm[p]; R.w = in.w_upd[p];
+    };
+    auto load_sr = [&](int L, SR *Q) {
+      size_t p = G.a3(L, i, j);
+  #pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        Q[q].rhs = MT.rt[G.tile(L, i, j, SP[q], MR_NV)];
+        const size_t ts = G.tile(L, i, j, 0, MS_NV), tl = G.tile(L, i, j, 0, ML_NV);
+        if (SP[q] == 3) { Q[q].sloss = 0.; Q[q].s0prod = 0.; }
+        else if (LIN && SP[q] == 0) {  // NO: sloss = lin2 + n2d lin3, s0prod = lin4 + n2d lin5
+          Q[q].sloss = MT.lt[tl + 128]; Q[q].la = MT.lt[tl + 192];
+          Q[q].s0prod = MT.lt[tl + 256]; Q[q].lb = MT.lt[tl + 320]; Q[q].n2d = MT.n2d[p];
+        } else if (LIN && SP[q] == 1) {  // N4S: s0prod = lin0 + n2d lin1
+          Q[q].sloss = MT.st[ts + ms_loss(1) * 64];
+          Q[q].s0prod = MT.lt[tl]; Q[q].lb = MT.lt[tl + 64]; Q[q].n2d = MT.n2d[p];
+        }
+        else { Q[q].sloss = MT.st[ts + ms_loss(SP[q]) * 64]; Q[q].s0prod = MT.st[ts + ms_prod(SP[q]) * 64]; }
+      }
+    };
+    // :66-126 interface quantities at L from levels A = L-1 and B = L (L >= 1),
+    // or from the lower boundary and B = level 0 (L = 0)
+    auto shared_at = [&](int L, const MR &A, const MR &B, MinorShared &S) {
+      if (L == 0) {
+        S.dmdz = (B.mbar - xmbari) * rdz;
+        S.pso1 = .5 * (bo1 + o1_0);
+        S.pso2 = .5 * (bo2 + o2_0);
+        S.pshe = .5 * (bhe + he_0);
+        S.do1dz = (o1_0 - bo1) * rdz;
+        S.do2dz = (o2_0 - bo2) * rdz;
+        S.dhedz = (he_0 - bhe) * rdz;
+        S.tni = in.tlbc[c2];
+      } else {
+        S.dmdz = (B.mbar - A.mbar) * rdz;
+        S.pso1 = .5 * (B.o1 + A.o1);
+        S.pso2 = .5 * (B.o2 + A.o2);
+        S.pshe = .5 * (B.he + A.he);
+        S.do1dz = (B.o1 - A.o1) * rdz;
+        S.do2dz = (B.o2 - A.o2) * rdz;
+        S.dhedz = (B.he - A.he) * rdz;
+        S.tni = L == nk - 1 ? A.tn : .5 * (B.tn + A.tn);  // :89-93
+      }
+      S.barm = B.barm;
+      double al[9];
+      const TPow tp = tpows(S.tni);
+      const double *df = tp.df;
+      S.q = tp.q;
+      al[0] = -(PHI(1, 4) + (PHI(1, 2) - PHI(1, 4)) * S.pso1 + (df[0] * PHI(1, 3) - PHI(1, 4)) * S.pshe);
+      al[4] = -(PHI(2, 4) + (PHI(2, 1) - PHI(2, 4)) * S.pso2 + (df[1] * PHI(2, 3) - PHI(2, 4)) * S.pshe);
+      al[8] = -(df[2] * PHI(3, 4) + (df[0] * PHI(3, 1) - df[2] * PHI(3, 4)) * S.pso2 +
+                (df[1] * PHI(3, 2) - df[2] * PHI(3, 4)) * S.pso1);
+      al[3] = (PHI(1, 2) - PHI(1, 4)) * S.pso2;
+      al[6] = (df[0] * PHI(1, 3) - PHI(1, 4)) * S.pso2;
+      al[1] = (PHI(2, 1) - PHI(2, 4)) * S.pso1;
+      al[7] = (df[1] * PHI(2, 3) - PHI(2, 4)) * S.pso1;
+      al[2] = (df[0] * PHI(3, 1) - df[2] * PHI(3, 4)) * S.pshe;
+      al[5] = (df[1] * PHI(3, 2) - df[2] * PHI(3, 4)) * S.pshe;
+      matinv3_r(al, S.inv);
+    };
+    auto species_at = [&](int q, const MinorShared &S, double dtnidz, const SR &R, MinorSpecies &T) {
+      const SpeciesConst &c = sc[q];
+      double sai[3];
+      for (int n = 0; n < 3; ++n) {
+        double s = 0.;
+        for (int m = 0; m < 3; ++m) s = s + c.salfax[m] * S.inv[m + 3 * n];
+        sai[n] = s;
+      }
+      const double rb = 1. / S.barm;
+      double ex = 1. - (c.rmx + S.dmdz) * rb +
+                  sai[0] * (S.do2dz - (1. - (RMO2 + S.dmdz) * rb) * S.pso2) +
+                  sai[1] * (S.do1dz - (1. - (RMO1 + S.dmdz) * rb) * S.pso1) +
+                  sai[2] * (S.dhedz - (1. - (RMHE + S.dmdz) * rb) * S.pshe);
+      // phi_x(He) in the nest form's sum (minor_ng.F90:135-136), phi_x(N2) in
+      // the global minor.F:359-362
+      T.ax = -(S.barm * (1. / (TAU * RMN2)) * S.q /
+               (c.phix[G.glb ? 3 : 2] + c.salfax[0] * S.pso2 + c.salfax[1] * S.pso1 + c.salfax[2] * S.pshe));
+      T.thdiff = ex - c.alfax * dtnidz / (dzp * S.tni);
+      T.sloss = R.sloss;
+      T.s0prod = R.s0prod;
+      if (LIN && SP[q] == 0) {
+        T.sloss = R.sloss + R.n2d * R.la;
+        T.s0prod = R.s0prod + R.n2d * R.lb;
+      } else if (LIN && SP[q] == 1) {
+        T.s0prod = R.s0prod + R.n2d * R.lb;
+      }
+      T.rhs = R.rhs;
+    };
+    // lower-boundary data flbc(:,:,1:3) of each species (comp_*_ng.F90)
+    double l1[2], l2[2], l3[2];
+  #pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      int s = SP[q];
+      size_t p = G.a3(0, i, j);
+      double xb = in.xnmbari[p];
+      l1[q] = 0.;
+      l2[q] = 1.;
+      if (s == 0) l3[q] = -4.e6 * RMNO / xb;
+      else if (s == 1)
+        l3[q] = -(RMN4S / xb *
+                  (in.qtef[p] * (1. - BRN2D) / xb +
+                   n2d_upd[p] * RIN2D * (BETA4 * xb * in.o1[p] * RIO1 + in.beta5[p] * in.ne[p] + BETA7) +
+                   in.beta8[p] * in.no[p] * RINO) /
+                  (in.beta1[p] * in.o2[p] * RIO2 + in.beta3[p] * in.no[p] * RINO +
+                   xb * in.beta17[p] * in.o1[p] * RIO1 * in.n2[p] * RIN2));
+      else if (s == 2)
+        l3[q] = -(RMN2D / xb * in.qtef[p] * BRN2D /
+                  (xb * (BETA2 * in.o2[p] * RIO2 + BETA4 * in.o1[p] * RIO1 + BETA6 * in.no[p] * RINO) + BETA7 +
+                   in.beta5[p] * in.ne[p]));
+      else l3[q] = -sqrt(g.ar_glbm1 * g.ar_glbm2);
+    }
+    const double fubc = 0.;  // every species sets fubc = 0 (comp_*_ng.F90)
+
+    // window of the shared fields at levels k (R0), k+1 (R1), k+2 (R2); Rm the level below
+    MR Rm, R0, R1, R2;
+    SR Y[2];
+    load_mr(max(k0 - 1, 0), Rm);
+    load_mr(k0, R0);
+    load_mr(min(k0 + 1, nk - 1), R1);
+    load_sr(k0, Y);
+    MinorShared Sc, Sn;
+    MinorSpecies Tc[2], Tn[2];
+    shared_at(k0, Rm, R0, Sc);
+    {
+      // tni on either side of level k0 (:89-93)
+      const double tni_p = k0 + 1 == nk - 1 ? R0.tn : .5 * (R1.tn + R0.tn);
+      double dtnidz;
+      if (k0 == 0) {
+        dtnidz = tni_p - Sc.tni;
+      } else {
+        const double tni_m = k0 == 1 ? in.tlbc[c2] : .5 * (Rm.tn + F3(in.tn, k0 - 2));
+        dtnidz = k0 == nk - 1 ? Sc.tni - tni_m : (tni_p - tni_m) / 2.;
+      }
+#pragma unroll
+      for (int q = 0; q < 2; ++q) species_at(q, Sc, dtnidz, Y[q], Tc[q]);
+    }
+    double wic = k0 < nk - 1 ? .5 * (R0.w + R1.w) : 1.5 * R0.w - .5 * Rm.w;
+    for (int k = k0; k < k1; ++k) {
+      if (k + 2 <= nk - 1) load_mr(k + 2, R2);
+      if (k + 1 <= nk - 1) load_sr(k + 1, Y);
+      const double difk0 = g.difk[k], difk1 = k + 1 <= nk - 1 ? g.difk[k + 1] : 0., expzk = g.expz[k];
+      double wi_n = 0.;
+      if (k + 1 <= nk - 1) {
+        shared_at(k + 1, R0, R1, Sn);
+        double tni_p = 0.;
+        if (k + 2 <= nk - 1) tni_p = k + 2 == nk - 1 ? R1.tn : .5 * (R2.tn + R1.tn);
+        double dtnidz = (k + 1 == nk - 1) ? Sn.tni - Sc.tni : (tni_p - Sc.tni) / 2.;
+  #pragma unroll
+        for (int q = 0; q < 2; ++q) species_at(q, Sn, dtnidz, Y[q], Tn[q]);
+        wi_n = k + 1 < nk - 1 ? .5 * (R1.w + R2.w) : 1.5 * R1.w - .5 * R0.w;
+      }
+      const double dmdzc = Sc.dmdz / Sc.barm;
+      const double dmdzn = k + 1 <= nk - 1 ? Sn.dmdz / Sn.barm : 0.;
+  #pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        double pc, qc, rc, fr;
+        if (k <= nk - 2) {
+          double molp = Tc[q].ax * (rdz + .5 * Tc[q].thdiff);
+          double molr = Tn[q].ax * (rdz - .5 * Tn[q].thdiff);
+          double molq = Tc[q].ax * (rdz - .5 * Tc[q].thdiff) + Tn[q].ax * (rdz + .5 * Tn[q].thdiff);
+          double eddyp = g.expzmid_inv * difk0 * (rdz - .5 * dmdzc);
+          double eddyr = g.expzmid * difk1 * (rdz + .5 * dmdzn);
+          double eddyq = g.expzmid_inv * difk0 * (rdz + .5 * dmdzc) +
+                         g.expzmid * difk1 * (rdz - .5 * dmdzn);
+          pc = molp * rdz - expzk * (eddyp * dfac + .5 * wic) * rdz;
+          rc = molr * rdz - expzk * (eddyr * dfac - .5 * wic) * rdz;
+          qc = -molq * rdz + expzk * (eddyq * dfac * rdz + dtx2inv - Tc[q].sloss);
+          fr = Tc[q].rhs + Tc[q].s0prod;
+          fr = fr * expzk;
+          if (k == 0) {
+            qc = qc + pc * (l1[q] + .5 * l2[q] * dzp) / (l1[q] - .5 * l2[q] * dzp);
+            fr = fr - pc * l3[q] * dzp / (l1[q] - .5 * l2[q] * dzp);
+            pc = 0.;
+          }
+        } else {
+          pc = 1. + .5 * dzp * Tc[q].thdiff;
+          qc = pc - 2.;
+          rc = 0.;
+          fr = -GRAV * sc[q].rmx * fubc * dzp / (P0 * Tc[q].ax * AVO);
+        }
+        double *S = P + 4 * q * rows + k * BC;
+        S[0] = pc;
+        S[rows] = qc;
+        S[2 * rows] = rc;
+        S[3 * rows] = fr;
+      }
+      Sc = Sn;
+      Tc[0] = Tn[0];
+      Tc[1] = Tn[1];
+      wic = wi_n;
+      R0 = R1;
+      R1 = R2;
+    }
+  }
+  __syncthreads();
+  // two systems per column, a thread each
+  if (B.s < 2 && B.solve) {
+    double *S = P + 4 * B.s * rows;
+    block_thomas<BC>(S, S + rows, S + 2 * rows, S + 3 * rows, nk);
+  }
+  __syncthreads();
+  if (!B.active || B.ghost) return;
+  // outputs (:234-237)
+  const bool raw = G.raw_row(j);
+  for (int k = B.s; k < nk; k += BSEG) {
+    const size_t p = G.a3(k, i, j);
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      double x = P[(4 * q + 3) * rows + k * BC];
+      if (B.lat) lateral_value(G, lonb[q], latb[q], k, i, j, x);
+      if (raw) {  // the raw solution; filter_minor and the post pass follow (minor.F:546-597)
+        outs[q][p] = x;
+        continue;
+      }
+      double nm = DTSMOOTH * fc[q][p] + DTSMOOTH_DIV2 * (fctm1[q][p] + x);
+      B.put(G, outs[q], p, x > small ? x : small);
+      B.put(G, outs_nm[q], p, nm > small ? nm : small);
+    }
+  }
+#undef F3
+}
+#define MINOR_BLOCK_KERNEL(name, SA, SB, LIN)                                                       \
+  template <int BC>                                                                                 \
+  __global__ void __launch_bounds__(BC * BSEG) name(tgx_ng_grid g, Geo G, tgx_ng_fields in, tgx_ng_out out, \
+                                                    MinorTerms MT) {                                \
+    minor_block<BC, SA, SB, LIN>(g, G, in, out, MT);                                                \
+  }
+MINOR_BLOCK_KERNEL(minor_block_a_kernel, 2, 3, false)
+MINOR_BLOCK_KERNEL(minor_block_b_kernel, 1, 0, false)
+MINOR_BLOCK_KERNEL(minor_block_b_lin_kernel, 1, 0, true)
+#undef MINOR_BLOCK_KERNEL
+
+// comp_ng.F90:71-457 for grids that do not fill the chip: the elimination is
+// one chain of 3x3 inverses per column, and its rows cost 1,100 operations per
+// level to assemble, so the two are split.  comp_rows_kernel assembles all
+// rows, 16 threads per column; comp_elim_kernel eliminates, four lanes per
+// column; comp_out_kernel applies the post pass, 16 threads per column.  The
+// rows go through the workspace (240 bytes per column and level), which these
+// grids keep in the last-level cache.  comp_kernel's arithmetic throughout.
+// Row values: p (9), q (9), r (9), f (3), column-major blocks; at level nk-1
+// the closed-form top level's three factors and two terms.
+constexpr int CR_NV = 30;
+template <int BC>
+__global__ void __launch_bounds__(BC * BSEG) comp_rows_kernel(tgx_ng_grid g, Geo G, tgx_ng_fields in, tgx_ng_out out,
+                                                              CompTerms CT, double *__restrict__ rw) {
+  const BlockCol<BC> B(G);
+  const int nk = G.nk, i = B.i, j = B.j;
+  if (!B.active) return;
+  const double dz = g.dz, dtx2inv = g.dtx2inv, thdiffalpha = -0.38, rdz = 1. / g.dz;
+  const size_t c2 = G.a2(i, j);
+  const double fhe = g.calc_helium == 0 ? 0. : in.flx_he[c2];
+  if (B.s == 0) out.flx_he[c2] = fhe;
+  int k0, k1;
+  B.run(nk - 1, k0, k1);
+  if (!B.solve || k0 >= k1) return;
+#define F3(f, k) (f)[G.a3((k), i, j)]
+  const double dfac = dfactor_at(g, j);
+  const double tl = in.t_lbc[c2];  // flds%tlbc after dt_ng of this step
+  const double rmass[3] = {RMO2, RMO1, RMHE};
+  const double o2_0 = F3(in.o2, 0), o1_0 = F3(in.o1, 0), he_0 = F3(in.he, 0);
+  double ps0[3];
+  for (int l = 0; l < 3; ++l)
+    ps0[l] = g.b[3 * l + 0] * o2_0 + g.b[3 * l + 1] * o1_0 + g.b[3 * l + 2] * he_0 + g.fb[l];
+  const double embar0 =
+      1. / (ps0[0] * RIO2 + ps0[1] * RIO1 + ps0[2] * RIHE + (1. - ps0[0] - ps0[1] - ps0[2]) * RIN2);
+  struct Lev { double o2i, o1i, hei, embari, tni, dembardz, dtndz, df[3], q; };
+  // Fields read at two neighbouring levels (interface means); one level of
+  // them is carried in registers.
+  struct LR { double o2, o1, he, mbar, tn, w; };
+  // Fields and level constants read at the level being eliminated only.
+  struct LS {
+    double fs[2][3];
+    double rhs[3], hdo2, hdo1, hdhe, expz, difk0, difk1;
+  };
+  auto load_lr = [&](int L, LR &R) {
+    size_t p = G.a3(L, i, j);
+    R.o2 = in.o2[p]; R.o1 = in.o1[p]; R.he = in.he[p]; R.mbar = in.mbar[p]; R.tn = in.tn[p];
+    R.w = in.w[p];
+  };
+  auto load_ls = [&](int L, LS &S) {
+    size_t p = G.a3(L, i, j);
+    const size_t t = G.tile(L, i, j, 0, CI_NV);
+    S.rhs[0] = CT.ci[t]; S.rhs[1] = CT.ci[t + 64]; S.rhs[2] = CT.ci[t + 128];
+    S.fs[0][1] = CT.ci[t + 192]; S.fs[0][2] = CT.ci[t + 256]; S.fs[1][1] = CT.ci[t + 320];
+    S.fs[1][2] = CT.ci[t + 384];
+    S.hdo2 = in.hdo2[p]; S.hdo1 = in.hdo1[p]; S.hdhe = in.hdhe[p];
+    S.expz = g.expz[L]; S.difk0 = g.difk[L]; S.difk1 = g.difk[L + 1];
+  };
+  auto lev_df = [&](Lev &Q) {  // comp_ng.F90:124-126
+    Q.dembardz = Q.dembardz * rdz;
+    Q.dtndz = Q.dtndz * rdz;
+    const TPow tp = tpows(Q.tni);
+    for (int n = 0; n < 3; ++n) Q.df[n] = tp.df[n];
+    Q.q = tp.q;
+  };
+  auto lev0 = [&](const LR &R, Lev &Q) {  // comp_ng.F90:80-97 at the bottom interface
+    Q.o2i = .5 * (ps0[0] + o2_0);
+    Q.o1i = .5 * (ps0[1] + o1_0);
+    Q.hei = .5 * (ps0[2] + he_0);
+    Q.embari = .5 * (embar0 + R.mbar);
+    Q.tni = tl;
+    Q.dembardz = R.mbar - embar0;
+    Q.dtndz = (R.tn - tl) * 2;
+    lev_df(Q);
+  };
+  // interface between A (L-1) and B (L); the global comp.F takes the top
+  // interface's temperature from the level below it (:174-175, :446-449)
+  auto levk = [&](const LR &A, const LR &B, Lev &Q, bool top) {
+    Q.o2i = .5 * (A.o2 + B.o2);
+    Q.o1i = .5 * (A.o1 + B.o1);
+    Q.hei = .5 * (A.he + B.he);
+    Q.embari = .5 * (A.mbar + B.mbar);
+    Q.tni = (G.glb && top) ? A.tn : .5 * (A.tn + B.tn);
+    Q.dembardz = B.mbar - A.mbar;
+    Q.dtndz = B.tn - A.tn;
+    lev_df(Q);
+  };
+  auto alpha_of = [&](const Lev &Q, double *al) {  // :139-151
+    const double *d_ = Q.df;
+    al[0] = -(PHI(1, 4) + (PHI(1, 2) - PHI(1, 4)) * Q.o1i + (d_[0] * PHI(1, 3) - PHI(1, 4)) * Q.hei);
+    al[4] = -(PHI(2, 4) + (PHI(2, 1) - PHI(2, 4)) * Q.o2i + (d_[1] * PHI(2, 3) - PHI(2, 4)) * Q.hei);
+    al[8] = -(d_[2] * PHI(3, 4) + (d_[0] * PHI(3, 1) - d_[2] * PHI(3, 4)) * Q.o2i +
+              (d_[1] * PHI(3, 2) - d_[2] * PHI(3, 4)) * Q.o1i);
+    al[3] = (PHI(1, 2) - PHI(1, 4)) * Q.o2i;
+    al[6] = (d_[0] * PHI(1, 3) - PHI(1, 4)) * Q.o2i;
+    al[1] = (PHI(2, 1) - PHI(2, 4)) * Q.o1i;
+    al[7] = (d_[1] * PHI(2, 3) - PHI(2, 4)) * Q.o1i;
+    al[2] = (d_[0] * PHI(3, 1) - d_[2] * PHI(3, 4)) * Q.hei;
+    al[5] = (d_[1] * PHI(3, 2) - d_[2] * PHI(3, 4)) * Q.hei;
+  };
+  LR r1, r2;
+  load_lr(k0, r1);
+  Lev Qc, Qn;
+  if (k0 == 0) {
+    lev0(r1, Qc);
+  } else {
+    LR rm;
+    load_lr(k0 - 1, rm);
+    levk(rm, r1, Qc, false);
+  }
+  double epm[3], epp[3], akm[9], akp[9], alpha[9];  // levels k (km) and k+1 (kp)
+  double wks3, wks4 = Qc.dembardz / (Qc.embari * 2.);
+  for (int l = 0; l < 3; ++l) epp[l] = 1. - 1. / Qc.embari * (rmass[l] + Qc.dembardz);
+  epp[2] = epp[2] - thdiffalpha * Qc.dtndz / Qc.tni;
+  alpha_of(Qc, alpha);
+  matinv3_r(alpha, akp);
+  double wks1 = Qc.embari * RIN2 * Qc.q * (1. / TAU);
+  for (int n = 0; n < 9; ++n) akp[n] = akp[n] * wks1;
+  double alpha22 = 0, alpha33 = 0, alpha23 = 0, alpha32 = 0, flx00 = 0;
+  for (int k = k0; k < k1; ++k) {
+    LS ls;
+    load_lr(k + 1, r2);
+    load_ls(k, ls);
+    for (int n = 0; n < 9; ++n) akm[n] = akp[n];
+    for (int n = 0; n < 3; ++n) epm[n] = epp[n];
+    levk(r1, r2, Qn, k == nk - 2);
+    const double rem = 1. / Qn.embari;
+    for (int l = 0; l < 3; ++l) epp[l] = 1. - rem * (rmass[l] + Qn.dembardz);
+    if (k != nk - 2) epp[2] = epp[2] - thdiffalpha * Qn.dtndz / Qn.tni;
+    alpha_of(Qn, alpha);
+    matinv3_r(alpha, akp);
+    wks1 = Qn.embari * RIN2 * Qn.q * (1. / TAU);
+    wks3 = wks4;
+    wks4 = Qn.dembardz / (Qn.embari * 2.);
+    for (int n = 0; n < 9; ++n) akp[n] = akp[n] * wks1;
+    double molp[9], molr[9], molq[9], pk[9], rk[9], qk[9], fk[3];
+    for (int isp = 0; isp < 3; ++isp)
+      for (int m = 0; m < 3; ++m) {
+        int e = isp + 3 * m;
+        molp[e] = akm[e] * (rdz + epm[m] / 2.);
+        molr[e] = akp[e] * (rdz - epp[m] / 2.);
+        molq[e] = akm[e] * (rdz - epm[m] / 2.) + akp[e] * (rdz + epp[m] / 2.);
+      }
+    double eddyp = g.expzmid_inv * ls.difk0 * (rdz - wks3);
+    double eddyr = g.expzmid * ls.difk1 * (rdz + wks4);
+    double eddyq = g.expzmid_inv * ls.difk0 * (rdz + wks3) + g.expzmid * ls.difk1 * (rdz - wks4);
+    const double(&fs)[2][3] = ls.fs;
+    const double expzk = ls.expz;
+    const double wik = .5 * (r1.w + r2.w);
+    for (int m = 0; m < 3; ++m)
+      for (int isp = 0; isp < 3; ++isp) {
+        int e = isp + 3 * m;
+        double delta = isp == m ? 1. : 0.;
+        double fsv = (isp < 2 && m < 2) ? fs[isp][m + 1] : 0.;
+        pk[e] = molp[e] * rdz - expzk * delta * rdz * (eddyp * dfac + .5 * wik);
+        rk[e] = molr[e] * rdz - expzk * delta * rdz * (eddyr * dfac - .5 * wik);
+        qk[e] = -molq[e] * rdz + expzk * delta * (eddyq * dfac * rdz + dtx2inv) - expzk * fsv;
+      }
+    fk[0] = expzk * (ls.rhs[0] + ls.hdo2);
+    fk[1] = expzk * (ls.rhs[1] + ls.hdo1);
+    fk[2] = expzk * (ls.rhs[2] + ls.hdhe);
+    if (k == 0) {
+      for (int m = 0; m < 3; ++m)
+        for (int n = 0; n < 3; ++n)
+          for (int isp = 0; isp < 3; ++isp) qk[isp + 3 * m] = qk[isp + 3 * m] + pk[isp + 3 * n] * g.b[3 * n + m];
+      for (int m = 0; m < 3; ++m)
+        for (int isp = 0; isp < 3; ++isp) fk[isp] = fk[isp] - pk[isp + 3 * m] * g.fb[m];
+      for (int n = 0; n < 9; ++n) pk[n] = 0.;
+    } else if (k == nk - 2) {
+      for (int m = 0; m < 3; ++m)
+        for (int isp = 0; isp < 3; ++isp)
+          qk[isp + 3 * m] = qk[isp + 3 * m] + (1. + .5 * epp[m] * dz) / (1. - .5 * epp[m] * dz) * rk[isp + 3 * m];
+      const double *d_ = Qn.df;
+      alpha22 = -(PHI(2, 4) + (PHI(2, 1) - PHI(2, 4)) * Qn.o2i + (d_[1] * PHI(2, 3) - PHI(2, 4)) * Qn.hei);
+      alpha33 = -(d_[2] * PHI(3, 4) + (d_[0] * PHI(3, 1) - d_[2] * PHI(3, 4)) * Qn.o2i +
+                  (d_[1] * PHI(3, 2) - d_[2] * PHI(3, 4)) * Qn.o1i);
+      alpha23 = (d_[1] * PHI(2, 3) - PHI(2, 4)) * Qn.o1i;
+      alpha32 = (d_[1] * PHI(3, 2) - d_[2] * PHI(3, 4)) * Qn.hei;
+      // the mean mass of the interface below (comp_ng.F90:272) or of the top
+      // interface (the global comp.F:632-633)
+      flx00 = (G.glb ? Qn.embari : Qc.embari) * RIN2 * P0 * pow(T00 / r1.tn, 0.25) / (TAU * GRAV);
+      for (int isp = 0; isp < 3; ++isp)
+        fk[isp] = fk[isp] - rk[isp + 3 * 1] * (alpha23 - alpha22) * fhe / (flx00 * (rdz - 0.5 * epp[1])) -
+                  rk[isp + 3 * 2] * (alpha33 - alpha32) * fhe / (flx00 * (rdz - 0.5 * epp[2]));
+      for (int n = 0; n < 9; ++n) rk[n] = 0.;
+    }
+    const size_t t = G.tile(k, i, j, 0, CR_NV);
+    for (int n = 0; n < 9; ++n) {
+      rw[t + n * 64] = pk[n];
+      rw[t + (9 + n) * 64] = qk[n];
+      rw[t + (18 + n) * 64] = rk[n];
+    }
+    for (int n = 0; n < 3; ++n) rw[t + (27 + n) * 64] = fk[n];
+    if (k == nk - 2) {
+      const size_t tt = G.tile(nk - 1, i, j, 0, CR_NV);
+      for (int n = 0; n < 3; ++n) rw[tt + n * 64] = (1. + .5 * epp[n] * dz) / (1. - .5 * epp[n] * dz);
+      rw[tt + 3 * 64] = (alpha23 - alpha22) * fhe / (flx00 * (rdz - 0.5 * epp[1]));
+      rw[tt + 4 * 64] = (alpha33 - alpha32) * fhe / (flx00 * (rdz - 0.5 * epp[2]));
+    }
+    Qc = Qn;
+    r1 = r2;
+  }
+#undef F3
+}
+
+// The elimination and back substitution (comp_ng.F90:281-326), four lanes per
+// column: lane m < 3 holds column m of the pivot block and of gamma while
+// they are formed, and row m of the inverse, so that a row's products,
+// cofactors and substitution are three lanes' work and its two exchanges are
+// quad permutations.  Writes the raw solution to out.o2, out.o1, out.he.
+// A chain of about 35 dependent FP64 operations per level bounds it.
+__global__ void __launch_bounds__(64) comp_elim_kernel(tgx_ng_grid g, Geo G, tgx_ng_out out,
+                                                       const double *__restrict__ rw, double *gs) {
+  const long c = (long)tgx_xcd_block(gridDim.x) * 16 + (threadIdx.x >> 2);
+  const int e = threadIdx.x & 3, m = e < 3 ? e : 2;  // lane 3 repeats lane 2 and stores nothing
+  const long ncol = (long)G.nlond * G.nlatd;
+  const long cc = c < ncol ? c : ncol - 1;
+  const int j = (int)(cc / G.nlond), i = (int)(cc - (long)j * G.nlond);
+  const int edge = G.glb ? 2 : 1;
+  const bool solve = c < ncol && j >= edge && j < G.nlatd - edge && i >= edge && i < G.nlond - edge;
+  const bool put = solve && e < 3;
+  const int nk = G.nk;
+  // values of lanes m+1 and m+2 (cyclic) of the quad
+  auto nxt = [](double v) { return quad<0x09>(v); };   // lanes 0,1,2 <- 1,2,0 (3 <- 0)
+  auto nxt2 = [](double v) { return quad<0x52>(v); };  // lanes 0,1,2 <- 2,0,1 (3 <- 1)
+  auto from = [&](double v, int l) {                   // lane l's value in all lanes, l a constant
+    return l == 0 ? quad<0x00>(v) : l == 1 ? quad<0x55>(v) : quad<0xaa>(v);
+  };
+  struct Row { double p[9], q[3], r[9], f; };
+  auto load = [&](int k, Row &R) {
+    const size_t t = G.tile(min(k, nk - 2), i, j, 0, CR_NV);
+#pragma unroll
+    for (int n = 0; n < 9; ++n) {
+      R.p[n] = rw[t + n * 64];
+      R.r[n] = rw[t + (18 + n) * 64];
+    }
+#pragma unroll
+    for (int n = 0; n < 3; ++n) R.q[n] = rw[t + (9 + 3 * m + n) * 64];
+    R.f = rw[t + (27 + m) * 64];
+  };
+  double gc[3] = {0., 0., 0.};               // gamma(:, m) of the level below
+  double z0 = 0., z1 = 0., z2 = 0., zl = 0.;  // its forward solution; row m's
+  auto level = [&](int k, const Row &a) {
+    double q[3];
+#pragma unroll
+    for (int r = 0; r < 3; ++r) {
+      q[r] = a.q[r];
+#pragma unroll
+      for (int n = 0; n < 3; ++n) q[r] = q[r] - a.p[r + 3 * n] * gc[n];
+    }
+    // the block's columns m+1 (x) and m+2 (y), and all of it for the determinant
+    double x[3], y[3], M[9];
+#pragma unroll
+    for (int r = 0; r < 3; ++r) {
+      x[r] = nxt(q[r]);
+      y[r] = nxt2(q[r]);
+      M[r] = from(q[r], 0);
+      M[3 + r] = from(q[r], 1);
+      M[6 + r] = from(q[r], 2);
+    }
+    const double d = M[0] * M[4] * M[8] - M[0] * M[7] * M[5] - M[3] * M[1] * M[8] + M[3] * M[7] * M[2] +
+                     M[6] * M[1] * M[5] - M[6] * M[4] * M[2];
+    const double ri = 1. / d;
+    // row m of the inverse: the cross product of columns m+1 and m+2 (each
+    // cofactor is matinv3_r's difference or its negative, which rounds alike)
+    const double w0 = (x[1] * y[2] - y[1] * x[2]) * ri;
+    const double w1 = (y[0] * x[2] - x[0] * y[2]) * ri;
+    const double w2 = (x[0] * y[1] - y[0] * x[1]) * ri;
+    double v = a.f;
+    {
+      const double p0 = m == 0 ? a.p[0] : m == 1 ? a.p[1] : a.p[2], p1 = m == 0 ? a.p[3] : m == 1 ? a.p[4] : a.p[5],
+                   p2 = m == 0 ? a.p[6] : m == 1 ? a.p[7] : a.p[8];
+      v = v - p0 * z0;
+      v = v - p1 * z1;
+      v = v - p2 * z2;
+    }
+    const double nz = w0 * from(v, 0) + w1 * from(v, 1) + w2 * from(v, 2);
+    double gr[3];  // gamma(m, :)
+#pragma unroll
+    for (int n = 0; n < 3; ++n) gr[n] = w0 * a.r[3 * n] + w1 * a.r[1 + 3 * n] + w2 * a.r[2 + 3 * n];
+    if (put) {
+      const size_t t = G.tile(k, i, j, 0, 12);
+#pragma unroll
+      for (int n = 0; n < 3; ++n) gs[t + (3 * n + m) * 64] = gr[n];
+      gs[t + (9 + m) * 64] = nz;
+    }
+    z0 = from(nz, 0);
+    z1 = from(nz, 1);
+    z2 = from(nz, 2);
+    zl = nz;
+    // its columns: gamma(n, m) from lane n
+#pragma unroll
+    for (int n = 0; n < 3; ++n) {
+      const double g0 = from(gr[0], n), g1 = from(gr[1], n), g2 = from(gr[2], n);
+      gc[n] = m == 0 ? g0 : m == 1 ? g1 : g2;
+    }
+  };
+  // three levels' loads in flight: four register slots rotate through a loop
+  // unrolled by four
+  Row s0, s1, s2, s3;
+  load(0, s0);
+  load(1, s1);
+  load(2, s2);
+#define ELIM_LEVEL(K, CUR, NEXT)              \
+  if ((K) < nk - 1) {                         \
+    load((K) + 3, NEXT);                      \
+    asm volatile("" ::: "memory");            \
+    level(K, CUR);                            \
+  }
+  for (int k = 0; k < nk - 1; k += 4) {
+    ELIM_LEVEL(k, s0, s3)
+    ELIM_LEVEL(k + 1, s1, s0)
+    ELIM_LEVEL(k + 2, s2, s1)
+    ELIM_LEVEL(k + 3, s3, s2)
+  }
+#undef ELIM_LEVEL
+  // the raw solution; He at its lower-boundary value where it is not solved
+  double *ou = m == 0 ? out.o2 : m == 1 ? out.o1 : out.he;
+  auto store = [&](int k, double u) {
+    if (put) ou[G.a3(k, i, j)] = m == 2 && g.calc_helium == 0 ? g.pshelb : u;
+  };
+  {  // level nk-2, and the closed-form top level (:317-332)
+    const size_t t = G.tile(nk - 1, i, j, 0, CR_NV);
+    double top = rw[t + m * 64] * zl;
+    if (m > 0) top = top + rw[t + (2 + m) * 64];
+    store(nk - 2, zl);
+    store(nk - 1, top);
+  }
+  // back substitution, row m in this lane, four levels read ahead
+  double u0 = from(zl, 0), u1 = from(zl, 1), u2 = from(zl, 2);
+  constexpr int CH = 4;
+  double zb[CH], g0[CH], g1[CH], g2[CH];
+  auto loadb = [&](int k) {
+#pragma unroll
+    for (int q = 0; q < CH; ++q) {
+      const size_t t = G.tile(max(k - q, 0), i, j, 0, 12);
+      zb[q] = gs[t + (9 + m) * 64];
+      g0[q] = gs[t + m * 64];
+      g1[q] = gs[t + (3 + m) * 64];
+      g2[q] = gs[t + (6 + m) * 64];
+    }
+  };
+  loadb(nk - 3);
+  for (int k = nk - 3; k >= 0; k -= CH) {
+    double zc[CH], h0[CH], h1[CH], h2[CH];
+#pragma unroll
+    for (int q = 0; q < CH; ++q) {
+      zc[q] = zb[q]; h0[q] = g0[q]; h1[q] = g1[q]; h2[q] = g2[q];
+    }
+    loadb(k - CH);
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int q = 0; q < CH; ++q)
+      if (k - q >= 0) {
+        double u = zc[q] - h0[q] * u0;
+        u = u - h1[q] * u1;
+        u = u - h2[q] * u2;
+        store(k - q, u);
+        u0 = from(u, 0);
+        u1 = from(u, 1);
+        u2 = from(u, 2);
+      }
+  }
+}
+
+// comp's post pass (comp_ng.F90:386-457, comp.F:936-1022) from the solution
+// in out.o2, out.o1 and out.he: the time smoothing, N2 above its lowest level
+// under 0.01 extrapolated in log(N2 n), the floors and the normalisation, in
+// place.  16 threads share a column and take every 16th level each (a thread
+// per column walked the levels twice, one memory round trip after another).
+// filtered: only the ring filter's latitudes.
+template <int BC>
+__global__ void __launch_bounds__(BC * BSEG) comp_post_block(tgx_ng_grid g, Geo G, tgx_ng_fields in, tgx_ng_out out,
+                                                             int filtered) {
+  __shared__ int skf[BC];         // the lowest level with N2 < 0.01
+  __shared__ double slog[2][BC];  // log(N2 n) there and one level below
+  BlockCol<BC> B(G);
+  if (filtered) {  // the grid covers 2 nfilt rows
+    B.j = B.j < G.nfilt ? 2 + B.j : G.nlat + 2 - 2 * G.nfilt + B.j;
+    B.active = B.i < G.nlond;
+    B.ghost = B.i < 2 || B.i >= G.nlon + 2;
+    B.solve = B.active && !B.ghost;
+  }
+  const int nk = G.nk, i = B.active ? B.i : 0, j = B.active ? B.j : 0;
+  const double small = 1.e-9;
+  if (B.lat && B.s == 0) comp_lateral_column(g, G, in, out, i, j);
+  if (B.s == 0) skf[B.c] = nk;
+  __syncthreads();
+  auto n2_of = [&](size_t p) { return 1. - out.o2[p] - out.o1[p] - out.he[p]; };
+  if (B.solve) {
+    int lo = nk;
+#pragma unroll 4
+    for (int k = B.s; k < nk; k += BSEG)
+      if (n2_of(G.a3(k, i, j)) < 0.01) lo = min(lo, k);
+    if (lo < nk) atomicMin(&skf[B.c], lo);
+  }
+  __syncthreads();
+  const int kf = skf[B.c];
+  const bool extrap = kf >= 1 && kf + 1 < nk;
+  if (B.solve && extrap)  // comp_ng.F90:419-431, comp.F:975-990, by the threads of the two levels
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+      if ((kf - q) % BSEG == B.s) {
+        const size_t p = G.a3(kf - q, i, j);
+        slog[q][B.c] = log(n2_of(p) * in.xnmbar[p]);
+      }
+  __syncthreads();
+  if (!B.solve) return;
+  double n2top = 0., dn2dz = 0., zmtop = 0.;
+  if (extrap) {
+    zmtop = g.zpmid[kf];
+    n2top = slog[0][B.c];
+    dn2dz = G.raw_row(j) ? (n2top - slog[1][B.c]) / g.dz : (n2top - slog[1][B.c]) * (1. / g.dz);
+  }
+#pragma unroll 2
+  for (int k = B.s; k < nk; k += BSEG) {
+    const size_t p = G.a3(k, i, j);
+    const double o2 = out.o2[p], o1 = out.o1[p], he = out.he[p];
+    const double o2nm = DTSMOOTH_DIV2 * (in.o2_nm[p] + o2) + DTSMOOTH * in.o2[p];
+    const double o1nm = DTSMOOTH_DIV2 * (in.o1_nm[p] + o1) + DTSMOOTH * in.o1[p];
+    const double henm = DTSMOOTH_DIV2 * (in.he_nm[p] + he) + DTSMOOTH * in.he[p];
+    double n2 = 1. - o2 - o1 - he;
+    const double n2nm = 1. - o2nm - o1nm - henm;
+    if (extrap && k > kf) n2 = exp(n2top + dn2dz * (g.zpmid[k] - zmtop)) / in.xnmbar[p];
+    const double a = o2 > small ? o2 : small, b = o1 > small ? o1 : small;
+    const double c = he > small ? he : small, d = n2 > small ? n2 : small;
+    const double norm = a + b + c + d;
+    B.put(G, out.o2, p, a / norm);
+    B.put(G, out.o1, p, b / norm);
+    B.put(G, out.he, p, c / norm);
+    const double an = o2nm > small ? o2nm : small, bn = o1nm > small ? o1nm : small;
+    const double cn = henm > small ? henm : small, dn = n2nm > small ? n2nm : small;
+    const double normn = an + bn + cn + dn;
+    B.put(G, out.o2_nm, p, an / normn);
+    B.put(G, out.o1_nm, p, bn / normn);
+    B.put(G, out.he_nm, p, cn / normn);
+  }
+}
+
 }  // namespace ng
 }  // namespace tgx
 
@@ -4769,6 +6262,19 @@ extern "C" int tgx_ng_launch(int which, const tgx_ng_grid *gp, const tgx_ng_fiel
     jb.kind = kind; jb.f = f; jb.out = o; jb.s = sh;
     return jb;
   };
+  // a block kernel whose columns hold `vals` LDS doubles per level, 16 columns
+  // per block or, where those take more than 64 KB, 8
+#define LAUNCH_BLOCK(kern, vals, ...)                                                                              \
+  do {                                                                                                             \
+    const size_t per = sizeof(double) * (vals) * (size_t)G.nk;                                                     \
+    const unsigned rows = (unsigned)G.nlatd;                                                                       \
+    if (16 * per <= BLOCK_LDS)                                                                                     \
+      hipLaunchKernelGGL((kern<16>), dim3((unsigned)((G.nlond + 15) / 16) * rows), dim3(16 * BSEG), 16 * per, s, g, G, \
+                         in, out, __VA_ARGS__);                                                                    \
+    else                                                                                                           \
+      hipLaunchKernelGGL((kern<8>), dim3((unsigned)((G.nlond + 7) / 8) * rows), dim3(8 * BSEG), 8 * per, s, g, G, in, \
+                         out, __VA_ARGS__);                                                                        \
+  } while (0)
   switch (which) {
     case 20:
       if (G.nk <= 64)
@@ -4778,6 +6284,17 @@ extern "C" int tgx_ng_launch(int which, const tgx_ng_grid *gp, const tgx_ng_fiel
         hipLaunchKernelGGL(dt_wave_kernel<2>, gridw, blockw, 0, s, g, G, in, out, (const double *)D(1),
                            (const double *)D(2));
       break;
+    case 38:  // dt, a block per 16 columns: bufs = {(unused), hadv_tn, smooth_tn_nm}
+      LAUNCH_BLOCK(dt_block_kernel, 4, (const double *)D(1), (const double *)D(2));
+      break;
+    case 39:  // duv stage 1, the same way: bufs = {ztmp}
+      LAUNCH_BLOCK(duv_stage1_block, 1, D(0));
+      break;
+    case 40: {  // duv stage 2: bufs = {ztmp, (unused), divx_ztmp, divy_z, unms, vnms, advu, advv}
+      UvTerms UT{D(2), D(3), D(4), D(5), D(6), D(7)};
+      LAUNCH_BLOCK(duv_block_kernel, 8, UT);
+      break;
+    }
     case 25: {  // bufs = {comp input tiles, fs(:,1,0), fs(:,2,0), (unused x3), minor source tiles,
                 //         (unused x2), linear-coefficient tiles, (unused x5), oploss, opprod}
       ChemOut C;
@@ -4824,13 +6341,26 @@ extern "C" int tgx_ng_launch(int which, const tgx_ng_grid *gp, const tgx_ng_fiel
     case 18:
     case 19:
     case 27:
-    case 30: {  // minors: bufs = {ratio tiles (MW_NV), right-hand-side tiles (MR_NV), (unused x8),
+    case 30:
+    case 44:
+    case 45:
+    case 46: {  // minors: bufs = {ratio tiles (MW_NV), right-hand-side tiles (MR_NV), (unused x8),
                 // source tiles (MS_NV), (unused x3)}; N2D's source values are reused by NO after
                 // N2D's solve
       MinorTerms MT{};
       MT.rt = D(1);
       MT.st = D(10);
-      if (which == 1 && g.capture)
+      if (which == 46) {
+        MT.lt = D(14);
+        MT.n2d = out.n2d;
+      }
+      if (which == 44)  // a block per 16 columns, as 1, 2 and 27
+        LAUNCH_BLOCK(minor_block_a_kernel, 8, MT);
+      else if (which == 45)
+        LAUNCH_BLOCK(minor_block_b_kernel, 8, MT);
+      else if (which == 46)
+        LAUNCH_BLOCK(minor_block_b_lin_kernel, 8, MT);
+      else if (which == 1 && g.capture)
         hipLaunchKernelGGL((minor_kernel<2, 3, true>), grid, block, 0, s, g, G, in, out, D(0), MT);
       else if (which == 1)
         hipLaunchKernelGGL((minor_kernel<2, 3, false>), grid, block, 0, s, g, G, in, out, D(0), MT);
@@ -4874,7 +6404,10 @@ extern "C" int tgx_ng_launch(int which, const tgx_ng_grid *gp, const tgx_ng_fiel
     case 29:
     case 31:
     case 32:
-    case 33: {  // O+: bufs = {dj bdotu bvel tpop diffj djbz opbm2 bdopj w2, op, optm1, opout,
+    case 33:
+    case 41:
+    case 42:
+    case 43: {  // O+: bufs = {dj bdotu bvel tpop diffj djbz opbm2 bdopj w2, op, optm1, opout,
                 //           optm1out, bd_diff bd_diffj bd_bvel vdotn bd_djbz opts2, oploss, opprod}
       OpWork W{D(0), D(1), D(2), D(3), D(4), D(5), D(6), D(7), D(8), which >= 31 ? D(21) : nullptr};
       const double *op = D(9), *optm1 = D(10);
@@ -4916,7 +6449,14 @@ extern "C" int tgx_ng_launch(int which, const tgx_ng_grid *gp, const tgx_ng_fiel
         const double *lonb = in.lonb_op + (size_t)sub * 2 * g.nk * (size_t)G.nlatd;
         const double *latb = in.latb_op + (size_t)sub * 2 * g.nk * (size_t)G.ld;
         dim3 gridt((unsigned)(((G.nlond + TILE_X - 1) / TILE_X) * ((G.nlatd + TILE_Y - 1) / TILE_Y)));
-        if (which == 32)  // first of several sub-steps: keeps the factorisation
+        const double *loss = D(19), *prod = D(20);
+        if (which == 41)  // a block per 16 columns, as 29, 32 and 33
+          LAUNCH_BLOCK(oplus_block_kernel, 4, op, optm1, lonb, latb, W, OT, loss, prod, opout, optm1out);
+        else if (which == 42)
+          LAUNCH_BLOCK(oplus_block_keep_kernel, 4, op, optm1, lonb, latb, W, OT, loss, prod, opout, optm1out);
+        else if (which == 43)
+          LAUNCH_BLOCK(oplus_block_reuse_kernel, 4, op, optm1, lonb, latb, W, OT, loss, prod, opout, optm1out);
+        else if (which == 32)  // first of several sub-steps: keeps the factorisation
           hipLaunchKernelGGL((oplus_tile_kernel<false, 1>), gridt, block, 0, s, g, G, in, op, optm1, lonb, latb, W,
                              (const double *)D(19), (const double *)D(20), opout, optm1out);
         else if (which == 33)  // a later sub-step: right-hand side and sweeps
@@ -4950,6 +6490,21 @@ extern "C" int tgx_ng_launch(int which, const tgx_ng_grid *gp, const tgx_ng_fiel
         hipLaunchKernelGGL(duv_wave_stage2<1>, gridw, blockw, 0, s, g, G, in, out, UT);
       else
         hipLaunchKernelGGL(duv_wave_stage2<2>, gridw, blockw, 0, s, g, G, in, out, UT);
+      break;
+    }
+    case 47: {  // comp, rows and elimination apart, before its post pass (48): bufs as 8, then {row tiles (CR_NV)}
+      CompTerms CT{D(1), {D(2), D(3)}};
+      const dim3 gridb((unsigned)((G.nlond + 15) / 16) * (unsigned)G.nlatd), blockb(16 * BSEG);
+      hipLaunchKernelGGL(comp_rows_kernel<16>, gridb, blockb, 0, s, g, G, in, out, CT, D(4));
+      hipLaunchKernelGGL(comp_elim_kernel, dim3((unsigned)((ncol + 15) / 16)), dim3(64), 0, s, g, G, out,
+                         (const double *)D(4), D(0));
+      break;
+    }
+    case 48: {  // comp's post pass: on every latitude (sub 0) or on the ring filter's (sub 1)
+      const unsigned rows = sub ? 2u * (unsigned)G.nfilt : (unsigned)G.nlatd;
+      if (rows)
+        hipLaunchKernelGGL(comp_post_block<16>, dim3((unsigned)((G.nlond + 15) / 16) * rows), dim3(16 * BSEG), 0, s, g,
+                           G, in, out, sub);
       break;
     }
     case 8:

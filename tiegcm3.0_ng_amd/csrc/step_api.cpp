@@ -2,6 +2,7 @@
 // O+ sub-cycle ping-pong (dynamics_ng.F90:99-121).
 #include <hip/hip_runtime.h>
 
+#include <cstdlib>
 #include <map>
 #include <mutex>
 #include <tuple>
@@ -23,9 +24,8 @@ extern "C" int tgx_ringfilter_post_dev(int nf, double *const *f, double *const *
                                        const double *const *fnmi, int kind, int nlev, int nk, int nlon, int nlat,
                                        int ld, int order, int oplus, double dlamda, int nlat_filter,
                                        const int *chunk, const double *gtab, int tord, hipStream_t s);
-extern "C" int tgx_glb_post(int which, int nfilt, const tgx_ng_grid *g, const tgx_ng_fields *in,
-                            const tgx_ng_out *out, const double *op_in, const double *nm_in, double *op_o,
-                            double *nm_o, hipStream_t s);
+extern "C" int tgx_glb_post(int which, const tgx_ng_grid *g, const tgx_ng_fields *in, const tgx_ng_out *out,
+                            double *op_o, double *nm_o, hipStream_t s);
 
 namespace {
 // The ring filters' cos/sin table of the global routines: harmonics 1..3
@@ -46,9 +46,11 @@ thread_local const double *t_glb_tab = nullptr;
 // oplus.F:896-941 (filter_op below the top level, one sub-step), comp.F:925-1022
 // (filter_o2o of O2, O, He, all levels, order 1).  All the routine's fields
 // are filtered in one launch, with the post pass applied to each filtered
-// value (comp's post pass, which needs the whole column, stays its own
-// kernel); tgx_glb_post then adds the periodic points.
-int glb_finish(int which, const tgx_ng_grid *g, const tgx_ng_fields *in, const tgx_ng_out *out,
+// value; comp's post pass, which needs the whole column, follows as its own
+// kernel.  tgx_glb_post then adds the periodic points, which the block
+// kernels (block) have written themselves.
+int comp_post(const tgx_ng_grid *g, const tgx_ng_fields *in, const tgx_ng_out *out, bool filtered, hipStream_t s);
+int glb_finish(int which, bool block, const tgx_ng_grid *g, const tgx_ng_fields *in, const tgx_ng_out *out,
                const double *op_in, const double *nm_in, double *op_o, double *nm_o, hipStream_t s) {
   enum { NONE = 0, DT, DUV, MINOR, OPLUS };  // the post kinds of tgx_ringfilter_post_dev
   double *f[4] = {}, *xnm[4] = {};
@@ -102,7 +104,9 @@ int glb_finish(int which, const tgx_ng_grid *g, const tgx_ng_fields *in, const t
   if (int rc = tgx_ringfilter_post_dev(nf, f, xnm, fi, fm, kind, nlev, g->nk, g->nlon, g->nlat, g->ld, order, oplus,
                                        g->dlamda, nfilt, t_glb->chunk, t_glb_tab, kGlbTableOrder, s))
     return rc;
-  return tgx_glb_post(which, nfilt, g, in, out, op_in, nm_in, op_o, nm_o, s);
+  if (which == 5)
+    if (int rc = comp_post(g, in, out, !block, s)) return rc;
+  return block ? 0 : tgx_glb_post(which, g, in, out, op_o, nm_o, s);
 }
 }  // namespace
 
@@ -131,7 +135,9 @@ enum {
   T_ML = T_MS + 4,  // minor species: NO / N4S source coefficients linear in N2D
   T_OF = T_ML + 6,  // O+: factorisation kept across the sub-cycles of a step
   T_CU = T_OF + 3,  // comp precision form: u (O2, O, He) between refinement sweeps
-  T_N = T_CU + 3
+  T_N = T_CU + 3,
+  T_CR = T_N,       // comp rows of the block form, on grids that use it (30)
+  T_N_BLOCK = T_CR + 30
 };
 
 size_t plane_elems(const tgx_ng_grid *g) { return (size_t)g->nk * (size_t)g->ld * (size_t)(g->nlat + 4); }
@@ -164,6 +170,24 @@ size_t tile_elems(const tgx_ng_grid *g) {
   return (size_t)g->nk * (ncol > nwt ? ncol : nwt);
 }
 
+// Columns below which the Thomas scheme of a routine (oplus, minors, dt, duv,
+// comp) runs the block kernels, 16 threads per column, rather than a thread
+// per column: where the whole forked step stops gaining, since a routine's
+// thread-per-column kernel is latency-bound and leaves room for the others'.
+// Measured, thread per column and block (global step, ms): 3,040 columns x 29
+// levels 0.36 and 0.21; 11,248 x 57 0.86 and 0.55 (ten O+ sub-cycles 2.96 and
+// 1.31); 11,248 x 113 1.63 and 1.23; 17,296 x 57 0.96 and 0.79; 24,640 x 57
+// 1.11 and 1.13, x 113 2.17 and 2.48.  dt and O+ alone gain further up
+// (43,216 x 113: dt 0.58 and 0.37; the step at five O+ sub-cycles 6.36 and
+// 5.86, at one 3.34 and 3.35; 66,976 x 57 loses 3%).  comp's block form moves
+// its rows through the workspace and only pays on the smallest grids (5,200 x
+// 57: step 0.36 and 0.34; 11,248 x 57: 0.55 and 0.65).
+constexpr long kBlockCols[5] = {49152, 20480, 49152, 20480, 5400};
+// (their LDS holds up to 128 levels)
+bool block_grid(const tgx_ng_grid *g, int routine) {
+  return g->nk <= 128 && (long)(g->nlon + 4) * (g->nlat + 4) < kBlockCols[routine];
+}
+
 double *tiles(void *work, const tgx_ng_grid *g, int idx) {
   return (double *)work + (size_t)W_NPLANES * plane_elems(g) + (size_t)idx * tile_elems(g);
 }
@@ -171,7 +195,8 @@ double *tiles(void *work, const tgx_ng_grid *g, int idx) {
 
 extern "C" unsigned long long tgx_ng_workspace_bytes(const tgx_ng_grid *g) {
   if (!g) return 0;
-  return ((unsigned long long)W_NPLANES * plane_elems(g) + (unsigned long long)T_N * tile_elems(g)) *
+  return ((unsigned long long)W_NPLANES * plane_elems(g) +
+          (unsigned long long)(block_grid(g, 4) ? T_N_BLOCK : T_N) * tile_elems(g)) *
          sizeof(double);
 }
 
@@ -245,7 +270,15 @@ enum { K_DT = 0, K_MIN_A, K_MIN_B, K_OP1, K_OP2, K_OP3, K_UV1, K_UV2, K_COMP, K_
        K_DT_PRE, K_MIN_PRE, K_CO_PRE, K_UV_PRE, K_O2O, K_MIN_SRC_A, K_MIN_SRC_B, K_OP_CHEM,
        K_MIN_WA, K_MIN_WB, K_DT_W, K_OP3_W, K_UV2_W, K_COMP_W, K_DT_TILE, K_CHEM, K_MIN_LIN,
        K_MIN_B_LIN, K_UV_TILE, K_OP_TILE, K_MIN_WB_LIN, K_OP1_LITE, K_OP_TILE_KEEP, K_OP_TILE_REUSE,
-       K_COMP_M0, K_COMP_M_REFINE, K_COMP_M_LAST, K_COMP_M_POST };
+       K_COMP_M0, K_COMP_M_REFINE, K_COMP_M_LAST, K_COMP_M_POST, K_DT_BLOCK,
+       K_UV1_BLOCK, K_UV2_BLOCK, K_OP_BLOCK, K_OP_BLOCK_KEEP, K_OP_BLOCK_REUSE, K_MIN_BLOCK_A, K_MIN_BLOCK_B,
+       K_MIN_BLOCK_B_LIN, K_COMP_BLOCK, K_COMP_POST };
+
+namespace {
+int comp_post(const tgx_ng_grid *g, const tgx_ng_fields *in, const tgx_ng_out *out, bool filtered, hipStream_t s) {
+  return tgx_ng_launch(K_COMP_POST, g, in, out, nullptr, filtered ? 1 : 0, s);
+}
+}  // namespace
 
 namespace {
 // Solve scheme of each routine.  The wavefront-per-column cyclic reduction
@@ -292,19 +325,33 @@ bool use_pcr(const tgx_ng_grid *g, int routine) {
 }
 }  // namespace
 
+namespace {
+// Whether a routine's Thomas scheme runs the block kernels.  Capture mode
+// (analysis) and TGX_LARGE_GRID_FORMS=1 in the environment (tests, which check
+// the two against each other: they give the same results bit for bit) run the
+// thread-per-column kernels on every grid.
+bool use_block(const tgx_ng_grid *g, int routine) {
+  const char *large = getenv("TGX_LARGE_GRID_FORMS");
+  return !g->capture && block_grid(g, routine) && !(large && large[0] == '1' && large[1] == 0);
+}
+}  // namespace
+
 extern "C" int tgx_ng_dt(const tgx_ng_grid *g, const tgx_ng_fields *in, const tgx_ng_out *out,
                          void *work, void *stream) {
   if (int rc = check(g, work)) return rc;
   hipStream_t s = (hipStream_t)stream;
   ProfScope prof(R_DT, s);
   void *b[3] = {tiles(work, g, T_DW), plane(work, g, W_DT_T), plane(work, g, W_DT_T + 1)};
-  if (!use_pcr(g, R_DT)) {  // Thomas: the stencils are fused into the column kernel
-    {
+  if (!use_pcr(g, R_DT)) {
+    const bool block = use_block(g, R_DT);
+    if (block)
+      if (int rc = tgx_ng_launch(K_DT_PRE, g, in, out, b, 0, s)) return rc;
+    {  // the tile kernel has the stencils fused in
       ProfScope kern(R_N + R_DT, s);
-      if (int rc = tgx_ng_launch(K_DT_TILE, g, in, out, b, 0, s)) return rc;
+      if (int rc = tgx_ng_launch(block ? K_DT_BLOCK : K_DT_TILE, g, in, out, b, 0, s)) return rc;
     }
     if (!t_glb) return 0;
-    return glb_finish(0, g, in, out, nullptr, nullptr, nullptr, nullptr, s);
+    return glb_finish(0, block, g, in, out, nullptr, nullptr, nullptr, nullptr, s);
   }
   if (int rc = tgx_ng_launch(K_DT_PRE, g, in, out, b, 0, s)) return rc;
   ProfScope kern(R_N + R_DT, s);
@@ -379,30 +426,30 @@ int run_minors(const tgx_ng_grid *g, const tgx_ng_fields *in, const tgx_ng_out *
   if (int rc = tgx_ng_launch(K_MIN_PRE, g, in, out, b, 0, s)) return rc;
   if (chem_ready) TGX_HIP(hipStreamWaitEvent(s, chem_ready, 0));
   // N2D and AR first; NO and N4S use this step's N2D (dynamics_ng.F90:147-165)
-  const bool pcr = use_pcr(g, R_MINORS);
+  const bool pcr = use_pcr(g, R_MINORS), block = !pcr && use_block(g, R_MINORS);
   if (!chem_done)
     if (int rc = tgx_ng_launch(K_MIN_SRC_A, g, in, out, b, 0, s)) return rc;
   {
     ProfScope kern(R_N + R_MINORS, s);  // the N2D + Ar column kernel
-    if (int rc = tgx_ng_launch(pcr ? K_MIN_WA : K_MIN_A, g, in, out, b, 0, s)) return rc;
+    if (int rc = tgx_ng_launch(pcr ? K_MIN_WA : block ? K_MIN_BLOCK_A : K_MIN_A, g, in, out, b, 0, s)) return rc;
   }
   // minor.F:546-597 for N2D and Ar before NO and N4S read this step's N2D
   // (dynamics.F:485-600): filter_minor, then the post pass
   if (t_glb)
-    if (int rc = glb_finish(2, g, in, out, nullptr, nullptr, nullptr, nullptr, s)) return rc;
+    if (int rc = glb_finish(2, block, g, in, out, nullptr, nullptr, nullptr, nullptr, s)) return rc;
   if (chem_done) {  // NO and N4S sources formed in the column kernel from the
                     // step's chemistry pass and this N2D
     void *b2[20];
     for (int q = 0; q < 14; ++q) b2[q] = b[q];
     b2[14] = tiles(work, g, T_ML);
     for (int q = 15; q < 20; ++q) b2[q] = nullptr;
-    if (int rc = tgx_ng_launch(pcr ? K_MIN_WB_LIN : K_MIN_B_LIN, g, in, out, b2, 0, s)) return rc;
+    if (int rc = tgx_ng_launch(pcr ? K_MIN_WB_LIN : block ? K_MIN_BLOCK_B_LIN : K_MIN_B_LIN, g, in, out, b2, 0, s)) return rc;
   } else {
     if (int rc = tgx_ng_launch(K_MIN_SRC_B, g, in, out, b, 0, s)) return rc;
-    if (int rc = tgx_ng_launch(pcr ? K_MIN_WB : K_MIN_B, g, in, out, b, 0, s)) return rc;
+    if (int rc = tgx_ng_launch(pcr ? K_MIN_WB : block ? K_MIN_BLOCK_B : K_MIN_B, g, in, out, b, 0, s)) return rc;
   }
   if (!t_glb) return 0;
-  return glb_finish(3, g, in, out, nullptr, nullptr, nullptr, nullptr, s);
+  return glb_finish(3, block, g, in, out, nullptr, nullptr, nullptr, nullptr, s);
 }
 
 // fe_ready, if given, is recorded on the stream once the last sub-step's
@@ -424,7 +471,7 @@ int run_oplus(const tgx_ng_grid *g, const tgx_ng_fields *in, const tgx_ng_out *o
   // Fe/Fn outputs, which the last sub-step writes.  Capture mode (analysis)
   // assembles every sub-step in full.
   const bool pcr = use_pcr(g, R_OPLUS);
-  const bool reuse = !pcr && nsub > 1 && !g->capture;
+  const bool reuse = !pcr && nsub > 1 && !g->capture, block = !pcr && use_block(g, R_OPLUS);
   for (int sub = 0; sub < nsub; ++sub) {
     // the last sub-step writes the outputs; earlier ones alternate so that
     // a sub-step never reads the buffer it writes
@@ -448,15 +495,18 @@ int run_oplus(const tgx_ng_grid *g, const tgx_ng_fields *in, const tgx_ng_out *o
     if (int rc = tgx_ng_launch(lite ? K_OP1_LITE : K_OP1, g, in, out, b, sub, s)) return rc;
     if (fe_ready && sub == nsub - 1) TGX_HIP(hipEventRecord(fe_ready, s));
     if (int rc = tgx_ng_launch(K_OP2, g, in, out, b, sub, s)) return rc;
-    if (pcr)  // Thomas: the stencils are fused into the column kernel
+    if (pcr || block)  // the tile kernel has the stencils fused in
       if (int rc = tgx_ng_launch(K_OP_PRE, g, in, out, b, sub, s)) return rc;
     {
       ProfScope kern(R_N + R_OPLUS, s);
-      const int col = pcr ? K_OP3_W : !reuse ? K_OP_TILE : sub == 0 ? K_OP_TILE_KEEP : K_OP_TILE_REUSE;
+      const int form = !reuse ? 0 : sub == 0 ? 1 : 2;
+      const int tile[3] = {K_OP_TILE, K_OP_TILE_KEEP, K_OP_TILE_REUSE};
+      const int blk[3] = {K_OP_BLOCK, K_OP_BLOCK_KEEP, K_OP_BLOCK_REUSE};
+      const int col = pcr ? K_OP3_W : block ? blk[form] : tile[form];
       if (int rc = tgx_ng_launch(col, g, in, out, b, sub, s)) return rc;
     }
     if (t_glb)  // oplus.F:896-941: filter_op below the top level, then the post pass
-      if (int rc = glb_finish(4, g, in, out, op_in, nm_in, op_o, nm_o, s)) return rc;
+      if (int rc = glb_finish(4, block, g, in, out, op_in, nm_in, op_o, nm_o, s)) return rc;
     op_in = op_o;
     nm_in = nm_o;
   }
@@ -515,13 +565,18 @@ extern "C" int tgx_ng_duv(const tgx_ng_grid *g, const tgx_ng_fields *in, const t
   b[0] = plane(work, g, W_UV);
   b[1] = tiles(work, g, T_UW);  // Thomas gamma and forward solution (K_UV_TILE)
   for (int q = 0; q < 6; ++q) b[2 + q] = plane(work, g, W_UV + 1 + q);
-  if (!use_pcr(g, R_DUV)) {  // Thomas: stage 1 and the stencils are fused into the column kernel
-    {
+  if (!use_pcr(g, R_DUV)) {
+    const bool block = use_block(g, R_DUV);
+    if (block) {
+      if (int rc = tgx_ng_launch(K_UV1_BLOCK, g, in, out, b, 0, s)) return rc;
+      if (int rc = tgx_ng_launch(K_UV_PRE, g, in, out, b, 0, s)) return rc;
+    }
+    {  // the tile kernel has stage 1 and the stencils fused in
       ProfScope kern(R_N + R_DUV, s);
-      if (int rc = tgx_ng_launch(K_UV_TILE, g, in, out, b, 0, s)) return rc;
+      if (int rc = tgx_ng_launch(block ? K_UV2_BLOCK : K_UV_TILE, g, in, out, b, 0, s)) return rc;
     }
     if (!t_glb) return 0;
-    return glb_finish(1, g, in, out, nullptr, nullptr, nullptr, nullptr, s);
+    return glb_finish(1, block, g, in, out, nullptr, nullptr, nullptr, nullptr, s);
   }
   if (int rc = tgx_ng_launch(K_UV1, g, in, out, b, 0, s)) return rc;
   if (int rc = tgx_ng_launch(K_UV_PRE, g, in, out, b, 0, s)) return rc;
@@ -535,7 +590,7 @@ int run_comp(const tgx_ng_grid *g, const tgx_ng_fields *in, const tgx_ng_out *ou
   hipStream_t s = (hipStream_t)stream;
   if (t_comp_nsweep >= 0) return run_comp_mixed(g, in, out, work, s, chem_done, t_comp_nsweep);
   ProfScope prof(R_COMP, s);
-  void *b[4];
+  void *b[5] = {};
   b[0] = tiles(work, g, T_CE);  // Thomas gamma and forward solution
   b[1] = tiles(work, g, T_CI);  // right-hand-side parts and fs(:,1:2,1:2)
   b[2] = plane(work, g, W_CO + 0);
@@ -545,12 +600,14 @@ int run_comp(const tgx_ng_grid *g, const tgx_ng_fields *in, const tgx_ng_out *ou
   if (!chem_done)
     if (int rc = tgx_ng_launch(K_O2O, g, in, out, b, 0, s)) return rc;
   if (int rc = tgx_ng_launch(K_CO_PRE, g, in, out, b, 0, s)) return rc;
+  const bool pcr = use_pcr(g, R_COMP), block = !pcr && use_block(g, R_COMP);
+  if (block) b[4] = tiles(work, g, T_CR);
   {
     ProfScope kern(R_N + R_COMP, s);
-    if (int rc = tgx_ng_launch(use_pcr(g, R_COMP) ? K_COMP_W : K_COMP, g, in, out, b, 0, s)) return rc;
+    if (int rc = tgx_ng_launch(pcr ? K_COMP_W : block ? K_COMP_BLOCK : K_COMP, g, in, out, b, 0, s)) return rc;
   }
-  if (!t_glb) return 0;
-  return glb_finish(5, g, in, out, nullptr, nullptr, nullptr, nullptr, s);
+  if (!t_glb) return block ? comp_post(g, in, out, false, s) : 0;
+  return glb_finish(5, block, g, in, out, nullptr, nullptr, nullptr, nullptr, s);
 }
 }  // namespace
 
