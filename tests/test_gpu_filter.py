@@ -80,3 +80,36 @@ def test_ringfilter_host_dropin_matches_oracle(pkg, oracle):
         if nc == 0:
             assert np.array_equal(got, f)
         assert float((np.abs(got - ref) / np.abs(ref).max(axis=1, keepdims=True)).max()) <= TOL, (lat, name)
+
+
+@pytest.mark.parametrize("oplus", [0, 1])
+@pytest.mark.parametrize("nlon,order,nk", [
+    (4, 3, 1), (63, 0, 8), (64, 1, 7), (65, 3, 9), (128, 4, 8), (129, 8, 1), (192, 3, 9), (320, 3, 8), (321, 2, 7),
+    (444, 4, 3), (576, 8, 9), (577, 3, 2), (1152, 1, 8), (1153, 3, 3), (2048, 0, 2), (2048, 8, 1)])
+def test_ringfilter_forms_at_their_limits(pkg, oracle, nlon, order, nk, oplus):
+    """Every row length class at its ends, the harmonics of both register
+    forms, levels beside a block's eight, and the chunk counts where lanes
+    share a chunk (up to 32), where they do not, with single longitudes as
+    chunks and with longitudes left over."""
+    import torch
+    chunk = sorted({max(1, min(c, nlon)) for c in (1, 2, 3, 7, 31, 32, 33, 64, 65, nlon // 2, nlon - 1, nlon)})
+    nlat = 2 * len(chunk) + 1
+    ld = nlon + 7
+    dlam = 2 * math.pi / nlon
+    host = _field(nk, nlat, nlon, ld, nlon + order, True)
+    dev = host.cuda()
+    print("case %d %d %d %d" % (nlon, order, nk, oplus), flush=True)
+    pkg.tgx.ringfilter_dev(dev, nlon, nlat, order, bool(oplus), dlam, chunk)
+    torch.cuda.synchronize()
+    got, ref = dev.cpu().numpy(), host.numpy()
+    for lat in range(1, nlat + 1):
+        nc = oracle.ringfilter_chunks(lat, nlat, chunk)
+        j = lat + 1
+        assert np.array_equal(got[:, j, nlon + 4:], ref[:, j, nlon + 4:]), lat
+        if nc == 0:
+            assert np.array_equal(got[:, j], ref[:, j]), lat
+            continue
+        row = np.ascontiguousarray(ref[:, j, :nlon + 4])
+        oracle.ringfilter_row(row, nlon, order, oplus, nc, dlam)
+        scale = np.abs(row).max(axis=1, keepdims=True)
+        assert float((np.abs(got[:, j, :nlon + 4] - row) / scale).max()) <= TOL, (lat, nc)

@@ -6,8 +6,8 @@
 // kept harmonics as wavefront reductions over a table of cos(m ang) and
 // sin(m ang) (the only transcendental work), the residual and the chunk
 // averages in its own LDS region.  Two forms of the launch:
-//  - tgx_ringfilter_dev and the host drop-in: a block of four wavefronts
-//    takes one row and a run of levels and first builds the table in LDS;
+//  - tgx_ringfilter_dev and the host drop-in: a block of eight wavefronts
+//    takes eight levels of one row and first builds the table in LDS;
 //  - the global routines (tgx_ringfilter_post_dev): the table is built once
 //    per call in the workspace, a block is one wavefront and one level (small
 //    blocks that find room beside the other routines' column kernels), all
@@ -24,6 +24,11 @@ namespace ring {
 
 constexpr int kMaxOrder = TGX_RING_MAX_ORDER;
 constexpr int kLdsMax = 65536;  // dynamic LDS of one block
+// Wavefronts of a block of the LDS-table form: they share one table (at 576
+// longitudes and order 3, 27 KB and 3.4 sincos per thread), and two blocks of
+// eight fit in a CU.  0.625 deg, 80 rows of 113 levels: 44 us with eight, 53
+// with four, 64 with two.
+constexpr int kWaves = 8;
 static_assert(64 * 32 >= TGX_RING_MAX_NLON, "ringfilter_kernel<32> covers the longest row");
 
 // The rows of one launch, by value in the kernel arguments: row r is at
@@ -70,24 +75,71 @@ __device__ __forceinline__ void post_point(int kind, double y, double fi, double
   }
 }
 
+// The sum of v over the wavefront, in every lane: DPP row shifts and row
+// broadcasts (no LDS traffic) leave it in lane 63.
+template <int CTRL>
+__device__ __forceinline__ double dpp_add(double v, int rows) {
+  union { double d; int w[2]; } a, b;
+  a.d = v;
+  b.w[0] = rows == 0xf ? __builtin_amdgcn_update_dpp(0, a.w[0], CTRL, 0xf, 0xf, true)
+                       : __builtin_amdgcn_update_dpp(0, a.w[0], CTRL, 0xa, 0xf, false);
+  b.w[1] = rows == 0xf ? __builtin_amdgcn_update_dpp(0, a.w[1], CTRL, 0xf, 0xf, true)
+                       : __builtin_amdgcn_update_dpp(0, a.w[1], CTRL, 0xa, 0xf, false);
+  return v + b.d;
+}
+__device__ __forceinline__ double wave_total(double v) {
+  v = dpp_add<0x111>(v, 0xf);  // row_shr:1, 2, 4, 8: the row's sum in its lane 15
+  v = dpp_add<0x112>(v, 0xf);
+  v = dpp_add<0x114>(v, 0xf);
+  v = dpp_add<0x118>(v, 0xf);
+  v = dpp_add<0x142>(v, 0xa);  // row_bcast:15 into rows 1 and 3
+  union { double d; int w[2]; } a, lo, hi;
+  a.d = v;
+  lo.w[0] = __builtin_amdgcn_readlane(a.w[0], 31);
+  lo.w[1] = __builtin_amdgcn_readlane(a.w[1], 31);
+  hi.w[0] = __builtin_amdgcn_readlane(a.w[0], 63);
+  hi.w[1] = __builtin_amdgcn_readlane(a.w[1], 63);
+  return lo.d + hi.d;
+}
+// Orders this wavefront's LDS writes before its LDS reads (the regions are
+// private to a wavefront).
+__device__ __forceinline__ void lds_wait() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+
 __device__ __forceinline__ double wave_sum(double v) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
   return v;
 }
 
+// Doubles of LDS of one wavefront for rows of nlon longitudes in at most maxc
+// chunks: the residual of a row, whose space the chunk averages and edges take
+// once the chunk sums have been read (2 maxc <= nlon unless a chunk is a single
+// longitude); with lanes sharing a chunk (at most 32 chunks) 64 parts, then 32
+// averages and 32 edges.
+inline int wave_doubles(int nlon, int maxc) {
+  const int w = nlon > 128 ? nlon : 128;
+  return 2 * maxc > w ? 2 * maxc : w;
+}
+
 // NPL: longitudes per lane (nlon <= 64 NPL); lane l holds i = l + 64 t.
 // LDS: the table cs[(m-1) nlon + i], sn[...] for m = 1..order, then per
-// wavefront fx[nlon] (the residual) and avg[nlon].  The launch covers nkp
+// wavefront wl doubles (wave_doubles) of its own.  The launch covers nkp
 // levels of each of the P.nf fields, field-major; wavefront w of block
-// (r, y) takes the levels (y lpw + kk) W + w, kk < lpw, of that order.
+// (r, y) takes level y W + w of that order.
 // GTAB: the table is given in device memory (gtab: cos of harmonics
 // 1..tord at (m-1) nlon + i, then their sin; ring_table_kernel) instead of
-// being built in LDS; the LDS then holds the wavefronts' fx and avg only.
+// being built in LDS; the LDS then holds the wavefronts' own regions only.
 // The kernels below wrap this body.
-template <int NPL, bool GTAB>
+// Bound by FP64 instructions and the wait for one level's loads: one level per
+// wavefront with no loop over levels keeps it under 96 VGPRs (a loop with the
+// next level's loads in flight let the compiler hold each longitude's chunk
+// geometry across levels, 247 VGPRs, two wavefronts per SIMD).  One component
+// at 0.625 deg, order 3: 83.9 us, 1.0 TB/s of its rows, before (LDS shuffles
+// for the sums, a block barrier per level, four divisions by 12 per point); 44.4
+// us, 1.9 TB/s, now.  2.5 deg 21.9 -> 10.7 us, 5 deg 20.4 -> 10.6 us.
+template <int NPL, bool GTAB, int MO>
 __device__ __forceinline__ void ringfilter_body(const Fields &P, long plane, const Rows &R, int nlon, int nkp,
-                                                int order, int oplus, double dlamda, int lpw,
+                                                int order, int oplus, double dlamda, int wl,
                                                 const double *__restrict__ gtab, int tord) {
   extern __shared__ double sh[];
   const int W = blockDim.x >> 6, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -95,205 +147,227 @@ __device__ __forceinline__ void ringfilter_body(const Fields &P, long plane, con
   const int nchnk = R.n[r];
   const int ntab = GTAB ? 0 : order * nlon;
   const double *cs = GTAB ? gtab : sh, *sn = GTAB ? gtab + (size_t)tord * nlon : sh + ntab;
-  double *fx = sh + 2 * ntab + (size_t)wave * 2 * nlon, *avg = fx + nlon;
-  for (int t = threadIdx.x; t < ntab; t += blockDim.x) {
-    const int m = t / nlon + 1, i = t - (m - 1) * nlon;
-    const double ang = (i + 1) * dlamda;
-    double s, c;
-    sincos(m * ang, &s, &c);
-    sh[t] = c;
-    sh[ntab + t] = s;
-  }
+  double *fx = sh + 2 * ntab + (size_t)wave * wl;
   auto trig = [&](int m, int i, double &c, double &s) {
     c = cs[(m - 1) * nlon + i];
     s = sn[(m - 1) * nlon + i];
   };
-  const int n = nlon / nchnk;
-  for (int kk = 0; kk < lpw; ++kk) {
-    const int kq = ((int)blockIdx.y * lpw + kk) * W + wave;
-    const bool live = kq < P.nf * nkp;  // every wavefront reaches every barrier
-    const int q = live ? kq / nkp : 0, k = live ? kq - q * nkp : 0;
-    const bool act = live && k < P.nlev;  // a level to filter (else the top, or nothing)
-    const size_t off = (size_t)k * plane + R.off[r];
-    double *row = P.f[q] + off;
-    double w[NPL], v[NPL];
-    __syncthreads();  // the table is written; this wavefront's fx, avg are free
-    if (act) {
-      // :40-42 the interior longitudes and their mean
-      double s0 = 0.;
+  const int kq = (int)blockIdx.y * W + wave;
+  const bool live = kq < P.nf * nkp;
+  const int q = live ? kq / nkp : 0, k = live ? kq - q * nkp : 0;
+  const bool act = live && k < P.nlev;  // a level to filter (else the top, or none)
+  const size_t off = (size_t)k * plane + R.off[r];
+  double *row = P.f[q] + off;
+  // :40 the interior longitudes, in flight while the table is built
+  double w[NPL], v[NPL];
 #pragma unroll
-      for (int t = 0; t < NPL; ++t) {
-        const int i = lane + 64 * t;
-        w[t] = i < nlon ? row[2 + i] : 0.;
-        if (i < nlon) s0 += w[t];
-      }
-      // :43-53 the Fourier sums of the kept harmonics (ang = i dlamda,
-      // i = 1..nlon), then every sum's wavefront reduction, their steps
-      // interleaved
-      double sum[2 * kMaxOrder + 1];
-      sum[0] = s0;
-#pragma unroll
-      for (int m = 1; m <= kMaxOrder; ++m) {
-        sum[2 * m - 1] = sum[2 * m] = 0.;
-        if (m > order) continue;
-        double sa = 0., sb = 0.;
-#pragma unroll
-        for (int t = 0; t < NPL; ++t) {
-          const int i = lane + 64 * t;
-          if (i < nlon) {
-            double cn, sg;
-            trig(m, i, cn, sg);
-            sa += w[t] * cn;
-            sb += w[t] * sg;
-          }
-        }
-        sum[2 * m - 1] = sa;
-        sum[2 * m] = sb;
-      }
-#pragma unroll
-      for (int o = 32; o > 0; o >>= 1) {
-#pragma unroll
-        for (int q = 0; q <= 2 * kMaxOrder; ++q)
-          if (q <= 2 * order) sum[q] += __shfl_xor(sum[q], o, 64);
-      }
-      // :42, :53-61 the mean and the harmonic part, harmonics in ascending
-      // order as the reference adds them
-      const double a0 = sum[0] / nlon;
-#pragma unroll
-      for (int t = 0; t < NPL; ++t) v[t] = a0;
-#pragma unroll
-      for (int m = 1; m <= kMaxOrder; ++m) {
-        if (m > order) continue;
-        const double am = 2. * sum[2 * m - 1] / nlon, bm = 2. * sum[2 * m] / nlon;
-#pragma unroll
-        for (int t = 0; t < NPL; ++t) {
-          const int i = lane + 64 * t;
-          if (i < nlon) {
-            double cn, sg;
-            trig(m, i, cn, sg);
-            v[t] = v[t] + am * cn + bm * sg;
-          }
-        }
-      }
-      // :63 the residual
-#pragma unroll
-      for (int t = 0; t < NPL; ++t) {
-        const int i = lane + 64 * t;
-        if (i >= nlon) continue;
-        w[t] = w[t] - v[t];
-        fx[i] = w[t];
-      }
+  for (int t = 0; t < NPL; ++t) {
+    const int i = lane + 64 * t;
+    w[t] = act && i < nlon ? row[2 + i] : 0.;
+  }
+  if (!GTAB) {
+    for (int t = threadIdx.x; t < ntab; t += blockDim.x) {
+      const int m = t / nlon + 1, i = t - (m - 1) * nlon;
+      const double ang = (i + 1) * dlamda;
+      double s, c;
+      sincos(m * ang, &s, &c);
+      sh[t] = c;
+      sh[ntab + t] = s;
     }
     __syncthreads();
-    // :65-69 chunk averages, each summed in longitude order; the values are
-    // read from LDS sixteen at a time so that the reads overlap the additions
-    if (act) {
-      for (int c = lane; c < nchnk; c += 64) {
-        const double *q = fx + c * n;
-        double s = 0.;
-        int m = 0;
-        for (; m + 16 <= n; m += 16) {
-          double x[16];
-#pragma unroll
-          for (int u = 0; u < 16; ++u) x[u] = q[m + u];
-#pragma unroll
-          for (int u = 0; u < 16; ++u) s = s + x[u];
-        }
-        for (; m < n; ++m) s = s + q[m];
-        avg[c] = s / n;
+  }
+  if (!live) return;
+  const bool post = P.kind != POST_NONE;
+  double *xr = post ? P.xnm[q] + off : row;
+  if (!act) {  // the top level: spval (dt.F:407-408, duv.F:385-386, :512-513), zero (oplus.F:922-923)
+    if (post) {
+      const double top = P.kind == POST_OPLUS ? 0. : SPVAL;
+      for (int i = lane; i < nlon + 4; i += 64) {
+        row[i] = top;
+        xr[i] = top;
       }
     }
-    __syncthreads();
-    if (!act) {
-      if (live && P.kind != POST_NONE) {  // the top level: spval (dt.F:407-408, duv.F:385-386, :512-513), zero (oplus.F:922-923)
-        const double top = P.kind == POST_OPLUS ? 0. : SPVAL;
-        double *xr = P.xnm[q] + off;
-        for (int i = lane; i < nlon + 4; i += 64) {
-          row[i] = top;
-          xr[i] = top;
-        }
-      }
-      continue;
-    }
-    const bool post = P.kind != POST_NONE;
-    const double *fin = post ? P.fin[q] + off : row, *fnmi = post ? P.fnmi[q] + off : row;  // the step inputs
-    double *xr = post ? P.xnm[q] + off : row;
-    // :71-101 reconstruction from the four neighbouring chunk averages, the
-    // harmonic part added back, the periodic points.  Longitude i = lane + 64 t
-    // is point m (1-based) of chunk c; both advance by 64 = q64 n + r64 per t.
-    const int q64 = 64 / n, r64 = 64 - q64 * n;
-    int c = lane / n, m = lane - c * n + 1;
+    return;
+  }
+  // :42 their mean and :43-53 the Fourier sums of the kept harmonics (ang =
+  // i dlamda, i = 1..nlon), then every sum over the wavefront
+  double sum[2 * MO + 1];
+  sum[0] = 0.;
+#pragma unroll
+  for (int t = 0; t < NPL; ++t) sum[0] += w[t];
+#pragma unroll
+  for (int m = 1; m <= MO; ++m) {
+    sum[2 * m - 1] = sum[2 * m] = 0.;
+    if (m > order) continue;
+    double sa = 0., sb = 0.;
 #pragma unroll
     for (int t = 0; t < NPL; ++t) {
       const int i = lane + 64 * t;
-      if (t > 0) {
-        c += q64;
-        m += r64;
-        if (m > n) {
-          m -= n;
-          ++c;
-        }
+      if (i < nlon) {
+        double cn, sg;
+        trig(m, i, cn, sg);
+        sa += w[t] * cn;
+        sb += w[t] * sg;
       }
-      if (i >= nlon) continue;
-      double x = w[t];
-      if (c < nchnk) {  // points past nchnk * n keep their residual (:84-93 stop at nchnk * n)
-        int im2 = c - 2, im1 = c - 1, ip1 = c + 1, ip2 = c + 2;  // :73-81, periodic in the chunks
-        if (im2 < 0) im2 += nchnk;
-        if (im2 < 0) im2 += nchnk;
-        if (im1 < 0) im1 += nchnk;
-        if (ip1 >= nchnk) ip1 -= nchnk;
-        if (ip2 >= nchnk) ip2 -= nchnk;
-        if (ip2 >= nchnk) ip2 -= nchnk;
+    }
+    sum[2 * m - 1] = sa;
+    sum[2 * m] = sb;
+  }
+#pragma unroll
+  for (int z = 0; z <= 2 * MO; ++z)
+    if (z <= 2 * order) sum[z] = wave_total(sum[z]);
+  // the table is read again below: its 2 order NPL values per lane would
+  // otherwise stay in registers and halve the wavefronts of a SIMD
+  lds_wait();
+  // :42, :53-61 the mean and the harmonic part, harmonics in ascending
+  // order as the reference adds them
+  const double a0 = sum[0] / nlon;
+#pragma unroll
+  for (int t = 0; t < NPL; ++t) v[t] = a0;
+#pragma unroll
+  for (int m = 1; m <= MO; ++m) {
+    if (m > order) continue;
+    const double am = 2. * sum[2 * m - 1] / nlon, bm = 2. * sum[2 * m] / nlon;
+#pragma unroll
+    for (int t = 0; t < NPL; ++t) {
+      const int i = lane + 64 * t;
+      if (i < nlon) {
+        double cn, sg;
+        trig(m, i, cn, sg);
+        v[t] = v[t] + am * cn + bm * sg;
+      }
+    }
+  }
+  // :63 the residual
+#pragma unroll
+  for (int t = 0; t < NPL; ++t) {
+    const int i = lane + 64 * t;
+    if (i >= nlon) continue;
+    w[t] = w[t] - v[t];
+    fx[i] = w[t];
+  }
+  lds_wait();
+  // :65-69 the chunk averages.  gsz lanes sum a chunk's parts of `per`
+  // longitudes and one adds the parts up, where a few chunks of many
+  // longitudes would leave most lanes idle and one lane a chain of n additions.
+  const int n = nlon / nchnk;
+  int gsz = nchnk <= 32 ? 64 / nchnk : 1;
+  while (gsz > 1 && (gsz - 1) * (gsz - 1) >= n) --gsz;
+  double *avg, *edge;
+  if (gsz > 1) {
+    const int per = (n + gsz - 1) / gsz;
+    const int c = lane / gsz, g = lane - c * gsz;
+    double s = 0.;
+    if (c < nchnk) {
+      const double *x = fx + c * n;
+      const int m1 = min((g + 1) * per, n);
+      for (int m = g * per; m < m1; ++m) s = s + x[m];
+    }
+    lds_wait();
+    fx[lane] = s;
+    lds_wait();
+    avg = fx + 64;
+    edge = avg + 32;
+    if (lane < nchnk) {
+      s = 0.;
+      for (int m = 0; m < gsz; ++m) s = s + fx[lane * gsz + m];
+      avg[lane] = s / n;
+    }
+  } else {
+    avg = fx;  // chunk c's average overwrites fx[c], which is read by then (c <= c n)
+    edge = fx + nchnk;
+    for (int c0 = 0; c0 < nchnk; c0 += 64) {
+      const int c = c0 + lane;
+      double s = 0.;
+      if (c < nchnk) {
+        const double *x = fx + c * n;
+        for (int m = 0; m < n; ++m) s = s + x[m];
+      }
+      lds_wait();  // all 64 chunks are read before their averages are written
+      if (c < nchnk) avg[c] = s / n;
+    }
+  }
+  lds_wait();
+  // :71-83 the value at each chunk's left edge from the four neighbouring
+  // averages, periodic in the chunks; a chunk's right edge is the next one's
+  // left edge, term by term
+  for (int c = lane; c < nchnk; c += 64) {
+    int im2 = c - 2, im1 = c - 1, ip1 = c + 1;
+    if (im2 < 0) im2 += nchnk;
+    if (im2 < 0) im2 += nchnk;
+    if (im1 < 0) im1 += nchnk;
+    if (ip1 >= nchnk) ip1 -= nchnk;
+    edge[c] = (-avg[im2] + 7. * avg[im1] + 7. * avg[c] - avg[ip1]) / 12.;
+  }
+  lds_wait();
+  const double *fin = post ? P.fin[q] + off : row, *fnmi = post ? P.fnmi[q] + off : row;  // the step inputs
+  // :84-101 reconstruction, the harmonic part added back, the periodic points.
+  // Longitude i = lane + 64 t is point m (1-based) of chunk c; both advance by
+  // 64 = q64 n + r64 per t.
+  const int q64 = 64 / n, r64 = 64 - q64 * n;
+  int c = lane / n, m = lane - c * n + 1;
+#pragma unroll
+  for (int t = 0; t < NPL; ++t) {
+    const int i = lane + 64 * t;
+    if (t > 0) {
+      c += q64;
+      m += r64;
+      if (m > n) {
+        m -= n;
+        ++c;
+      }
+    }
+    if (i >= nlon) continue;
+    double x = w[t];
+    if (c < nchnk) {  // points past nchnk * n keep their residual (:84-93 stop at nchnk * n)
+      const double left = edge[c], right = edge[c + 1 < nchnk ? c + 1 : 0];
+      if (oplus) {
         const double A0 = avg[c];
-        const double left = (-avg[im2] + 7. * avg[im1] + 7. * A0 - avg[ip1]) / 12.;
-        const double right = (-avg[im1] + 7. * A0 + 7. * avg[ip1] - avg[ip2]) / 12.;
-        if (oplus) {
-          const double fa = (left + right - 2. * A0) / (double)(n * n);
-          const double fb = (3. * A0 - 2. * left - right) / n;
-          x = fa * (3. * (m * m) - 3. * m + 1.) + fb * (2. * m - 1.) + left;
-        } else {
-          x = (left * (n - m) + right * m) / n;
-        }
+        const double fa = (left + right - 2. * A0) / (double)(n * n);
+        const double fb = (3. * A0 - 2. * left - right) / n;
+        x = fa * (3. * (m * m) - 3. * m + 1.) + fb * (2. * m - 1.) + left;
+      } else {
+        x = (left * (n - m) + right * m) / n;
       }
-      const double y = x + v[t];
-      double xo = y, xn = 0.;
-      if (post) {
-        post_point(P.kind, y, fin[2 + i], fnmi[2 + i], xo, xn);
-        xr[2 + i] = xn;
-        if (i == nlon - 2) xr[0] = xn;
-        if (i == nlon - 1) xr[1] = xn;
-        if (i == 0) xr[nlon + 2] = xn;
-        if (i == 1) xr[nlon + 3] = xn;
-      }
-      row[2 + i] = xo;
-      if (i == nlon - 2) row[0] = xo;
-      if (i == nlon - 1) row[1] = xo;
-      if (i == 0) row[nlon + 2] = xo;
-      if (i == 1) row[nlon + 3] = xo;
+    }
+    const double y = x + v[t];
+    double xo = y, xn = 0.;
+    if (post) {
+      post_point(P.kind, y, fin[2 + i], fnmi[2 + i], xo, xn);
+      xr[2 + i] = xn;
+    }
+    row[2 + i] = xo;
+    if (t == 0 && i < 2) {
+      row[nlon + 2 + i] = xo;
+      if (post) xr[nlon + 2 + i] = xn;
+    }
+    if (64 * t + 66 > nlon && i >= nlon - 2) {
+      row[i - (nlon - 2)] = xo;
+      if (post) xr[i - (nlon - 2)] = xn;
     }
   }
 }
 
-template <int NPL>
-__global__ void __launch_bounds__(256) ringfilter_kernel(Fields P, long plane, Rows R, int nlon, int nkp, int order,
-                                                         int oplus, double dlamda, int lpw) {
-  ringfilter_body<NPL, false>(P, plane, R, nlon, nkp, order, oplus, dlamda, lpw, nullptr, 0);
+template <int NPL, int MO>
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(NPL <= 9 ? 4 : 2)))
+ringfilter_kernel(Fields P, long plane, Rows R, int nlon, int nkp, int order, int oplus, double dlamda, int wl) {
+  ringfilter_body<NPL, false, MO>(P, plane, R, nlon, nkp, order, oplus, dlamda, wl, nullptr, 0);
 }
 
 // With the table in device memory: one wavefront per block, at most 128
 // VGPRs, so that four wavefronts of it fit on a SIMD beside the column
 // kernels of the routines running at the same time.
-template <int NPL>
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4)))
-ringfilter_gtab_kernel(Fields P, long plane, Rows R, int nlon, int nkp, int order, int oplus, double dlamda,
+template <int NPL, int MO>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(NPL <= 9 ? 4 : NPL <= 18 ? 3 : 2)))
+ringfilter_gtab_kernel(Fields P, long plane, Rows R, int nlon, int nkp, int order, int oplus, double dlamda, int wl,
                        const double *__restrict__ gtab, int tord) {
-  ringfilter_body<NPL, true>(P, plane, R, nlon, nkp, order, oplus, dlamda, 1, gtab, tord);
+  ringfilter_body<NPL, true, MO>(P, plane, R, nlon, nkp, order, oplus, dlamda, wl, gtab, tord);
 }
 
 // The table of ringfilter_gtab_kernel: cos(m ang) and sin(m ang) of
 // longitude i (ang = (i + 1) dlamda, i < nlon) for m = 1..tord, the values
 // the LDS form computes.
-__global__ void __launch_bounds__(256) ring_table_kernel(double *__restrict__ tab, int nlon, int tord,
+__global__ void __launch_bounds__(64) ring_table_kernel(double *__restrict__ tab, int nlon, int tord,
                                                          double dlamda) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= tord * nlon) return;
@@ -389,11 +463,11 @@ __global__ void __launch_bounds__(64) ringfilter_direct_kernel(double *__restric
   if (lane == 3) row[nlon + 3] = wm[1];
 }
 
-// Whether the table and four wavefronts' rows fit in a block's LDS; if not,
+// Whether the table and the rows of up to kWaves wavefronts fit in a block's LDS; if not,
 // the launcher filters with ringfilter_direct_kernel (one field, no post pass).
-inline bool table_fits(int nlon, int order, int *waves) {
-  const size_t tab = sizeof(double) * 2 * (size_t)order * nlon, per = sizeof(double) * 2 * (size_t)nlon;
-  int W = 4;
+inline bool table_fits(int nlon, int order, int wl, int *waves) {
+  const size_t tab = sizeof(double) * 2 * (size_t)order * nlon, per = sizeof(double) * wl;
+  int W = kWaves;
   while (W > 1 && tab + W * per > kLdsMax) W >>= 1;
   if (waves) *waves = W;
   return tab + W * per <= kLdsMax;
@@ -402,30 +476,36 @@ inline bool table_fits(int nlon, int order, int *waves) {
 template <int NPL>
 int launch(const Fields &P, int nkp, long plane, int nrows, const Rows &R, int nlon, int order, int oplus,
            double dlamda, const double *gtab, int tord, hipStream_t s) {
-  int W;
+  int W, maxc = 1;
+  for (int r = 0; r < nrows; ++r) maxc = R.n[r] > maxc ? R.n[r] : maxc;
+  const int wl = wave_doubles(nlon, maxc);
   if (gtab) {
-    // one wavefront per block and level: small blocks (9 KB of LDS at 576
+    // one wavefront per block and level: small blocks (4.6 KB of LDS at 576
     // longitudes) that find room beside the column kernels of the other
     // routines running at the same time
-    const size_t lds = sizeof(double) * 2 * (size_t)nlon;
+    const size_t lds = sizeof(double) * wl;
     const unsigned ny = (unsigned)((long)P.nf * nkp);
-    hipLaunchKernelGGL(ringfilter_gtab_kernel<NPL>, dim3((unsigned)nrows, ny), dim3(64), lds, s, P, plane, R, nlon,
-                       nkp, order, oplus, dlamda, gtab, tord);
-  } else if (!table_fits(nlon, order, &W)) {
+    if (order <= 3)
+      hipLaunchKernelGGL((ringfilter_gtab_kernel<NPL, 3>), dim3((unsigned)nrows, ny), dim3(64), lds, s, P, plane, R,
+                         nlon, nkp, order, oplus, dlamda, wl, gtab, tord);
+    else
+      hipLaunchKernelGGL((ringfilter_gtab_kernel<NPL, kMaxOrder>), dim3((unsigned)nrows, ny), dim3(64), lds, s, P,
+                         plane, R, nlon, nkp, order, oplus, dlamda, wl, gtab, tord);
+  } else if (!table_fits(nlon, order, wl, &W)) {
     if (P.nf != 1 || P.kind != POST_NONE || nkp != P.nlev)
       return tgx_set_error(TGX_ERR_ARG, "ring filter: fused post pass needs the LDS table (nlon %d, order %d)",
                            nlon, order);
     hipLaunchKernelGGL(ringfilter_direct_kernel, dim3((unsigned)nrows, (unsigned)nkp), dim3(64),
                        sizeof(double) * 3 * (size_t)nlon, s, P.f[0], plane, R, nlon, order, oplus, dlamda);
   } else {
-    // wavefronts per block and levels per wavefront: the table in LDS beside
-    // each wavefront's fx and avg, at most kLdsMax bytes
-    const size_t lds = sizeof(double) * (2 * (size_t)order * nlon + 2 * (size_t)W * nlon);
-    const int lpw = 3;
-    const long nlev = (long)P.nf * nkp;
-    const unsigned ny = (unsigned)((nlev + W * lpw - 1) / (W * lpw));
-    hipLaunchKernelGGL(ringfilter_kernel<NPL>, dim3((unsigned)nrows, ny), dim3(64 * W), lds, s, P, plane, R, nlon,
-                       nkp, order, oplus, dlamda, lpw);
+    const size_t lds = sizeof(double) * (2 * (size_t)order * nlon + (size_t)W * wl);
+    const unsigned ny = (unsigned)(((long)P.nf * nkp + W - 1) / W);
+    if (order <= 3)  // the model's orders: seven sums held instead of seventeen
+      hipLaunchKernelGGL((ringfilter_kernel<NPL, 3>), dim3((unsigned)nrows, ny), dim3(64 * W), lds, s, P, plane, R, nlon,
+                         nkp, order, oplus, dlamda, wl);
+    else
+      hipLaunchKernelGGL((ringfilter_kernel<NPL, kMaxOrder>), dim3((unsigned)nrows, ny), dim3(64 * W), lds, s, P,
+                         plane, R, nlon, nkp, order, oplus, dlamda, wl);
   }
   TGX_HIP(hipGetLastError());
   return 0;
@@ -521,7 +601,7 @@ extern "C" int tgx_ring_table_dev(double *tab, int nlon, int tord, double dlamda
     return tgx_set_error(TGX_ERR_ARG, "ring filter table: nlon %d (4..%d), order %d (1..%d)", nlon, TGX_RING_MAX_NLON,
                          tord, tgx::ring::kMaxOrder);
   const int n = tord * nlon;
-  hipLaunchKernelGGL(tgx::ring::ring_table_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, tab, nlon,
+  hipLaunchKernelGGL(tgx::ring::ring_table_kernel, dim3((unsigned)((n + 63) / 64)), dim3(64), 0, s, tab, nlon,
                      tord, dlamda);
   TGX_HIP(hipGetLastError());
   return 0;
