@@ -3541,17 +3541,19 @@ struct OpWork {
   double *fac;  // the factorisation of the sub-cycles' common matrix (OF_NV values per level)
 };
 struct OpTerms {  // prelude planes of one sub-step
-  const double *bd_diff, *bd_diffj, *bd_bvel, *vdotn, *bd_djbz, *opts2;
+  double *bd_diff, *bd_diffj, *bd_bvel, *vdotn, *bd_djbz, *opts2;
 };
 
 // FULL = false (the middle sub-steps of a sub-cycled step): only the values
 // that depend on O+ (bvel, tp_op, diffj, op/bmod2**2); dj, bdotu and dj*bz
 // stay those of the first sub-step, and Fe, Fn are left to the last one.
+// keep_vni: Fe receives the collision frequency, from which the last
+// sub-step's oplus_sub_prelude forms Fe and Fn.
 template <bool RUNS, bool FULL>  // RUNS false: nrun == 1, the whole column (a fixed loop)
 __global__ void __launch_bounds__(256) oplus_stage1(tgx_ng_grid g, Geo G, tgx_ng_fields in,
                                                     const double *__restrict__ op, OpWork W,
                                                     double *__restrict__ Fe, double *__restrict__ Fn,
-                                                    int nrun) {
+                                                    int nrun, int keep_vni) {
   const int nb = gridDim.x;
   const long tid = (long)tgx_xcd_block(nb) * blockDim.x + threadIdx.x;
   const int nk = G.nk;
@@ -3600,9 +3602,13 @@ __global__ void __launch_bounds__(256) oplus_stage1(tgx_ng_grid g, Geo G, tgx_ng
       dj = dj < cap ? dj : cap;
     }
     double bdotu = bx * in.un[p] + by * in.vn[p] + hj * bz * wni;
-    double wd = vni * diffj * dj;
-    Fe[p] = wd * sncsdip * sndec;
-    Fn[p] = wd * sncsdip * csdec;
+    if (keep_vni) {
+      Fe[p] = vni;
+    } else {
+      double wd = vni * diffj * dj;
+      Fe[p] = wd * sncsdip * sndec;
+      Fn[p] = wd * sncsdip * csdec;
+    }
     W.dj[p] = dj;
     W.bdotu[p] = bdotu;
     W.bvel[p] = bdotu * op[p];
@@ -3638,6 +3644,169 @@ __global__ void __launch_bounds__(256) oplus_stage2(tgx_ng_grid g, Geo G, tgx_ng
     W.bdopj[p] = bdotdh(W.tpop + off, G, i, j, bx, by, cs, g.dlamda, g.dphi) * W.dj[p];
   }
 }
+
+// Stages 1 and 2 and the stencils of a later sub-step (those of FULL = false
+// and KindsOplus, less djbz's, which only the factorisation takes) in one
+// kernel, for the block form: a block covers a TILE_X x TILE_Y tile and a run of
+// STENCIL_RUN levels.  At each level the values that depend on O+ are formed at
+// the tile and its 2-point halo (tp, and tp's horizontal derivative times dj one
+// point inside it) in LDS, where the stencils of the tile read them; the next
+// level's loads are in flight meanwhile.  Separately, the three launches wrote
+// and read back five planes and took 11.6 + 6.7 + 20.3 us on 148x76x57 columns,
+// bound by the latency of each; the values are bitwise the same.
+// LAST: also Fe and Fn, from the collision frequency kept in Fe.
+template <bool LAST>
+__global__ void __launch_bounds__(256) oplus_sub_prelude(tgx_ng_grid g, Geo G, tgx_ng_fields in,
+                                                         const double *__restrict__ op,
+                                                         const double *__restrict__ optm1, OpWork W, OpTerms OT,
+                                                         double shap, double *Fe, double *__restrict__ Fn) {
+  constexpr int TS = TILE_R * TILE_W, TL = TILE_Y * TILE_W;
+  __shared__ double tpl[TS], smo[TS], bdo[TS], dif[TS], bve[TS], obm[TS], tl[TL];
+  const int ntx = (G.nlond + TILE_X - 1) / TILE_X, nty = (G.nlatd + TILE_Y - 1) / TILE_Y;
+  const int nk = G.nk, nrun = (nk + STENCIL_RUN - 1) / STENCIL_RUN;
+  const int b = tgx_xcd_block(gridDim.x);
+  if (b >= ntx * nty * nrun) return;  // uniform per block
+  const int bxi = b % ntx, rr = b / ntx, byj = rr % nty, run = rr / nty;
+  const int k0 = run * STENCIL_RUN, k1 = min(k0 + STENCIL_RUN, nk);
+  const int i0 = bxi * TILE_X, j0 = byj * TILE_Y;
+  const int i = i0 + (int)threadIdx.x % TILE_X, j = j0 + (int)threadIdx.x / TILE_X;
+  const bool inside = i < G.nlond && j < G.nlatd;
+  const double dz = g.dz;
+  // this thread's elements of the tile with its halo (two at most)
+  bool ok[2], in1[2];  // in the domain; and at most one point outside the tile
+  int ei[2], ej[2];
+  size_t qr[2];
+  double bxe[2], bye[2], cse[2], bm2[2];
+#pragma unroll
+  for (int r = 0; r < 2; ++r) {
+    const int e = (int)threadIdx.x + r * 256, ix = e % TILE_W, jx = e / TILE_W;
+    ei[r] = i0 - TILE_H + ix;
+    ej[r] = j0 - TILE_H + jx;
+    ok[r] = e < TS && ei[r] >= 0 && ei[r] < G.nlond && ej[r] >= 0 && ej[r] < G.nlatd;
+    in1[r] = ok[r] && ix > 0 && ix < TILE_W - 1 && jx > 0 && jx < TILE_R - 1;
+    qr[r] = ok[r] ? (size_t)ej[r] * G.ld + ei[r] : 0;
+    const double bm = ok[r] ? in.bmod2[qr[r]] : 1.;
+    bm2[r] = bm * bm;
+    bxe[r] = ok[r] ? in.bx[qr[r]] : 0.;
+    bye[r] = ok[r] ? in.by[qr[r]] : 0.;
+    cse[r] = ok[r] ? g.cs[ej[r]] : 1.;
+  }
+  const size_t c2 = inside ? (size_t)j * G.ld + i : 0;
+  const double bx = inside ? in.bx[c2] : 0., by = inside ? in.by[c2] : 0., csj = inside ? g.cs[j] : 1.;
+  const double bm = inside ? in.bmod2[c2] : 0.;
+  double sncsdip = 0., sndec = 0., csdec = 0.;
+  if (LAST && inside) {
+    sncsdip = sin(in.dipmag[c2]) * cos(in.dipmag[c2]);
+    sndec = in.sndec[c2];
+    csdec = in.csdec[c2];
+  }
+  // tp and O+ at levels k-1, k, k+1; the other fields at level k
+  double tpm[2], tpc[2], tpn[2], opc[2], opn[2], sch[2], bdu[2], djv[2], otm[2];
+  auto tp_at = [&](int r, int L, double &o) {
+    const size_t q = (size_t)L * G.P + qr[r];
+    o = op[q];
+    return (in.te[q] + in.ti[q]) * o;
+  };
+  auto fields = [&](int L) {
+#pragma unroll
+    for (int r = 0; r < 2; ++r)
+      if (ok[r]) {
+        const size_t q = (size_t)L * G.P + qr[r];
+        sch[r] = in.scht[q];
+        bdu[r] = W.bdotu[q];
+        djv[r] = W.dj[q];
+        otm[r] = optm1[q];
+      }
+  };
+#pragma unroll
+  for (int r = 0; r < 2; ++r) {
+    double o;
+    tpm[r] = ok[r] && k0 > 0 ? tp_at(r, k0 - 1, o) : 0.;
+    tpc[r] = ok[r] ? tp_at(r, k0, opc[r]) : 0.;
+    tpn[r] = tpc[r];
+    if (ok[r] && k0 + 1 < nk) tpn[r] = tp_at(r, k0 + 1, opn[r]);
+  }
+  fields(k0);
+  const LdsPlane T{tpl, i0 - TILE_H, j0 - TILE_H}, S{smo, i0 - TILE_H, j0 - TILE_H}, B{bdo, i0 - TILE_H, j0 - TILE_H},
+      D{dif, i0 - TILE_H, j0 - TILE_H}, V{bve, i0 - TILE_H, j0 - TILE_H}, M{obm, i0 - TILE_H, j0 - TILE_H};
+  for (int k = k0; k < k1; ++k) {
+    double djk[2];
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+      djk[r] = djv[r];
+      if (!ok[r]) continue;
+      const int e = (int)threadIdx.x + r * 256;
+      double dtp;
+      if (k == 0) dtp = tpn[r] - tpc[r];
+      else if (k <= nk - 3) dtp = (tpn[r] - tpm[r]) / 2.;
+      else dtp = tpc[r] - tpm[r];
+      tpl[e] = tpc[r];
+      smo[e] = otm[r];
+      dif[e] = 1. / (sch[r] * dz) * dtp + RMOP * GRAV / GASK * opc[r];
+      bve[e] = bdu[r] * opc[r];
+      obm[e] = opc[r] / bm2[r];
+      tpm[r] = tpc[r];
+      tpc[r] = tpn[r];
+      opc[r] = opn[r];
+    }
+    const size_t p = (size_t)k * G.P + c2;
+    double ui0 = 0., ui1 = 0., vi0 = 0., vi1 = 0., vni = 0., djc = 0.;
+    if (inside) {  // :196-209
+      const size_t p1 = k < nk - 1 ? p + G.P : p - G.P;
+      ui0 = in.ui[p];
+      ui1 = in.ui[p1];
+      vi0 = in.vi[p];
+      vi1 = in.vi[p1];
+      if (LAST) {
+        vni = Fe[p];
+        djc = W.dj[p];
+      }
+    }
+    if (k + 1 < k1) {
+#pragma unroll
+      for (int r = 0; r < 2; ++r)
+        if (ok[r] && k + 2 < nk) tpn[r] = tp_at(r, k + 2, opn[r]);
+      fields(k + 1);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < 2; ++r)  // :175-176 one point around the tile
+      if (in1[r])
+        bdo[threadIdx.x + r * 256] = bdotdh(T, G, ei[r], ej[r], bxe[r], bye[r], cse[r], g.dlamda, g.dphi) * djk[r];
+    for (int e = threadIdx.x; e < TL; e += 256) {  // smooth_ng.F90:283-294 for the tile rows and their longitude halo
+      const int ii = i0 - TILE_H + e % TILE_W, jj = j0 + e / TILE_W;
+      if (ii >= 0 && ii < G.nlond && jj < G.nlatd) tl[e] = smooth_lat(S, G, ii, jj, shap);
+    }
+    __syncthreads();
+    if (inside) {
+      W.bdopj[p] = pv(B, G, i, j);
+      OT.bd_diff[p] = bdotdh(B, G, i, j, bx, by, csj, g.dlamda, g.dphi);
+      OT.bd_diffj[p] = bdotdh(D, G, i, j, bx, by, csj, g.dlamda, g.dphi);
+      OT.bd_bvel[p] = bdotdh(V, G, i, j, bx, by, csj, g.dlamda, g.dphi);
+      const double uii = k < nk - 1 ? .5 * (ui0 + ui1) : 1.5 * ui0 - .5 * ui1;
+      const double vii = k < nk - 1 ? .5 * (vi0 + vi1) : 1.5 * vi0 - .5 * vi1;
+      double vx = uii * dflon1(M, G, i, j), vy = vii * dflat1(M, G, i, j);
+      vx = vx / csj;
+      const double vh = 1. / RE * (vx / g.dlamda + vy / g.dphi);
+      OT.vdotn[p] = vh * (bm * bm);
+      const double *row = tl + (j - j0) * TILE_W + TILE_H - i0;  // smooth_ng.F90:296-307
+      const int L1 = G.nlond - 1;
+      const bool edge = i == 0 || i == L1, near = i == 1 || i == L1 - 1;
+      const int i1p = i < L1 ? i + 1 : L1, i1m = i > 0 ? i - 1 : 0;
+      const int i2p = i + 2 <= L1 ? i + 2 : L1, i2m = i >= 2 ? i - 2 : 0;
+      const double t0 = row[i], fm1 = (row[i1p] + row[i1m]) * 0.5, fm2 = (row[i2p] + row[i2m]) * 0.5;
+      const double gen = t0 - shap * (2. * fm2 - 8. * fm1 + 6. * t0), nr = t0 - shap * (-8. * fm1 + 8. * t0);
+      OT.opts2[p] = edge ? t0 : (near ? nr : gen);
+      if (LAST) {
+        const double wd = vni * pv(D, G, i, j) * djc;
+        Fe[p] = wd * sncsdip * sndec;
+        Fn[p] = wd * sncsdip * csdec;
+      }
+    }
+    __syncthreads();  // the next level overwrites the tiles
+  }
+}
+
 // Grids of fewer than 65,536 columns do not fill the chip with one thread
 // per column: there the chemistry pass and O+ stage 1 take runs of two
 // levels, O+ stage 2 single levels, and duv's stage 1 one wavefront per
@@ -6407,7 +6576,10 @@ extern "C" int tgx_ng_launch(int which, const tgx_ng_grid *gp, const tgx_ng_fiel
     case 33:
     case 41:
     case 42:
-    case 43: {  // O+: bufs = {dj bdotu bvel tpop diffj djbz opbm2 bdopj w2, op, optm1, opout,
+    case 43:
+    case 49:
+    case 50:
+    case 51: {  // O+: bufs = {dj bdotu bvel tpop diffj djbz opbm2 bdopj w2, op, optm1, opout,
                 //           optm1out, bd_diff bd_diffj bd_bvel vdotn bd_djbz opts2, oploss, opprod}
       OpWork W{D(0), D(1), D(2), D(3), D(4), D(5), D(6), D(7), D(8), which >= 31 ? D(21) : nullptr};
       const double *op = D(9), *optm1 = D(10);
@@ -6416,18 +6588,28 @@ extern "C" int tgx_ng_launch(int which, const tgx_ng_grid *gp, const tgx_ng_fiel
       if (which == 17) {
         hipLaunchKernelGGL(oplus_chem_kernel, gridp, block, 0, s, g, G, in, D(19), D(20), out.xiop2p,
                            out.xiop2d);
-      } else if (which == 3 || which == 31) {  // 31: the O+-dependent values only
+      } else if (which == 50 || which == 51) {  // a later sub-step's stages 1, 2 and stencils; 51: the last one's
+        const int ntx = (G.nlond + TILE_X - 1) / TILE_X, nty = (G.nlatd + TILE_Y - 1) / TILE_Y;
+        dim3 gridp2((unsigned)(ntx * nty * ((G.nk + STENCIL_RUN - 1) / STENCIL_RUN)));
+        const double shap = g.shapiro / g.nstep_sub;
+        if (which == 51)
+          hipLaunchKernelGGL(oplus_sub_prelude<true>, gridp2, block, 0, s, g, G, in, op, optm1, W, OT, shap, out.Fe,
+                             out.Fn);
+        else
+          hipLaunchKernelGGL(oplus_sub_prelude<false>, gridp2, block, 0, s, g, G, in, op, optm1, W, OT, shap, out.Fe,
+                             out.Fn);
+      } else if (which == 3 || which == 49 || which == 31) {  // 31: the O+-dependent values only; 49: keeps vni in Fe
         const int nrun = oplus_runs(ncol, G.nk, 1);
         dim3 grid1((unsigned)((ncol * nrun + 255) / 256));
         if (which == 31) {
           if (nrun > 1)
-            hipLaunchKernelGGL((oplus_stage1<true, false>), grid1, block, 0, s, g, G, in, op, W, out.Fe, out.Fn, nrun);
+            hipLaunchKernelGGL((oplus_stage1<true, false>), grid1, block, 0, s, g, G, in, op, W, out.Fe, out.Fn, nrun, which == 49);
           else
-            hipLaunchKernelGGL((oplus_stage1<false, false>), grid1, block, 0, s, g, G, in, op, W, out.Fe, out.Fn, 1);
+            hipLaunchKernelGGL((oplus_stage1<false, false>), grid1, block, 0, s, g, G, in, op, W, out.Fe, out.Fn, 1, which == 49);
         } else if (nrun > 1)
-          hipLaunchKernelGGL((oplus_stage1<true, true>), grid1, block, 0, s, g, G, in, op, W, out.Fe, out.Fn, nrun);
+          hipLaunchKernelGGL((oplus_stage1<true, true>), grid1, block, 0, s, g, G, in, op, W, out.Fe, out.Fn, nrun, which == 49);
         else
-          hipLaunchKernelGGL((oplus_stage1<false, true>), grid1, block, 0, s, g, G, in, op, W, out.Fe, out.Fn, 1);
+          hipLaunchKernelGGL((oplus_stage1<false, true>), grid1, block, 0, s, g, G, in, op, W, out.Fe, out.Fn, 1, which == 49);
       } else if (which == 4) {
         const int nrun = oplus_runs(ncol, G.nk, 2);
         dim3 grid2((unsigned)((ncol * nrun + 255) / 256));

@@ -272,7 +272,7 @@ enum { K_DT = 0, K_MIN_A, K_MIN_B, K_OP1, K_OP2, K_OP3, K_UV1, K_UV2, K_COMP, K_
        K_MIN_B_LIN, K_UV_TILE, K_OP_TILE, K_MIN_WB_LIN, K_OP1_LITE, K_OP_TILE_KEEP, K_OP_TILE_REUSE,
        K_COMP_M0, K_COMP_M_REFINE, K_COMP_M_LAST, K_COMP_M_POST, K_DT_BLOCK,
        K_UV1_BLOCK, K_UV2_BLOCK, K_OP_BLOCK, K_OP_BLOCK_KEEP, K_OP_BLOCK_REUSE, K_MIN_BLOCK_A, K_MIN_BLOCK_B,
-       K_MIN_BLOCK_B_LIN, K_COMP_BLOCK, K_COMP_POST };
+       K_MIN_BLOCK_B_LIN, K_COMP_BLOCK, K_COMP_POST, K_OP1_KEEP, K_OP_SUB_PRE, K_OP_SUB_PRE_LAST };
 
 namespace {
 int comp_post(const tgx_ng_grid *g, const tgx_ng_fields *in, const tgx_ng_out *out, bool filtered, hipStream_t s) {
@@ -495,11 +495,17 @@ int run_oplus(const tgx_ng_grid *g, const tgx_ng_fields *in, const tgx_ng_out *o
     if (sub == 0 && !chem_done)
       if (int rc = tgx_ng_launch(K_OP_CHEM, g, in, out, b, sub, s)) return rc;
     const bool lite = reuse && sub > 0 && sub < nsub - 1;
-    if (int rc = tgx_ng_launch(lite ? K_OP1_LITE : K_OP1, g, in, out, b, sub, s)) return rc;
-    if (fe_ready && sub == nsub - 1) TGX_HIP(hipEventRecord(fe_ready, s));
-    if (int rc = tgx_ng_launch(K_OP2, g, in, out, b, sub, s)) return rc;
-    if (pcr || block)  // the tile kernel has the stencils fused in
-      if (int rc = tgx_ng_launch(K_OP_PRE, g, in, out, b, sub, s)) return rc;
+    if (reuse && block && sub > 0) {  // stages 1 and 2 and the stencils in one kernel
+      if (int rc = tgx_ng_launch(lite ? K_OP_SUB_PRE : K_OP_SUB_PRE_LAST, g, in, out, b, sub, s)) return rc;
+      if (fe_ready && sub == nsub - 1) TGX_HIP(hipEventRecord(fe_ready, s));
+    } else {
+      const int first = reuse && block ? K_OP1_KEEP : K_OP1;
+      if (int rc = tgx_ng_launch(lite ? K_OP1_LITE : first, g, in, out, b, sub, s)) return rc;
+      if (fe_ready && sub == nsub - 1) TGX_HIP(hipEventRecord(fe_ready, s));
+      if (int rc = tgx_ng_launch(K_OP2, g, in, out, b, sub, s)) return rc;
+      if (pcr || block)  // the tile kernel has the stencils fused in
+        if (int rc = tgx_ng_launch(K_OP_PRE, g, in, out, b, sub, s)) return rc;
+    }
     {
       ProfScope kern(R_N + R_OPLUS, s);
       const int form = !reuse ? 0 : sub == 0 ? 1 : 2;
