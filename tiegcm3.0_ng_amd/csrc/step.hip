@@ -386,7 +386,20 @@ constexpr int OF_NV = 3;
 // passes of all smoothed fields share one barrier.  Dynamic LDS: one tile per
 // job (+ u, v when a job advects) and one latitude-pass buffer per smoothed
 // field.
-constexpr int STENCIL_RUN = 3;
+//
+// Levels per block: as few as keep the blocks of a launch resident at once (at
+// three per CU, what the registers and LDS of these kernels allow), because a
+// run is a chain of loads and barriers, up to STENCIL_RUN (SUB_RUN for the O+
+// sub-step's kernel, which reads two more levels per run).  O+ with ten
+// sub-cycles on 76x40x29 columns: 298 us with 1, 340 with 3; on 148x76x57 736,
+// 721, 682 and 713 us with 1, 3, 4 and 5; five on 292x148x57: 1402, 1270 and 1250
+// us with 1, 3 and 5.
+constexpr int STENCIL_RUN = 3, SUB_RUN = 5, RESIDENT_BLOCKS = 3 * 256;
+__host__ inline int run_levels(int tiles, int nk, int most) {
+  const int runs = RESIDENT_BLOCKS / tiles;
+  if (runs * most <= nk) return most;
+  return (nk + runs - 1) / runs;
+}
 template <int... K>
 struct StencilKinds {
   static constexpr int n = sizeof...(K);
@@ -409,17 +422,17 @@ struct StencilKinds {
 
 template <class KS, int COMB>
 __global__ void __launch_bounds__(256) stencil_run_kernel(tgx_ng_grid g, Geo G, tgx_ng_fields in,
-                                                          StencilJobs J) {
+                                                          StencilJobs J, int levels) {
   extern __shared__ double smem[];
   constexpr int NJ = KS::n, NT = KS::ntiles(), NS = KS::nsmooth();
   constexpr bool ADV = KS::adv();
   constexpr int TS = TILE_R * TILE_W, TL = TILE_Y * TILE_W;
   const int ntx = (G.nlond + TILE_X - 1) / TILE_X, nty = (G.nlatd + TILE_Y - 1) / TILE_Y;
-  const int nrun = (G.nk + STENCIL_RUN - 1) / STENCIL_RUN;
+  const int nrun = (G.nk + levels - 1) / levels;
   const int b = tgx_xcd_block(gridDim.x);
   if (b >= ntx * nty * nrun) return;  // uniform per block
   const int bxi = b % ntx, rr = b / ntx, byj = rr % nty, run = rr / nty;
-  const int k0 = run * STENCIL_RUN, k1 = min(k0 + STENCIL_RUN, G.nk);
+  const int k0 = run * levels, k1 = min(k0 + levels, G.nk);
   const int i0 = bxi * TILE_X, j0 = byj * TILE_Y;
   const int i = i0 + (int)threadIdx.x % TILE_X, j = j0 + (int)threadIdx.x / TILE_X;
   const bool inside = i < G.nlond && j < G.nlatd;
@@ -3648,7 +3661,7 @@ __global__ void __launch_bounds__(256) oplus_stage2(tgx_ng_grid g, Geo G, tgx_ng
 // Stages 1 and 2 and the stencils of a later sub-step (those of FULL = false
 // and KindsOplus, less djbz's, which only the factorisation takes) in one
 // kernel, for the block form: a block covers a TILE_X x TILE_Y tile and a run of
-// STENCIL_RUN levels.  At each level the values that depend on O+ are formed at
+// levels (run_levels).  At each level the values that depend on O+ are formed at
 // the tile and its 2-point halo (tp, and tp's horizontal derivative times dj one
 // point inside it) in LDS, where the stencils of the tile read them; the next
 // level's loads are in flight meanwhile.  Separately, the three launches wrote
@@ -3659,15 +3672,15 @@ template <bool LAST>
 __global__ void __launch_bounds__(256) oplus_sub_prelude(tgx_ng_grid g, Geo G, tgx_ng_fields in,
                                                          const double *__restrict__ op,
                                                          const double *__restrict__ optm1, OpWork W, OpTerms OT,
-                                                         double shap, double *Fe, double *__restrict__ Fn) {
+                                                         double shap, int levels, double *Fe, double *__restrict__ Fn) {
   constexpr int TS = TILE_R * TILE_W, TL = TILE_Y * TILE_W;
   __shared__ double tpl[TS], smo[TS], bdo[TS], dif[TS], bve[TS], obm[TS], tl[TL];
   const int ntx = (G.nlond + TILE_X - 1) / TILE_X, nty = (G.nlatd + TILE_Y - 1) / TILE_Y;
-  const int nk = G.nk, nrun = (nk + STENCIL_RUN - 1) / STENCIL_RUN;
+  const int nk = G.nk, nrun = (nk + levels - 1) / levels;
   const int b = tgx_xcd_block(gridDim.x);
   if (b >= ntx * nty * nrun) return;  // uniform per block
   const int bxi = b % ntx, rr = b / ntx, byj = rr % nty, run = rr / nty;
-  const int k0 = run * STENCIL_RUN, k1 = min(k0 + STENCIL_RUN, nk);
+  const int k0 = run * levels, k1 = min(k0 + levels, nk);
   const int i0 = bxi * TILE_X, j0 = byj * TILE_Y;
   const int i = i0 + (int)threadIdx.x % TILE_X, j = j0 + (int)threadIdx.x / TILE_X;
   const bool inside = i < G.nlond && j < G.nlatd;
@@ -6404,9 +6417,9 @@ static void launch_stencil_run(const tgx_ng_grid &g, const tgx::ng::Geo &G, cons
                                const tgx::ng::StencilJobs &J, hipStream_t s) {
   using namespace tgx::ng;
   const int ntx = (G.nlond + TILE_X - 1) / TILE_X, nty = (G.nlatd + TILE_Y - 1) / TILE_Y;
-  const int nrun = (G.nk + STENCIL_RUN - 1) / STENCIL_RUN;
+  const int levels = run_levels(ntx * nty, G.nk, STENCIL_RUN), nrun = (G.nk + levels - 1) / levels;
   hipLaunchKernelGGL((stencil_run_kernel<KS, COMB>), dim3((unsigned)(ntx * nty * nrun)), dim3(256), KS::lds_bytes(),
-                     s, g, G, in, J);
+                     s, g, G, in, J, levels);
 }
 
 
@@ -6590,13 +6603,14 @@ extern "C" int tgx_ng_launch(int which, const tgx_ng_grid *gp, const tgx_ng_fiel
                            out.xiop2d);
       } else if (which == 50 || which == 51) {  // a later sub-step's stages 1, 2 and stencils; 51: the last one's
         const int ntx = (G.nlond + TILE_X - 1) / TILE_X, nty = (G.nlatd + TILE_Y - 1) / TILE_Y;
-        dim3 gridp2((unsigned)(ntx * nty * ((G.nk + STENCIL_RUN - 1) / STENCIL_RUN)));
+        const int levels = run_levels(ntx * nty, G.nk, SUB_RUN);
+        dim3 gridp2((unsigned)(ntx * nty * ((G.nk + levels - 1) / levels)));
         const double shap = g.shapiro / g.nstep_sub;
         if (which == 51)
-          hipLaunchKernelGGL(oplus_sub_prelude<true>, gridp2, block, 0, s, g, G, in, op, optm1, W, OT, shap, out.Fe,
+          hipLaunchKernelGGL(oplus_sub_prelude<true>, gridp2, block, 0, s, g, G, in, op, optm1, W, OT, shap, levels, out.Fe,
                              out.Fn);
         else
-          hipLaunchKernelGGL(oplus_sub_prelude<false>, gridp2, block, 0, s, g, G, in, op, optm1, W, OT, shap, out.Fe,
+          hipLaunchKernelGGL(oplus_sub_prelude<false>, gridp2, block, 0, s, g, G, in, op, optm1, W, OT, shap, levels, out.Fe,
                              out.Fn);
       } else if (which == 3 || which == 49 || which == 31) {  // 31: the O+-dependent values only; 49: keeps vni in Fe
         const int nrun = oplus_runs(ncol, G.nk, 1);
