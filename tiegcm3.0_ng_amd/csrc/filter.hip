@@ -369,14 +369,7 @@ ringfilter_gtab_kernel(Fields P, long plane, Rows R, int nlon, int nkp, int orde
 // the LDS form computes.
 __global__ void __launch_bounds__(64) ring_table_kernel(double *__restrict__ tab, int nlon, int tord,
                                                          double dlamda) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= tord * nlon) return;
-  const int m = t / nlon + 1, i = t - (m - 1) * nlon;
-  const double ang = (i + 1) * dlamda;
-  double s, c;
-  sincos(m * ang, &s, &c);
-  tab[t] = c;
-  tab[(size_t)tord * nlon + t] = s;
+  tgx_ring_table_entry(tab, nlon, tord, dlamda, blockIdx.x * blockDim.x + threadIdx.x);
 }
 
 // The same filter where the table does not fit in LDS (long rows, many

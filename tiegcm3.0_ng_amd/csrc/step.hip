@@ -1372,6 +1372,7 @@ struct ChemOut {
   double *st;                          // tiled minor sources: N2D loss, s0prod, N4S loss
   double *lt;                          // tiled N4S s0prod a, b; NO sloss a, b; NO s0prod a, b
   double *oploss, *opprod;             // O+ loss and production
+  double *tab;                         // the ring filters' table of a global step, or null
 };
 
 // Fields chem_kernel reads at two neighbouring levels (interface means, the
@@ -1524,8 +1525,15 @@ __device__ __forceinline__ void chem_level(const tgx_ng_fields &in, const tgx_ng
 // fields read at two levels are loaded once each (runs of about CHEM_RUN
 // levels; shorter on small grids, which would not fill the chip).
 __global__ void __launch_bounds__(256) chem_kernel(tgx_ng_grid g, Geo G, tgx_ng_fields in,
-                                                   tgx_ng_out out, ChemOut C, int nrun) {
-  int nb = gridDim.x;
+                                                   tgx_ng_out out, ChemOut C, int nrun, int tab_blocks) {
+  // the last tab_blocks blocks fill the ring filters' table of a global step,
+  // which no kernel of the step reads before this one ends
+  const int nb = (int)gridDim.x - tab_blocks;
+  if ((int)blockIdx.x >= nb) {
+    tgx_ring_table_entry(C.tab, g.nlon, TGX_GLB_RING_ORDER, g.dlamda,
+                         ((int)blockIdx.x - nb) * (int)blockDim.x + (int)threadIdx.x);
+    return;
+  }
   long t = (long)tgx_xcd_block(nb) * blockDim.x + threadIdx.x;
   const int nk = G.nk;
   long npt = (long)G.nlond * G.nlatd * nrun;
@@ -6478,7 +6486,8 @@ extern "C" int tgx_ng_launch(int which, const tgx_ng_grid *gp, const tgx_ng_fiel
       break;
     }
     case 25: {  // bufs = {comp input tiles, fs(:,1,0), fs(:,2,0), (unused x3), minor source tiles,
-                //         (unused x2), linear-coefficient tiles, (unused x5), oploss, opprod}
+                //         (unused x2), linear-coefficient tiles, (unused x5), oploss, opprod, the ring
+                //         filters' table or null}
       ChemOut C;
       C.ci = D(0);
       C.fs0[0] = D(1);
@@ -6490,8 +6499,10 @@ extern "C" int tgx_ng_launch(int which, const tgx_ng_grid *gp, const tgx_ng_fiel
         return tgx_set_error(1, "chem_kernel: a field of %d levels x %ld points exceeds 4 GiB", G.nk, (long)G.P);
       const int nrun = small_grid(ncol) ? (G.nk + 1) / 2 : chem_runs(G.nk);
       long nt = (long)G.nlond * G.nlatd * nrun;
-      dim3 gridc((unsigned)((nt + 255) / 256));
-      hipLaunchKernelGGL(chem_kernel, gridc, block, 0, s, g, G, in, out, C, nrun);
+      C.tab = D(17);
+      const int tab_blocks = C.tab ? (TGX_GLB_RING_ORDER * g.nlon + 255) / 256 : 0;
+      dim3 gridc((unsigned)((nt + 255) / 256) + (unsigned)tab_blocks);
+      hipLaunchKernelGGL(chem_kernel, gridc, block, 0, s, g, G, in, out, C, nrun, tab_blocks);
       break;
     }
     case 28: {  // duv with stage 1 and the stencils fused: bufs = {ztmp (unused), Thomas tiles (UW_NV)}

@@ -30,7 +30,7 @@ extern "C" int tgx_glb_post(int which, const tgx_ng_grid *g, const tgx_ng_fields
 namespace {
 // The ring filters' cos/sin table of the global routines: harmonics 1..3
 // (the largest order they filter with), at the end of the workspace.
-constexpr int kGlbTableOrder = 3;
+constexpr int kGlbTableOrder = TGX_GLB_RING_ORDER;
 // The global grid of the tgx_glb_* call running on this host thread, or null
 // for a nest domain.  The routines below then run the Thomas scheme with the
 // global grid's column kernels and, after each column kernel, the ring filter
@@ -377,6 +377,7 @@ int run_chem(const tgx_ng_grid *g, const tgx_ng_fields *in, const tgx_ng_out *ou
              hipStream_t s) {
   void *b[20];
   chem_bufs(work, g, b);
+  b[17] = t_glb ? const_cast<double *>(t_glb_tab) : nullptr;  // a global step's ring filter table
   return tgx_ng_launch(K_CHEM, g, in, out, b, 0, s);
 }
 // The parts of a routine that tgx_ng_step queues separately.
@@ -622,8 +623,9 @@ int run_comp(const tgx_ng_grid *g, const tgx_ng_fields *in, const tgx_ng_out *ou
 
 // Concurrency of the step: oplus, the minor species, dt and comp read only
 // the step's inputs and write disjoint outputs and workspace planes, so they
-// run on four streams forked from the caller's stream; duv needs dt's TN and
-// oplus' Fe/Fn and joins both.  All streams have the default priority.
+// run on streams forked from the caller's (three, or on small grids one:
+// two_streams); duv needs dt's TN and oplus' Fe/Fn and joins both.  All streams
+// have the default priority.
 namespace {
 // The fork streams and events belong to the calling host thread (one set per
 // thread and device): calls from several threads never share an event, and
@@ -744,6 +746,19 @@ extern "C" int tgx_ng_scheme_choice(const tgx_ng_grid *g, int routine) {
   return c == TGX_SCHEME_AUTO ? TGX_SCHEME_PCR : c;
 }
 
+// Small grids outside a graph run O+, dt and duv on the caller's stream and the
+// minor species and comp on one other.  There the step is bound by the host:
+// a launch costs it 3 us, but a wait for another stream's event 8-10 us, and
+// two streams take three waits where four take eight.  72x36x29: 235 us per step
+// with two streams, 290 with four, 270 on one; 100x50x57 nest with five O+
+// sub-cycles: 488 and 510 us; but 144x72x57 with ten: 1185 and 1140 us, and in a
+// graph, where waits cost the host nothing, four are faster at any size.
+static bool two_streams(const tgx_ng_grid *g, hipStream_t s) {
+  if ((long)(g->nlon + 4) * (g->nlat + 4) * g->nk > 450000) return false;
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing(s, &st) == hipSuccess && st == hipStreamCaptureStatusNone;
+}
+
 extern "C" int tgx_ng_step(const tgx_ng_grid *g, const tgx_ng_fields *in, const tgx_ng_out *out,
                            void *work, void *stream) {
   // dynamics_ng.F90 order: oplus (:99-121), minors (:147-165), dt (:203),
@@ -753,7 +768,9 @@ extern "C" int tgx_ng_step(const tgx_ng_grid *g, const tgx_ng_fields *in, const 
     if (int rc = tgx_ng_autotune(g, in, out, work, stream)) return rc;
   Fork *F = nullptr;
   if (int rc = get_fork(&F)) return rc;
-  hipStream_t s0 = (hipStream_t)stream, sa = F->s[0], sb = F->s[1], sc = F->s[2];
+  const bool two = two_streams(g, (hipStream_t)stream);
+  hipStream_t s0 = (hipStream_t)stream, sb = F->s[1];
+  hipStream_t sa = two ? s0 : F->s[0], sc = two ? sb : F->s[2];
   // Fork: every stream starts after what the caller queued before the step,
   // stream b at once (ev[5]) and a and c after the chemistry pass (ev[0]).
   // From here on every return joins the forked streams back into s0, so that a
@@ -792,10 +809,12 @@ extern "C" int tgx_ng_step(const tgx_ng_grid *g, const tgx_ng_fields *in, const 
   if (int rc = run_minors(g, in, out, work, sb, true, PART_PRELUDE)) return rc;
   if (int rc = run_chem(g, in, out, work, s0)) return rc;
   TGX_HIP(hipEventRecord(F->ev[0], s0));
-  TGX_HIP(join.fork(0, 0));
-  TGX_HIP(join.fork(2, 0));
-  // stream a; ev[4]: its Fe/Fn are written (the last sub-step's stage 1)
-  if (int rc = run_oplus(g, in, out, work, sa, true, g->nstep_sub, F->ev[4])) return rc;
+  if (!two) {
+    TGX_HIP(join.fork(0, 0));
+    TGX_HIP(join.fork(2, 0));
+  }
+  // ev[4]: its Fe/Fn are written (the last sub-step's stage 1)
+  if (int rc = run_oplus(g, in, out, work, sa, true, g->nstep_sub, two ? nullptr : F->ev[4])) return rc;  // stream a
   if (int rc = tgx_ng_dt(g, in, out, work, s0)) return rc;       // caller's stream
   TGX_HIP(hipStreamWaitEvent(sb, F->ev[0], 0));
   if (int rc = run_minors(g, in, out, work, sb, true, PART_COLUMNS)) return rc;  // stream b
@@ -803,7 +822,7 @@ extern "C" int tgx_ng_step(const tgx_ng_grid *g, const tgx_ng_fields *in, const 
   // duv reads Fe/Fn of oplus and no other output or workspace region of it,
   // so it starts while the rest of the O+ sub-step (its column solve, ring
   // filter, post pass) still runs
-  TGX_HIP(hipStreamWaitEvent(s0, F->ev[4], 0));
+  if (!two) TGX_HIP(hipStreamWaitEvent(s0, F->ev[4], 0));
   return tgx_ng_duv(g, in, out, work, s0);  // the fork streams joined on return
 }
 
@@ -871,12 +890,16 @@ struct GlbScope {
 double *glb_table(const tgx_ng_grid *g, void *work) {
   return (double *)((char *)work + tgx_ng_workspace_bytes(g));
 }
+// A step's chemistry pass fills the table, a routine called on its own gets it
+// from a launch before (whole_step false): one launch of 2.5 deg's step that
+// took 7 us and a gap of 10 before the pass.
 int glb_call(RoutineFn fn, const tgx_glb_grid *gg, const tgx_ng_fields *in, const tgx_ng_out *out, void *work,
-             void *stream) {
+             void *stream, bool whole_step = false) {
   if (int rc = check_glb(gg)) return rc;
   if (!work) return tgx_set_error(TGX_ERR_ARG, "tgx_glb: null workspace");
   double *tab = glb_table(&gg->g, work);
-  if (int rc = tgx_ring_table_dev(tab, gg->g.nlon, kGlbTableOrder, gg->g.dlamda, (hipStream_t)stream)) return rc;
+  if (!whole_step)
+    if (int rc = tgx_ring_table_dev(tab, gg->g.nlon, kGlbTableOrder, gg->g.dlamda, (hipStream_t)stream)) return rc;
   GlbScope scope(gg, tab);
   return fn(&gg->g, in, out, work, stream);
 }
@@ -908,9 +931,9 @@ extern "C" int tgx_glb_comp(const tgx_glb_grid *gg, const tgx_ng_fields *in, con
 }
 extern "C" int tgx_glb_step(const tgx_glb_grid *gg, const tgx_ng_fields *in, const tgx_ng_out *out, void *work,
                             void *stream) {
-  return glb_call(tgx_ng_step, gg, in, out, work, stream);
+  return glb_call(tgx_ng_step, gg, in, out, work, stream, true);
 }
 extern "C" int tgx_glb_step_serial(const tgx_glb_grid *gg, const tgx_ng_fields *in, const tgx_ng_out *out,
                                    void *work, void *stream) {
-  return glb_call(tgx_ng_step_serial, gg, in, out, work, stream);
+  return glb_call(tgx_ng_step_serial, gg, in, out, work, stream, true);
 }

@@ -36,3 +36,17 @@ __device__ __forceinline__ int tgx_xcd_block(int nblocks) {
   int q = nblocks / nxcd, r = nblocks % nxcd;
   return x * q + (x < r ? x : r) + slot;
 }
+
+// Harmonics of the ring filters' table of a global grid (the routines keep at most three).
+#define TGX_GLB_RING_ORDER 3
+// Entry t of the ring filters' table: cos(m ang) and sin(m ang) of longitude i
+// (ang = (i + 1) dlamda) at (m - 1) nlon + i and tord nlon further, m = 1..tord.
+__device__ __forceinline__ void tgx_ring_table_entry(double *tab, int nlon, int tord, double dlamda, int t) {
+  if (t >= tord * nlon) return;
+  const int m = t / nlon + 1, i = t - (m - 1) * nlon;
+  const double ang = (i + 1) * dlamda;
+  double s, c;
+  sincos(m * ang, &s, &c);
+  tab[t] = c;
+  tab[(size_t)tord * nlon + t] = s;
+}
