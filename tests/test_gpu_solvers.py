@@ -322,3 +322,42 @@ def test_partitioned_solver_bad_segments(pkg, nblk, n):
         y = torch.zeros_like(x)
         pkg.tgx.trsolv_dev(*sys_, y, 0, n - 1, scheme=1)
         assert torch.equal(x[2::3], y[2::3])
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 57, 63, 64, 65, 95, 96, 128, 255, 256, 511, 512])
+def test_thomas_scheme_bit_for_bit(pkg, n):
+    """The Thomas scheme in the reference's order, trsolv.F:38-54, exactly: rows
+    at the limits of each LDS form and beyond (512), blocks with and without
+    columns left over, columns from the middle of the batch, rows from the middle
+    of the levels; nothing else of x is written, and what no equation reads (NaN
+    here) does not enter."""
+    import torch
+    rng = np.random.default_rng(n)
+    for ncol, col0, k1, pad in ((1, 0, 0, 0), (7, 3, 1, 2), (16, 0, 0, 1), (33, 5, 2, 0)):
+        ldk = k1 + n + pad
+        tot = col0 + ncol + 2
+        a, c = -rng.uniform(.5, 2., (tot, ldk)), -rng.uniform(.5, 2., (tot, ldk))
+        b = -(a + c) + rng.uniform(.1, 1., (tot, ldk))
+        f = rng.normal(0., 5., (tot, ldk))
+        k2 = k1 + n - 1
+        a[:, k1] = np.nan
+        c[:, k2] = np.nan
+        x = np.full((tot, ldk), -7.)
+        ref = x.copy()
+        cols = slice(col0, col0 + ncol)
+        w1, w3 = b[cols, k1], f[cols, k1] / b[cols, k1]
+        ref[cols, k1] = w3
+        w2s = np.zeros((ncol, ldk))
+        for k in range(k1 + 1, k2 + 1):
+            w2 = c[cols, k - 1] / w1
+            w2s[:, k - 1] = w2
+            w1 = b[cols, k] - a[cols, k] * w2
+            w3 = (f[cols, k] - a[cols, k] * w3) / w1
+            ref[cols, k] = w3
+        for k in range(k2 - 1, k1 - 1, -1):
+            ref[cols, k] = ref[cols, k] - w2s[:, k] * ref[cols, k + 1]
+        d = [torch_dev(v) for v in (a, b, c, f, x)]
+        print("case", n, ncol, flush=True)
+        pkg.tgx.trsolv_dev(*d, k1, k2, scheme=pkg.tgx.SCHEME_THOMAS, col0=col0, ncol=ncol)
+        torch.cuda.synchronize()
+        assert np.array_equal(d[4].cpu().numpy(), ref), (n, ncol)

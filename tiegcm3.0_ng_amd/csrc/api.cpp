@@ -180,7 +180,8 @@ int run_scalar(int scheme, const double *a, const double *b, const double *c, co
   }
   void *w2 = nullptr;
   size_t need = sizeof(double) * (size_t)ldk * (size_t)ncol;
-  if (int rc = get_scratch(need, s, &w2)) return rc;
+  if (k2 - k1 + 1 > TGX_THOMAS_LDS_ROWS)
+    if (int rc = get_scratch(need, s, &w2)) return rc;
   return tgx_launch_thomas_f64(a, b, c, f, x, (double *)w2, ldk, k1, k2, col0, ncol, s);
 }
 

@@ -3,9 +3,9 @@
 //   blktri              (2x2 block tridiagonal, duv.F:801-908)
 //   comp 3x3 elimination (comp_ng.F90:281-326 on pre-assembled blocks)
 //
-// Thread per column in the reference's operation order (bit-compatible with
-// the Fortran when FP contraction is off): the scalar Thomas scheme, and block
-// columns beyond 256 rows.  segsolve.hip holds the partitioned solver the
+// In the reference's operation order (bit-compatible with the Fortran when FP
+// contraction is off): the scalar Thomas scheme, from LDS or, beyond 511 rows,
+// a thread per column, and block columns beyond 256 rows.  segsolve.hip holds the partitioned solver the
 // other calls take.
 // Beside them a mixed-precision PCR, one wavefront (or half) per column: FP32
 // reduction in registers with cross-lane shuffles, FP64 residual r = f - A x,
@@ -44,6 +44,67 @@ __global__ void __launch_bounds__(256) thomas_kfast_f64(
     double xk = x[o + k] - w2c[k] * xn;
     x[o + k] = xk;
     xn = xk;
+  }
+}
+
+// The same elimination with the columns staged through LDS: the block's
+// wavefronts load CPB columns' levels (contiguous in memory, so coalesced),
+// CPB lanes eliminate from LDS in the order above, and the wavefronts store x.
+// Rows of a column are n | 1 doubles apart in LDS (no bank conflict between
+// lanes at the same level).  Bound by the chain of two divisions per level on
+// CPB lanes; a thread per column read its own column 8 bytes at a time and wrote
+// the ratios to HBM.
+template <int CPB>
+__global__ void __launch_bounds__(256) thomas_lds_f64(
+    const double *__restrict__ a, const double *__restrict__ b, const double *__restrict__ c,
+    const double *__restrict__ f, double *__restrict__ x, int ldk, int k1, int k2, int col0, int ncol) {
+  extern __shared__ double sh[];
+  const int n = k2 - k1 + 1, st = n | 1;
+  double *A = sh, *B = A + CPB * st, *C = B + CPB * st, *F = C + CPB * st;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int t0 = tgx_xcd_block(gridDim.x) * CPB, nc = min(CPB, ncol - t0);
+  const size_t o = (size_t)(col0 + t0) * (size_t)ldk + k1;
+  for (int q = wave; q < nc; q += 4) {
+    const size_t oq = o + (size_t)q * ldk;
+    for (int k = lane; k < n; k += 64) {
+      const double av = a[oq + k], bv = b[oq + k], cv = c[oq + k], fv = f[oq + k];
+      A[q * st + k] = av;
+      B[q * st + k] = bv;
+      C[q * st + k] = cv;
+      F[q * st + k] = fv;
+    }
+  }
+  __syncthreads();
+  if ((int)threadIdx.x < nc) {
+    const double *Aq = A + threadIdx.x * st, *Bq = B + threadIdx.x * st;
+    double *Cq = C + threadIdx.x * st, *Fq = F + threadIdx.x * st;  // then the ratios and x
+    double w1 = Bq[0], w3 = Fq[0] / w1, ck = Cq[0];
+    double an = Aq[min(1, n - 1)], bn = Bq[min(1, n - 1)], fn = Fq[min(1, n - 1)], cn = Cq[min(1, n - 1)];
+    Fq[0] = w3;
+    for (int k = 1; k < n; ++k) {
+      const double ak = an, bk = bn, fk = fn;
+      const double w2 = ck / w1;
+      ck = cn;
+      const int kn = min(k + 1, n - 1);
+      an = Aq[kn];
+      bn = Bq[kn];
+      fn = Fq[kn];
+      cn = Cq[kn];
+      Cq[k - 1] = w2;
+      w1 = bk - ak * w2;
+      w3 = (fk - ak * w3) / w1;
+      Fq[k] = w3;
+    }
+    double xn = w3;
+    for (int k = n - 2; k >= 0; --k) {
+      xn = Fq[k] - Cq[k] * xn;
+      Fq[k] = xn;
+    }
+  }
+  __syncthreads();
+  for (int q = wave; q < nc; q += 4) {
+    const size_t oq = o + (size_t)q * ldk;
+    for (int k = lane; k < n; k += 64) x[oq + k] = F[q * st + k];
   }
 }
 
@@ -463,9 +524,29 @@ extern "C" int tgx_launch_thomas_f64(const double *a, const double *b, const dou
                                      const double *f, double *x, double *w2s, int ldk, int k1,
                                      int k2, int col0, int ncol, hipStream_t s) {
   if (ncol <= 0 || k2 < k1) return 0;
-  int nb = (ncol + 255) / 256;
-  hipLaunchKernelGGL(tgx::thomas_kfast_f64, dim3(nb), dim3(256), 0, s, a, b, c, f, x, w2s, ldk,
-                     k1, k2, col0, ncol);
+  // Columns per block of the LDS form: 16 up to 95 rows (48 KB, three blocks per
+  // CU), 8 up to 255 and 4 up to 511 (64 KB); beyond, a thread per column.
+  //   columns x rows   per thread     4      8     16   per block
+  //      7936 x  57          87 us   23     20     18
+  //     10368 x  90         188      47     38     22
+  //     41472 x 113         388     150    118    131
+  //    165888 x 113        2468     508    397    500
+  //      7936 x 255         539     150    121
+  //      4000 x 511        1073     232
+  const int n = k2 - k1 + 1;
+  const size_t per = sizeof(double) * 4 * (size_t)(n | 1);
+  if (n <= 95)
+    hipLaunchKernelGGL(tgx::thomas_lds_f64<16>, dim3((ncol + 15) / 16), dim3(256), 16 * per, s, a, b, c, f, x, ldk, k1,
+                       k2, col0, ncol);
+  else if (n <= 255)
+    hipLaunchKernelGGL(tgx::thomas_lds_f64<8>, dim3((ncol + 7) / 8), dim3(256), 8 * per, s, a, b, c, f, x, ldk, k1, k2,
+                       col0, ncol);
+  else if (n <= TGX_THOMAS_LDS_ROWS)
+    hipLaunchKernelGGL(tgx::thomas_lds_f64<4>, dim3((ncol + 3) / 4), dim3(256), 4 * per, s, a, b, c, f, x, ldk, k1, k2,
+                       col0, ncol);
+  else
+    hipLaunchKernelGGL(tgx::thomas_kfast_f64, dim3((ncol + 255) / 256), dim3(256), 0, s, a, b, c, f, x, w2s, ldk, k1, k2,
+                       col0, ncol);
   TGX_HIP(hipGetLastError());
   return 0;
 }

@@ -10,6 +10,10 @@
 #define TGX_TILE_X 32
 #define TGX_TILE_Y 8
 
+// Rows up to which the scalar Thomas scheme keeps its columns in LDS; beyond, it
+// needs the scratch array of ratios.
+#define TGX_THOMAS_LDS_ROWS 511
+
 // Record a HIP failure in the library's error slot and return the status code.
 int tgx_set_error(int code, const char *fmt, ...);
 // True on the process's main thread.  Per-thread device resources are
