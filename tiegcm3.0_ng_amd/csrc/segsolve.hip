@@ -26,7 +26,10 @@
 // Rows per lane M, lanes per column S: more rows per lane mean fewer reduction
 // steps and less rounding (scalar, relative error 2.4e-16 with M = 8, 2.6e-16
 // with 4, 2.9e-16 reduced row by row), and more registers for y, g and h.
-// Scalar rows take M = 8 and 4 to 32 lanes.  2x2 rows at M = 4 just fit two
+// Scalar rows take M = 4 and 8 or 16 lanes up to 64 rows (28 rows, 2,592, 10,368
+// and 165,888 columns: 5.3, 6.4 and 32 us against 7.6, 8.4 and 40 with M = 8; 56
+// rows, 2,592 and 41,472: 4.5 and 17 us against 6.1 and 19), beyond that M = 8,
+// where DPP no longer reaches across a column of M = 4.  2x2 rows at M = 4 just fit two
 // wavefronts per SIMD (113 levels: 168 us, 190 with M = 2); up to 32 rows
 // M = 2 fits three (43 us against 48, 41,472 x 28).  3x3 rows at M = 4 use
 // every register of a SIMD (56 rows: 78 us, 118 with M = 2), up to 32 rows
@@ -416,8 +419,8 @@ extern "C" int tgx_launch_segment(int nblk, const double *a, const double *b, co
   if (ncol <= 0 || n <= 0) return 0;
   if (n > 256) return tgx_set_error(1, "the partitioned solver holds at most 256 rows per column (got %d)", n);
   if (nblk == 1) {
-    if (n <= 32) return launch<1, 4, 8>(a, b, c, f, x, ldk, n, ncol, s);
-    if (n <= 64) return launch<1, 8, 8>(a, b, c, f, x, ldk, n, ncol, s);
+    if (n <= 32) return launch<1, 8, 4>(a, b, c, f, x, ldk, n, ncol, s);
+    if (n <= 64) return launch<1, 16, 4>(a, b, c, f, x, ldk, n, ncol, s);
     if (n <= 128) return launch<1, 16, 8>(a, b, c, f, x, ldk, n, ncol, s);
     return launch<1, 32, 8>(a, b, c, f, x, ldk, n, ncol, s);
   }
