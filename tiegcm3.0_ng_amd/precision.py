@@ -97,7 +97,7 @@ def solve_mixed(field, A, B, Cc, F, valid_dev, nk, nsweep, stream=None):
     L = _lib()
     wb = L.tgx_blk_mixed_work_bytes(n, nrow, ncol)
     work = torch.empty((wb + 7) // 8, dtype=torch.float64, device=B.device)
-    s = torch.cuda.current_stream().cuda_stream if stream is None else stream
+    s = _tgx.current_stream() if stream is None else stream
     rc = L.tgx_blk_mixed_dev(n, A.data_ptr(), B.data_ptr(), Cc.data_ptr(), F.data_ptr(), X.data_ptr(),
                              ncol * nk, nk, nrow, valid_dev.data_ptr(), ncol, nsweep, work.data_ptr(), s)
     if rc != 0:

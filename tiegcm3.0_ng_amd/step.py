@@ -261,7 +261,7 @@ class NestState:
     _STEPS = ("tgx_ng_step", "tgx_ng_step_serial", "tgx_ng_step_mixed")
 
     def _call(self, name, stream=None, extra=()):
-        s = torch.cuda.current_stream().cuda_stream if stream is None else stream
+        s = _tgx.current_stream() if stream is None else stream
         f, o = (self.f, self.o)
         phases = getattr(self, "_phases", None)
         if phases and name in self._STEPS:
@@ -291,7 +291,7 @@ class NestState:
     def comp_mixed(self, nsweep, stream=None):
         """comp's precision form: FP32 assembly and elimination with FP64 block
         pivots and nsweep (0..2) FP64-residual refinement sweeps."""
-        s = torch.cuda.current_stream().cuda_stream if stream is None else stream
+        s = _tgx.current_stream() if stream is None else stream
         rc = _lib().tgx_ng_comp_mixed(C.byref(self.g), C.byref(self.f), C.byref(self.o),
                                       C.c_void_p(self.work.data_ptr()), C.c_void_p(s), C.c_int(int(nsweep)))
         if rc != 0:
@@ -587,7 +587,7 @@ class GlobalState(NestState):
             self.work = torch.empty((nbytes + 7) // 8, dtype=torch.float64, device=self.work.device)
 
     def _call(self, name, stream=None):
-        s = torch.cuda.current_stream().cuda_stream if stream is None else stream
+        s = _tgx.current_stream() if stream is None else stream
         f, o = (self.f, self.o)
         phases = getattr(self, "_phases", None)
         stepping = name in ("tgx_ng_step", "tgx_ng_step_serial")
@@ -614,7 +614,7 @@ class GlobalState(NestState):
         """tgx_glb_halos on the current value of each field: its periodic
         points and the rows across the poles (as the model does before a
         step, mk_polelat.F), sign-flipped for synth.POLE_ODD."""
-        s = torch.cuda.current_stream().cuda_stream if stream is None else stream
+        s = _tgx.current_stream() if stream is None else stream
         for n in names:
             t = self.current(n)
             nk = t.shape[0] if t.dim() == 3 else 1

@@ -100,10 +100,17 @@ def _dp(t):
     return C.c_void_p(t.data_ptr())
 
 
+def current_stream():
+    """The current stream of the current device as a number.  (The stream object
+    of torch.cuda.current_stream() takes 2.8 us to make, a third of a small
+    solve's call; this takes 0.4.)"""
+    import torch
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+
+
 def _stream(stream):
     if stream is None:
-        import torch
-        return C.c_void_p(torch.cuda.current_stream().cuda_stream)
+        return C.c_void_p(current_stream())
     return C.c_void_p(stream)
 
 
