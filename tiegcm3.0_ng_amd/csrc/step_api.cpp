@@ -672,9 +672,17 @@ int get_fork(Fork **out) {
 
 typedef int (*RoutineFn)(const tgx_ng_grid *, const tgx_ng_fields *, const tgx_ng_out *, void *, void *);
 
+// In the step a routine runs beside the others, where the block kernels (16
+// threads per column) leave more room than a wavefront per column does, so
+// Thomas is kept unless the other scheme is this much faster alone.  104x54x57
+// columns, alone, block and wavefront: minor species 129 and 111 us, dt 40 and
+// 38; the nested outer step 4.03 ms with the block forms, 4.21 with what is
+// faster alone.  (60x40: minor species 88 and 66, left to the wavefront.)
+constexpr float BLOCK_FAVOUR = 0.83f;
+
 // Times every routine under both schemes on `stream` (reference order, so
 // duv sees this step's dt and oplus outputs) and keeps the faster scheme per
-// routine for this device and shape.  The outputs are left as a full step
+// routine for this device and shape, the block kernels favoured.  The outputs are left as a full step
 // computed with the last scheme timed; the caller runs its step afterwards.
 extern "C" int tgx_ng_autotune(const tgx_ng_grid *g, const tgx_ng_fields *in, const tgx_ng_out *out,
                                void *work, void *stream) {
@@ -716,7 +724,7 @@ extern "C" int tgx_ng_autotune(const tgx_ng_grid *g, const tgx_ng_fields *in, co
     if (rc == 0) {
       int q = 0;
       for (int c = 1; c < nsch; ++c)
-        if (best[c] < best[q]) q = c;
+        if (best[c] < (q == 0 && block_grid(g, r) ? BLOCK_FAVOUR : 1.f) * best[q]) q = c;
       std::lock_guard<std::mutex> lk(g_tune_mu);
       g_tune[tune_key(g, r)] = schemes[q];
       if (q > 0) g_tune_cols[tune_key(g, r)] = cols[q];
