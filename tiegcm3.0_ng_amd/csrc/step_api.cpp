@@ -754,14 +754,15 @@ extern "C" int tgx_ng_scheme_choice(const tgx_ng_grid *g, int routine) {
   return c == TGX_SCHEME_AUTO ? TGX_SCHEME_PCR : c;
 }
 
-// Small grids outside a graph run O+, dt and duv on the caller's stream and the
-// minor species and comp on one other.  There the step is bound by the host:
-// a launch costs it 3 us, but a wait for another stream's event 8-10 us, and
-// two streams take three waits where four take eight.  72x36x29: 235 us per step
-// with two streams, 290 with four, 270 on one; 100x50x57 nest with five O+
-// sub-cycles: 488 and 510 us; but 144x72x57 with ten: 1185 and 1140 us, and in a
-// graph, where waits cost the host nothing, four are faster at any size.
-static bool two_streams(const tgx_ng_grid *g, hipStream_t s) {
+// Small grids outside a graph run comp on the minor species' stream and, with
+// one O+ sub-cycle, O+ on the caller's.  There the step is bound by the host: a
+// launch costs it 3 us, but a wait for another stream's event 8-10 us, and two
+// streams take three waits where four take eight.  72x36x29: 235 us per step
+// with two streams, 290 with four, 270 on one.  100x50x57 nest with five
+// sub-cycles, whose O+ chain is the longest: 461 us with three streams, 478 with
+// two, 510 with four; 144x72x57 with ten: 1185 us with two and 1140 with four, and
+// in a graph, where waits cost the host nothing, four are faster at any size.
+static bool few_streams(const tgx_ng_grid *g, hipStream_t s) {
   if ((long)(g->nlon + 4) * (g->nlat + 4) * g->nk > 450000) return false;
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
   return hipStreamIsCapturing(s, &st) == hipSuccess && st == hipStreamCaptureStatusNone;
@@ -776,11 +777,12 @@ extern "C" int tgx_ng_step(const tgx_ng_grid *g, const tgx_ng_fields *in, const 
     if (int rc = tgx_ng_autotune(g, in, out, work, stream)) return rc;
   Fork *F = nullptr;
   if (int rc = get_fork(&F)) return rc;
-  const bool two = two_streams(g, (hipStream_t)stream);
+  const bool few = few_streams(g, (hipStream_t)stream), two = few && g->nstep_sub == 1;
   hipStream_t s0 = (hipStream_t)stream, sb = F->s[1];
-  hipStream_t sa = two ? s0 : F->s[0], sc = two ? sb : F->s[2];
-  // Fork: every stream starts after what the caller queued before the step,
-  // stream b at once (ev[5]) and a and c after the chemistry pass (ev[0]).
+  hipStream_t sa = two ? s0 : F->s[0], sc = few ? sb : F->s[2];
+  // Fork: every stream starts after what the caller queued before the step:
+  // stream b at once (ev[5]), as stream c where it takes dt, and the others
+  // after the chemistry pass (ev[0]).
   // From here on every return joins the forked streams back into s0, so that a
   // failed call still leaves a graph capture joined and no forked kernel
   // running past the caller's stream.
@@ -800,38 +802,49 @@ extern "C" int tgx_ng_step(const tgx_ng_grid *g, const tgx_ng_fields *in, const 
   } join{F, s0};
   TGX_HIP(hipEventRecord(F->ev[5], s0));
   TGX_HIP(join.fork(1, 5));
-  // The minor species' stencil prelude on stream b, beside the pointwise
-  // chemistry of all routines in one pass on s0 (ev[0]: done), which it does
-  // not read; the rest of every routine starts after the pass.
+  // The minor species' stencil prelude on stream b and a nest's dt on stream c,
+  // beside the pointwise chemistry of all routines in one pass on s0 (ev[0]:
+  // done), which neither reads (a global dt ends with the ring filter, whose
+  // table the pass fills); the rest of every routine starts after the pass.
   //
   // The order of the calls below fixes no dependency, but a HIP graph of the
   // step puts its branches on four queues by walking the edges in the order
-  // they were recorded.  With O+ and dt recorded before the minor species and
-  // comp, and without edges from the step before to streams a and c (they
-  // follow the chemistry pass), the minor species' prelude gets a queue that is
-  // idle during the chemistry pass; recorded in the reference's order it was
-  // queued behind comp, the minor species ran alone at the end of each step, and
-  // a nested outer step (one 144x72x57, two 120x60x57 and ten 100x50x57 steps) took
-  // 4.99 ms instead of 4.38.  Of 20 orders this one and its neighbours were the
-  // fastest; steps outside a graph do not depend on it.
+  // they were recorded.  Recorded in the reference's order, and with edges from
+  // the step before to the streams that follow the chemistry pass, the minor
+  // species' prelude was queued behind comp, the minor species ran alone at the
+  // end of each step, and a nested outer step (one 144x72x57, two 120x60x57 and ten
+  // 100x50x57 steps) took 4.99 ms; prelude, O+, dt, minor species, comp: 4.38 (4.00
+  // with the block kernels favoured); with a nest's dt first on its own stream
+  // and comp before the minor species, 3.91.  Some 40 orders were tried; steps
+  // outside a graph hardly depend on it.
+  const bool early = !few && !t_glb;
   if (int rc = run_minors(g, in, out, work, sb, true, PART_PRELUDE)) return rc;
+  if (early) {
+    TGX_HIP(join.fork(2, 5));
+    if (int rc = tgx_ng_dt(g, in, out, work, sc)) return rc;
+  }
   if (int rc = run_chem(g, in, out, work, s0)) return rc;
   TGX_HIP(hipEventRecord(F->ev[0], s0));
-  if (!two) {
-    TGX_HIP(join.fork(0, 0));
-    TGX_HIP(join.fork(2, 0));
+  if (!two) TGX_HIP(join.fork(0, 0));
+  // stream a; ev[4]: its Fe/Fn are written (the last sub-step's stage 1)
+  if (int rc = run_oplus(g, in, out, work, sa, true, g->nstep_sub, two ? nullptr : F->ev[4])) return rc;
+  hipStream_t sd = early ? sc : s0;  // dt and duv
+  if (early) {
+    if (int rc = run_comp(g, in, out, work, s0, true)) return rc;
+  } else {
+    if (int rc = tgx_ng_dt(g, in, out, work, s0)) return rc;
   }
-  // ev[4]: its Fe/Fn are written (the last sub-step's stage 1)
-  if (int rc = run_oplus(g, in, out, work, sa, true, g->nstep_sub, two ? nullptr : F->ev[4])) return rc;  // stream a
-  if (int rc = tgx_ng_dt(g, in, out, work, s0)) return rc;       // caller's stream
   TGX_HIP(hipStreamWaitEvent(sb, F->ev[0], 0));
-  if (int rc = run_minors(g, in, out, work, sb, true, PART_COLUMNS)) return rc;  // stream b
-  if (int rc = run_comp(g, in, out, work, sc, true)) return rc;     // stream c
+  if (int rc = run_minors(g, in, out, work, sb, true, PART_COLUMNS)) return rc;
+  if (!early) {
+    if (!few) TGX_HIP(join.fork(2, 0));
+    if (int rc = run_comp(g, in, out, work, sc, true)) return rc;
+  }
   // duv reads Fe/Fn of oplus and no other output or workspace region of it,
   // so it starts while the rest of the O+ sub-step (its column solve, ring
   // filter, post pass) still runs
-  if (!two) TGX_HIP(hipStreamWaitEvent(s0, F->ev[4], 0));
-  return tgx_ng_duv(g, in, out, work, s0);  // the fork streams joined on return
+  if (!two) TGX_HIP(hipStreamWaitEvent(sd, F->ev[4], 0));
+  return tgx_ng_duv(g, in, out, work, sd);  // the fork streams joined on return
 }
 
 // The same step strictly in the reference's order on one stream.
