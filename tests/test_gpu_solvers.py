@@ -361,3 +361,63 @@ def test_thomas_scheme_bit_for_bit(pkg, n):
         pkg.tgx.trsolv_dev(*d, k1, k2, scheme=pkg.tgx.SCHEME_THOMAS, col0=col0, ncol=ncol)
         torch.cuda.synchronize()
         assert np.array_equal(d[4].cpu().numpy(), ref), (n, ncol)
+
+
+def _growing_segments(nblk, n, period, g, ncol, seed):
+    """Columns whose rows taken `period` at a time grow by about g per row of a
+    segment, although the whole column is well conditioned (and Thomas, which
+    never meets the small pivots unreduced, solves it to rounding): segment
+    starts 1/g between unit couplings, rows inside 1 + 1/g after a coupling 1/g,
+    the last row 2.5.  Rows, and the condition number of the scalar column."""
+    k = np.arange(n)
+    e = k % period
+    b = np.where(k == 0, 2., np.where(e == 0, 1. / g, np.where(e == period - 1, 2.5, 1. + 1. / g)))
+    a = np.where((e == 0) | (e == period - 1), 1., 1. / g)
+    eye = np.eye(nblk)
+    A, B = (np.tile(v[:, None, None] * eye, (ncol, 1, 1, 1)) for v in (a, b))
+    C = np.tile(eye, (ncol, n, 1, 1))
+    F = np.random.default_rng(seed).normal(size=(ncol, n, nblk))
+    A[:, 0] = 0.
+    C[:, n - 1] = 0.
+    return A, B, C, F, np.linalg.cond(np.diag(b) + np.diag(a[1:], -1) + np.diag(np.ones(n - 1), 1))
+
+
+def _device_segments(pkg, nblk, A, B, C, F):
+    import torch
+    from test_oracle_solvers import to_colmajor
+    sys_ = [torch_dev(to_colmajor(v) if nblk > 1 else v[..., 0, 0]) for v in (A, B, C)]
+    sys_.append(torch_dev(F if nblk > 1 else F[..., 0]))
+    x = torch.zeros_like(sys_[3])
+    _segment_solve(pkg, nblk, sys_, x, F.shape[1])
+    return x.cpu().numpy().reshape(F.shape)
+
+
+def _refined(A, B, C, F):
+    """The solutions of block tridiagonal columns, refined to beyond 64 bits."""
+    ncol, n, m = F.shape
+    M = np.zeros((ncol, n, m, n, m))
+    for k in range(n):
+        M[:, k, :, k] = B[:, k]
+        if k:
+            M[:, k, :, k - 1] = A[:, k]
+        if k < n - 1:
+            M[:, k, :, k + 1] = C[:, k]
+    M = M.reshape(ncol, n * m, n * m)
+    f = F.reshape(ncol, n * m, 1)
+    x = np.linalg.solve(M, f).astype(np.longdouble)
+    for _ in range(3):
+        r = f - np.stack([(Mi.astype(np.longdouble) @ xi) for Mi, xi in zip(M, x)])
+        x = x + np.linalg.solve(M, r.astype(np.float64))
+    return x.reshape(F.shape)
+
+
+@pytest.mark.parametrize("nblk", [2, 3])
+@pytest.mark.parametrize("n", [56, 112, 200])
+def test_block_rows_with_a_large_correction(pkg, nblk, n):
+    """A block column whose correction from the residual shows that its
+    segments lost digits is not stored: an accepted correction is at most 1e-12
+    of the unknowns and all that an error contracts by is the unit couplings
+    over 2.5 (a factor of 5 at most), so 5e-12."""
+    A, B, C, F, cond = _growing_segments(nblk, n, 4, 31., 40, n + nblk)
+    assert cond < 400.
+    assert relerr(_device_segments(pkg, nblk, A, B, C, F), _refined(A, B, C, F).astype(np.float64)) <= 5e-12

@@ -266,6 +266,11 @@ __device__ __noinline__ void serial_column(const double *A, const double *B, con
 // pivots on unreduced): it is solved again in the reference's order.  Rows
 // with diagonal dominance keep them at 1 or below.
 constexpr double GROWTH = 32.;
+// The largest correction of a block row, relative to the largest unknown of the
+// row and its neighbours, that is rounding: 1e-15 on dominant rows, 7e-14 where
+// the dominance is 1e-5 to 1e-3 (56 to 200 rows), 1e-12 for a solution that falls
+// by a decade per row; 1e-11 where a segment lost five digits.
+constexpr double CORRECTION = 1e-12;
 
 template <int N, int S, int M>
 __global__ void __launch_bounds__(64, 1)
@@ -350,21 +355,28 @@ segment_kernel(const double *__restrict__ a, const double *__restrict__ b, const
   xs[M - 1] = X;
 #pragma unroll
   for (int e = M - 2; e >= 0; --e) xs[e] = sub(sub(y[e], h[e], xl), g[e], xs[e + 1]);
+  bool bad = !(gr <= GROWTH);
   if (N > 1) {
     // One correction of each row from its neighbours, x(k) += B^-1 (F - A
     // x(k-1) - B x(k) - C x(k+1)): takes the rounding of the two extra
     // substitutions of a partitioned solve back out (relative error 1.0e-16
     // on dominant 2x2 rows and 1.1e-16 on 3x3, 2.0e-16 and 2.4e-16 without;
-    // Thomas 1.5e-16 and 1.8e-16).
+    // Thomas 1.5e-16 and 1.8e-16).  It is also the proof of the solution: a
+    // column with a correction beyond CORRECTION is solved again.
     const Vec<N> xn = above<S, 1>(xs[0], lane);
     Vec<N> prev = xl;
 #pragma unroll
     for (int e = 0; e < M; ++e) {
       const Vec<N> next = e < M - 1 ? xs[e < M - 1 ? e + 1 : 0] : xn, here = xs[e];
       const Vec<N> r = mul(inverse(B[e]), sub(sub(sub(F[e], A[e], prev), B[e], here), Cm[e], next));
+      double big = 0.;
 #pragma unroll
-      for (int q = 0; q < N; ++q)
-        if (fabs(r.v[q]) <= 1e-9 * fabs(here.v[q])) xs[e].v[q] = here.v[q] + r.v[q];
+      for (int q = 0; q < N; ++q) big = fmax(fmax(big, fabs(here.v[q])), fmax(fabs(prev.v[q]), fabs(next.v[q])));
+#pragma unroll
+      for (int q = 0; q < N; ++q) {
+        bad |= !(fabs(r.v[q]) <= CORRECTION * big);
+        xs[e].v[q] = here.v[q] + r.v[q];
+      }
       prev = here;
     }
   }
@@ -374,7 +386,7 @@ segment_kernel(const double *__restrict__ a, const double *__restrict__ b, const
     for (int q = 0; q < N; ++q) sv[t * LV + e * N + q] = xs[e].v[q];
   __syncthreads();
   // a column some lane of which is badly pivoted goes by another way
-  const unsigned long long vote = __ballot(col && !(gr <= GROWTH));
+  const unsigned long long vote = __ballot(col && bad);
   const int len = n * N;
 #pragma unroll
   for (int cc = 0; cc < C; ++cc) {
