@@ -421,3 +421,47 @@ def test_block_rows_with_a_large_correction(pkg, nblk, n):
     A, B, C, F, cond = _growing_segments(nblk, n, 4, 31., 40, n + nblk)
     assert cond < 400.
     assert relerr(_device_segments(pkg, nblk, A, B, C, F), _refined(A, B, C, F).astype(np.float64)) <= 5e-12
+
+
+@pytest.mark.parametrize("nblk", [1, 2, 3])
+@pytest.mark.parametrize("n", [28, 56, 112, 200])
+def test_partitioned_solver_growing_segments(pkg, oracle, nblk, n):
+    """Columns whose multipliers compound over a segment, for segments of 2, 4
+    and 8 rows, one small pivot per segment on its own, multipliers on both
+    sides of every limit the kernel could put to a single one.  Accepted columns
+    have multipliers and products of them of at most 4 and the others are solved
+    in the reference's order, so the worst error stays within twice that (a
+    substitution and a reduction use them) of the reference order's."""
+    from test_oracle_solvers import to_colmajor
+    parts, what = [], []
+    for g in (2.2, 5., 10., 20., 31., 33.):
+        for period in (2, 4, 8):
+            *p, cond = _growing_segments(nblk, n, period, g, 4, int(100 * g) + period)
+            if cond < 400.:
+                parts.append(p)
+                what += [(g, period)] * 4
+            k = np.arange(n)
+            A, _, C, F = (v.copy() for v in p)
+            A[:, 1:] = C[:, :n - 1] = np.eye(nblk)
+            B = np.tile(np.where((k % period == 0) & (k > 0), 1. / g, 4.)[:, None, None] * np.eye(nblk), (4, 1, 1, 1))
+            if period > 2:
+                parts.append([A, B, C, F])
+                what += [(g, -period)] * 4
+    A, B, C, F = (np.concatenate(v) for v in zip(*parts))
+    ncol = len(what)
+    y = np.zeros_like(F)
+    if nblk == 1:
+        oracle.trsolv_ng(*(np.ascontiguousarray(v[..., 0, 0]) for v in (A, B, C)), np.ascontiguousarray(F[..., 0]),
+                         y[..., 0], n, ncol, n)
+    elif nblk == 2:
+        ext = [np.concatenate([v, v[:, :1]], axis=1) for v in (A, B, C, F)]
+        z = np.zeros((ncol, n + 1, 2))
+        oracle.blktri(*[to_colmajor(v) for v in ext[:3]], np.ascontiguousarray(ext[3]), z, 1, n + 1, 5, 5 + ncol - 1, 100000)
+        y = z[:, :n]
+    else:
+        oracle.blktri3(to_colmajor(A), to_colmajor(B), to_colmajor(C), F, y, n, ncol, n)
+    exact = _refined(A, B, C, F)
+    scale = np.abs(exact).max(axis=(1, 2))
+    err = [(np.abs(v - exact).max(axis=(1, 2)) / scale).astype(np.float64) for v in (_device_segments(pkg, nblk, A, B, C, F), y)]
+    worst = int(np.argmax(err[0]))
+    assert err[0].max() <= 8. * err[1].max(), (what[worst], err[0].max(), err[1].max())
