@@ -465,3 +465,24 @@ def test_partitioned_solver_growing_segments(pkg, oracle, nblk, n):
     err = [(np.abs(v - exact).max(axis=(1, 2)) / scale).astype(np.float64) for v in (_device_segments(pkg, nblk, A, B, C, F), y)]
     worst = int(np.argmax(err[0]))
     assert err[0].max() <= 8. * err[1].max(), (what[worst], err[0].max(), err[1].max())
+
+
+@pytest.mark.parametrize("nblk", [1, 2, 3])
+@pytest.mark.parametrize("n", [28, 56, 112, 200])
+def test_partitioned_solver_in_place(pkg, nblk, n):
+    """The solution written over the right-hand side: columns that are refined
+    read theirs again after their neighbours in the wavefront have been stored."""
+    import torch
+    from test_oracle_solvers import to_colmajor
+    parts = [_growing_segments(nblk, n, period, g, 3, n + period)[:4] for g in (1., 31.) for period in (4, 8)]
+    A, B, C, F = (np.concatenate(v) for v in zip(*parts))
+    B[1::4, ::8] = 0.  # and in the reference's order
+    B[:, 0] = 2. * np.eye(nblk)
+    perm = np.random.default_rng(n).permutation(len(F))
+    A, B, C, F = (v[perm] for v in (A, B, C, F))
+    sys_ = [torch_dev(to_colmajor(v) if nblk > 1 else v[..., 0, 0]) for v in (A, B, C)]
+    sys_.append(torch_dev(F if nblk > 1 else F[..., 0]))
+    x = torch.zeros_like(sys_[3])
+    _segment_solve(pkg, nblk, sys_, x, n)
+    _segment_solve(pkg, nblk, sys_, sys_[3], n)
+    assert torch.equal(x, sys_[3]) and bool(torch.isfinite(x).all())

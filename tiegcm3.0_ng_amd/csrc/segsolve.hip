@@ -176,7 +176,7 @@ __device__ __forceinline__ T above(const T &a, int lane) {
 
 // Multipliers beyond this mark a column whose segments are badly pivoted on
 // their own (a diagonal block small beside its couplings, which Thomas never
-// pivots on unreduced): it is solved again in the reference's order.  Held
+// pivots on unreduced): it is refined (refine_columns).  Held
 // against it are a row's multipliers and their products over the lane's rows, by
 // which an error of one row reaches another: multipliers of 2 to 31 in a
 // segment of eight scalar rows, all below a limit of 32 for each, lost 2 to 11
@@ -281,20 +281,30 @@ __device__ __noinline__ void serial_column(const double *A, const double *B, con
 // the dominance is 1e-5 to 1e-3 (56 to 200 rows), 1e-12 for a solution that falls
 // by a decade per row; 1e-11 where a segment lost five digits.
 constexpr double CORRECTION = 1e-12;
+// A badly pivoted column is refined: the same elimination solves for the
+// residual, which is computed in 64 bits from the rows themselves, until a
+// correction is within REFINED of the unknowns, so that what it leaves
+// (its own relative error squared) is below rounding.  At most REFINEMENTS
+// times, then in the reference's order by one lane, as where a pivot
+// vanished and nothing finite came out.  Emulated on the families above, one
+// pass suffices but for multipliers of 20 and more over eight rows (two) and 1
+// in 100 random 3x3 columns (three); the error is 0.2 to 0.9 times that of the
+// reference's order.  One lane per column for all of them instead: scalar
+// 165,888 x 112, every column bad, 1,280 us; 2x2 41,472 x 112 1,660; 3x3 10,368 x
+// 56 520; refined 361, 259 and 137 (a wavefront per column reduced row by row, or a
+// thread per column, took 355, 577 and 337).
+constexpr double REFINED = 1e-8;
+constexpr int REFINEMENTS = 3;
 
+// The rows of a block's nc columns, column c0 the first: 64 consecutive doubles
+// per load, every load in flight at once, then through LDS (sm) to the lanes
+// that own the rows, one array after the other.  Identity rows past the column.
 template <int N, int S, int M>
-__global__ void __launch_bounds__(64, 1)
-segment_kernel(const double *__restrict__ a, const double *__restrict__ b, const double *__restrict__ c,
-               const double *f, double *x, int ldk, int n, int ncol) {
+__device__ __forceinline__ void load_rows(int t, const double *a, const double *b, const double *c, const double *f,
+                                          long c0, int nc, int ldk, int n, double *sm, Mat<N> (&A)[M], Mat<N> (&B)[M],
+                                          Mat<N> (&Cm)[M], Vec<N> (&F)[M]) {
   constexpr int C = 64 / S, NN = N * N;
-  constexpr int LM = M * NN + 1, LV = M * N + 1;  // LDS doubles of a lane's rows, one of padding
   constexpr int QM = (S * M * NN + 63) / 64, QV = (S * M * N + 63) / 64;  // loads of one column
-  __shared__ double sm[64 * LM], sv[64 * LV];
-  const int t = threadIdx.x, lane = t % S, cw = t / S;
-  const long c0 = (long)tgx_xcd_block(gridDim.x) * C;
-  const int nc = (int)min((long)C, ncol - c0);  // at least 1
-
-  // the columns, 64 consecutive doubles per load, every load in flight at once
   double va[C * QM], vb[C * QM], vc[C * QM], vf[C * QV];
 #define SEG_LOAD(buf, src, per, Q)                                                                          \
   _Pragma("unroll") for (int cc = 0; cc < C; ++cc) _Pragma("unroll") for (int q = 0; q < Q; ++q)          \
@@ -304,29 +314,32 @@ segment_kernel(const double *__restrict__ a, const double *__restrict__ b, const
   SEG_LOAD(vc, c, NN, QM)
   SEG_LOAD(vf, f, N, QV)
 #undef SEG_LOAD
-  // through LDS to the lanes that own the rows, one array after the other
-  Mat<N> A[M], B[M], Cm[M];
-  Vec<N> F[M];
-  const bool col = cw < nc;
-  const int r0 = lane * M;
-#define SEG_ROWS(dst, buf, sh, per, Q, on, other)                                                           \
+  const bool col = t / S < nc;
+  const int r0 = t % S * M;
+#define SEG_ROWS(dst, buf, per, Q, on, other)                                                               \
   _Pragma("unroll") for (int cc = 0; cc < C; ++cc) _Pragma("unroll") for (int q = 0; q < Q; ++q)          \
-      if (64 * q + t < S * M * (per)) sh[cc * S * (M * (per) + 1) + (64 * q + t) + (64 * q + t) / (M * (per))] = buf[cc * Q + q]; \
+      if (64 * q + t < S * M * (per)) sm[cc * S * (M * (per) + 1) + (64 * q + t) + (64 * q + t) / (M * (per))] = buf[cc * Q + q]; \
   __syncthreads();                                                                                        \
   _Pragma("unroll") for (int e = 0; e < M; ++e) _Pragma("unroll") for (int q = 0; q < (per); ++q) {       \
-    const double w = sh[t * (M * (per) + 1) + e * (per) + q];                                             \
+    const double w = sm[t * (M * (per) + 1) + e * (per) + q];                                             \
     dst[e].v[q] = col && (on) ? w : (other);                                                              \
   }                                                                                                       \
   __syncthreads();
-  SEG_ROWS(A, va, sm, NN, QM, r0 + e > 0 && r0 + e < n, 0.)
-  SEG_ROWS(B, vb, sm, NN, QM, r0 + e < n, q % (N + 1) == 0 ? 1. : 0.)  // identity rows past the column
-  SEG_ROWS(Cm, vc, sm, NN, QM, r0 + e < n - 1, 0.)
-  SEG_ROWS(F, vf, sv, N, QV, r0 + e < n, 0.)
+  SEG_ROWS(A, va, NN, QM, r0 + e > 0 && r0 + e < n, 0.)
+  SEG_ROWS(B, vb, NN, QM, r0 + e < n, q % (N + 1) == 0 ? 1. : 0.)
+  SEG_ROWS(Cm, vc, NN, QM, r0 + e < n - 1, 0.)
+  SEG_ROWS(F, vf, N, QV, r0 + e < n, 0.)
 #undef SEG_ROWS
+}
 
+// The partitioned elimination: xs the lane's unknowns, xl the previous lane's
+// last one; bad: a multiplier or a product of them is beyond GROWTH.
+template <int N, int S, int M>
+__device__ __forceinline__ void eliminate(const Mat<N> (&A)[M], const Mat<N> (&B)[M], const Mat<N> (&Cm)[M],
+                                          const Vec<N> (&F)[M], int lane, Vec<N> (&xs)[M], Vec<N> &xl, bool &bad) {
   Mat<N> g[M - 1], h[M - 1];
   Vec<N> y[M - 1];
-  bool bad = false;
+  bad = false;
 #pragma unroll
   for (int e = 0; e < M - 1; ++e) {
     if (e == 0) {
@@ -361,11 +374,120 @@ segment_kernel(const double *__restrict__ a, const double *__restrict__ b, const
     bad |= beyond(ra, GROWTH) | beyond(rc, GROWTH);
     reduce<N, S, 1>(ra, rc, X, lane, bad);
   }
-  Vec<N> xs[M];
-  const Vec<N> xl = below<S, 1>(X, lane);
+  xl = below<S, 1>(X, lane);
   xs[M - 1] = X;
 #pragma unroll
   for (int e = M - 2; e >= 0; --e) xs[e] = sub(sub(y[e], h[e], xl), g[e], xs[e + 1]);
+}
+
+// The largest unknown of a row and its neighbours.
+template <int N>
+__device__ __forceinline__ double largest(const Vec<N> &p, const Vec<N> &q, const Vec<N> &r) {
+  double big = 0.;
+#pragma unroll
+  for (int n = 0; n < N; ++n) big = fmax(fmax(big, fabs(p.v[n])), fmax(fabs(q.v[n]), fabs(r.v[n])));
+  return big;
+}
+
+// Stores the columns whose lanes are in `done` from the lanes' rows in sv.
+template <int N, int S, int M>
+__device__ __forceinline__ void store_columns(unsigned long long done, double *x, long c0, int ldk, int n,
+                                              const double *sv) {
+  constexpr int C = 64 / S, LV = M * N + 1, QV = (S * M * N + 63) / 64;
+#pragma unroll
+  for (int cc = 0; cc < C; ++cc)
+    if (done >> (cc * S) & 1)
+#pragma unroll
+      for (int q = 0; q < QV; ++q) {
+        const int e = 64 * q + (int)threadIdx.x;
+        if (e < n * N) x[(size_t)(c0 + cc) * ldk * N + e] = sv[cc * S * LV + e + e / (M * N)];
+      }
+}
+
+// The columns whose lanes are in todo, badly pivoted, their first solution in sv.
+template <int N, int S, int M>
+__device__ __forceinline__ void refine_columns(const double *a, const double *b, const double *c, const double *f,
+                                            double *x, int ldk, int n, long c0, int nc, double *sm, double *sv,
+                                            unsigned long long todo) {
+  constexpr int NN = N * N, LM = M * NN + 1, LV = M * N + 1;
+  unsigned long long serial = 0;
+  int t = threadIdx.x;
+  // the solution so far, rows -1 and M from the neighbouring lanes
+  auto solved = [&](int e) {
+    const int lane = t % S;
+    Vec<N> r;
+    const bool in = (e >= 0 || lane > 0) && (e < M || lane + 1 < S);
+    const int o = !in ? 0 : e < 0 ? (t - 1) * LV + (M - 1) * N : e < M ? t * LV + e * N : (t + 1) * LV;
+#pragma unroll
+    for (int q = 0; q < N; ++q) r.v[q] = in ? sv[o + q] : 0.;
+    return r;
+  };
+#pragma unroll 1
+  for (int pass = 0; pass < REFINEMENTS && todo; ++pass) {
+    asm volatile("" : "+v"(t));  // addresses formed anew in every pass: the registers are the rows'
+    const int lane = t % S;
+    const unsigned long long own = (S == 64 ? ~0ull : (1ull << (S & 63)) - 1) << (t / S * S & 63);  // this column's lanes
+    Mat<N> A[M], B[M], Cm[M];
+    Vec<N> F[M], d[M], dl;
+    load_rows<N, S, M>(t, a, b, c, f, c0, nc, ldk, n, sm, A, B, Cm, F);
+#pragma unroll
+    for (int e = 0; e < M; ++e) {
+      F[e] = sub(sub(sub(F[e], A[e], solved(e - 1)), B[e], solved(e)), Cm[e], solved(e + 1));
+      asm volatile("" ::: "memory");  // read again below: the registers are the elimination's
+    }
+    bool bad;
+    eliminate<N, S, M>(A, B, Cm, F, lane, d, dl, bad);
+    bad = false;
+    bool lost = false;  // nothing to refine
+#pragma unroll
+    for (int e = 0; e < M; ++e) {
+      asm volatile("" ::: "memory");
+      const Vec<N> here = solved(e);
+      const double big = largest(solved(e - 1), here, solved(e + 1));
+#pragma unroll
+      for (int q = 0; q < N; ++q) {
+        bad |= !(fabs(d[e].v[q]) <= REFINED * big);
+        d[e].v[q] = here.v[q] + d[e].v[q];
+        lost |= !(fabs(d[e].v[q]) <= 1.e300);
+      }
+    }
+    __syncthreads();  // the neighbours have read this lane's solution
+#pragma unroll
+    for (int e = 0; e < M; ++e)
+#pragma unroll
+      for (int q = 0; q < N; ++q) sv[t * LV + e * N + q] = d[e].v[q];
+    __syncthreads();
+    const unsigned long long bads = __ballot(bad), losts = __ballot(lost);
+    serial |= __ballot((losts & own) != 0) & todo;
+    const unsigned long long again = __ballot((bads & own) != 0) & todo & ~serial;
+    store_columns<N, S, M>(todo & ~serial & ~again, x, c0, ldk, n, sv);
+    todo = again;
+  }
+  serial |= todo;
+  if (!serial) return;
+  __syncthreads();
+  const int cw = t / S;
+  if (t % S == 0 && (serial >> t & 1)) {
+    const size_t o = (size_t)(c0 + cw) * ldk;
+    serial_column<N>(a + o * NN, b + o * NN, c + o * NN, f + o * N, sm + cw * S * LM, sv + cw * S * LV, n);
+    for (int e = 0; e < n * N; ++e) x[o * N + e] = sv[cw * S * LV + e];
+  }
+}
+
+template <int N, int S, int M>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(N == 1 ? (M == 4 ? 6 : S == 16 ? 5 : 4) : N == 3 ? 1 : M == 2 ? 3 : 2)))
+segment_kernel(const double *__restrict__ a, const double *__restrict__ b, const double *__restrict__ c,
+               const double *f, double *x, int ldk, int n, int ncol) {
+  constexpr int C = 64 / S, LV = M * N + 1;
+  __shared__ double sm[64 * (M * N * N + 1)], sv[64 * LV];  // a lane's rows and one double of padding
+  const int t = threadIdx.x, lane = t % S, cw = t / S;
+  const long c0 = (long)tgx_xcd_block(gridDim.x) * C;
+  const int nc = (int)min((long)C, ncol - c0);  // at least 1
+  Mat<N> A[M], B[M], Cm[M];
+  Vec<N> F[M], xs[M], xl;
+  load_rows<N, S, M>(t, a, b, c, f, c0, nc, ldk, n, sm, A, B, Cm, F);
+  bool bad;
+  eliminate<N, S, M>(A, B, Cm, F, lane, xs, xl, bad);
   if (N > 1) {
     // One correction of each row from its neighbours, x(k) += B^-1 (F - A
     // x(k-1) - B x(k) - C x(k+1)): takes the rounding of the two extra
@@ -379,9 +501,7 @@ segment_kernel(const double *__restrict__ a, const double *__restrict__ b, const
     for (int e = 0; e < M; ++e) {
       const Vec<N> next = e < M - 1 ? xs[e < M - 1 ? e + 1 : 0] : xn, here = xs[e];
       const Vec<N> r = mul(inverse(B[e]), sub(sub(sub(F[e], A[e], prev), B[e], here), Cm[e], next));
-      double big = 0.;
-#pragma unroll
-      for (int q = 0; q < N; ++q) big = fmax(fmax(big, fabs(here.v[q])), fmax(fabs(prev.v[q]), fabs(next.v[q])));
+      const double big = largest(prev, here, next);
 #pragma unroll
       for (int q = 0; q < N; ++q) {
         bad |= !(fabs(r.v[q]) <= CORRECTION * big);
@@ -395,29 +515,10 @@ segment_kernel(const double *__restrict__ a, const double *__restrict__ b, const
 #pragma unroll
     for (int q = 0; q < N; ++q) sv[t * LV + e * N + q] = xs[e].v[q];
   __syncthreads();
-  // a column some lane of which is badly pivoted goes by another way
-  const unsigned long long vote = __ballot(col && bad);
-  const int len = n * N;
-#pragma unroll
-  for (int cc = 0; cc < C; ++cc) {
-    const unsigned long long mine = (S == 64 ? ~0ull : ((1ull << (S & 63)) - 1)) << (cc * S & 63);
-    if (cc < nc && !(vote & mine))
-#pragma unroll
-      for (int q = 0; q < QV; ++q) {
-        const int e = 64 * q + t;
-        if (e < len) x[(size_t)(c0 + cc) * ldk * N + e] = sv[cc * S * LV + e + e / (M * N)];
-      }
-  }
-  if (vote) {
-    const unsigned long long mine = (S == 64 ? ~0ull : ((1ull << (S & 63)) - 1)) << (cw * S & 63);
-    const size_t o = (size_t)(c0 + cw) * ldk;
-    __syncthreads();
-    const bool redo = col && lane == 0 && (vote & mine);
-    if (redo) {
-      serial_column<N>(a + o * NN, b + o * NN, c + o * NN, f + o * N, sm + cw * S * LM, sv + cw * S * LV, n);
-      for (int e = 0; e < len; ++e) x[o * N + e] = sv[cw * S * LV + e];
-    }
-  }
+  const unsigned long long own = (S == 64 ? ~0ull : (1ull << (S & 63)) - 1) << (cw * S & 63);
+  const unsigned long long all = __ballot(cw < nc), vote = __ballot(bad), todo = __ballot((vote & own) != 0) & all;
+  store_columns<N, S, M>(all & ~todo, x, c0, ldk, n, sv);
+  if (todo) refine_columns<N, S, M>(a, b, c, f, x, ldk, n, c0, nc, sm, sv, todo);
 }
 
 template <int N, int S, int M>
