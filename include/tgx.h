@@ -154,6 +154,14 @@ int tgx_blktri2_dev_f64(const double *a, const double *b, const double *c, const
 int tgx_blktri3_dev_f64(const double *p, const double *q, const double *r, const double *f,
                         double *x, int ldk, int nrow, int col0, int ncol, void *stream);
 
+/* The same with the scheme chosen: TGX_SCHEME_THOMAS is the reference's
+ * operation order at every row count (thread per column, block gammas in
+ * scratch), TGX_SCHEME_PCR and TGX_SCHEME_AUTO what the calls above take. */
+int tgx_blktri2_dev_f64_scheme(const double *a, const double *b, const double *c, const double *f,
+                               double *x, int ldk, int nrow, int col0, int ncol, int scheme, void *stream);
+int tgx_blktri3_dev_f64_scheme(const double *p, const double *q, const double *r, const double *f,
+                               double *x, int ldk, int nrow, int col0, int ncol, int scheme, void *stream);
+
 /* Mixed precision for N x N block rows (N = 1, 2, 3; N = 1 is the scalar
  * system): FP32 elimination with each block pivot inverted in FP64, FP64
  * residual r = F - A x, nsweep (0..8) refinement sweeps reusing the FP32

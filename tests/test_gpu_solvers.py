@@ -486,3 +486,37 @@ def test_partitioned_solver_in_place(pkg, nblk, n):
     _segment_solve(pkg, nblk, sys_, x, n)
     _segment_solve(pkg, nblk, sys_, sys_[3], n)
     assert torch.equal(x, sys_[3]) and bool(torch.isfinite(x).all())
+
+
+@pytest.mark.parametrize("nblk", [2, 3])
+@pytest.mark.parametrize("n", [1, 2, 57, 256, 257])
+def test_block_rows_in_the_reference_order(pkg, oracle, nblk, n):
+    """TGX_SCHEME_THOMAS on block rows: the oracle's order of operations, to its
+    own 1e-14 on dominant rows, also where the default takes another (2 to 256
+    rows, whose bits differ); an unknown scheme is refused."""
+    import torch
+    from test_oracle_solvers import to_colmajor
+    rng = np.random.default_rng(n)
+    ncol = 70
+    A, B, C = (rng.uniform(-1, 1, (ncol, n, nblk, nblk)) for _ in range(3))
+    B = B + np.eye(nblk) * (np.abs(A) + np.abs(B) + np.abs(C)).sum((2, 3), keepdims=True)
+    F = rng.normal(size=(ncol, n, nblk))
+    A[:, 0] = 0.
+    C[:, n - 1] = 0.
+    y = np.zeros_like(F)
+    if nblk == 2:
+        ext = [np.concatenate([v, v[:, :1]], axis=1) for v in (A, B, C, F)]
+        z = np.zeros((ncol, n + 1, 2))
+        oracle.blktri(*[to_colmajor(v) for v in ext[:3]], np.ascontiguousarray(ext[3]), z, 1, n + 1, 5, 5 + ncol - 1, 100000)
+        y = z[:, :n]
+    else:
+        oracle.blktri3(to_colmajor(A), to_colmajor(B), to_colmajor(C), F, y, n, ncol, n)
+    solve = pkg.tgx.blktri2_dev if nblk == 2 else pkg.tgx.blktri3_dev
+    sys_ = [torch_dev(to_colmajor(v)) for v in (A, B, C)] + [torch_dev(F)]
+    x, d = (torch.zeros_like(sys_[3]) for _ in range(2))
+    solve(*sys_, x, n, scheme=pkg.tgx.SCHEME_THOMAS)
+    assert relerr(x.cpu().numpy(), y) <= 1e-14
+    solve(*sys_, d, n)
+    assert torch.equal(x, d) == (n > 256) or n == 1
+    with pytest.raises(pkg.tgx.TgxError):
+        solve(*sys_, x, n, scheme=7)

@@ -274,34 +274,38 @@ extern "C" int tgx_trsolv_dev_mixed(const double *a, const double *b, const doub
   return tgx_launch_mixed(a, b, c, f, x, ldk, k1, k2, col0, ncol, nsweep, (hipStream_t)stream);
 }
 
-extern "C" int tgx_blktri2_dev_f64(const double *a, const double *b, const double *c,
-                                   const double *f, double *x, int ldk, int nrow, int col0,
-                                   int ncol, void *stream) {
-  if (ldk <= 0 || nrow < 1 || nrow > ldk || col0 < 0 || ncol < 0)
-    return tgx_set_error(1, "tgx_blktri2_dev_f64: bad shape");
-  if (nrow <= kSegRows) {
-    const size_t o = (size_t)col0 * ldk;
-    return tgx_launch_segment(2, a + 4 * o, b + 4 * o, c + 4 * o, f + 2 * o, x + 2 * o, ldk, nrow, ncol,
-                              (hipStream_t)stream);
+namespace {
+int run_blocks(int nblk, const char *what, const double *a, const double *b, const double *c, const double *f, double *x,
+               int ldk, int nrow, int col0, int ncol, int scheme, hipStream_t s) {
+  if (ldk <= 0 || nrow < 1 || nrow > ldk || col0 < 0 || ncol < 0) return tgx_set_error(1, "%s: bad shape", what);
+  if (scheme < TGX_SCHEME_AUTO || scheme > TGX_SCHEME_PCR) return tgx_set_error(1, "%s: unknown scheme %d", what, scheme);
+  if (nrow <= kSegRows && scheme != TGX_SCHEME_THOMAS) {
+    const size_t o = (size_t)col0 * ldk, m = nblk * nblk * o, v = nblk * o;
+    return tgx_launch_segment(nblk, a + m, b + m, c + m, f + v, x + v, ldk, nrow, ncol, s);
   }
   void *gs = nullptr;
-  if (int rc = get_scratch(sizeof(double) * 4 * (size_t)ldk * (size_t)(col0 + ncol), (hipStream_t)stream, &gs)) return rc;
-  return tgx_launch_blktri2_f64(a, b, c, f, x, (double *)gs, ldk, nrow, col0, ncol, (hipStream_t)stream);
+  const size_t need = sizeof(double) * nblk * nblk * (size_t)ldk * (size_t)(col0 + ncol);
+  if (int rc = get_scratch(need, s, &gs)) return rc;
+  return (nblk == 2 ? tgx_launch_blktri2_f64 : tgx_launch_blktri3_f64)(a, b, c, f, x, (double *)gs, ldk, nrow, col0,
+                                                                      ncol, s);
 }
+}  // namespace
 
-extern "C" int tgx_blktri3_dev_f64(const double *p, const double *q, const double *r,
-                                   const double *f, double *x, int ldk, int nrow, int col0,
-                                   int ncol, void *stream) {
-  if (ldk <= 0 || nrow < 1 || nrow > ldk || col0 < 0 || ncol < 0)
-    return tgx_set_error(1, "tgx_blktri3_dev_f64: bad shape");
-  if (nrow <= kSegRows) {
-    const size_t o = (size_t)col0 * ldk;
-    return tgx_launch_segment(3, p + 9 * o, q + 9 * o, r + 9 * o, f + 3 * o, x + 3 * o, ldk, nrow, ncol,
-                              (hipStream_t)stream);
-  }
-  void *gs = nullptr;
-  if (int rc = get_scratch(sizeof(double) * 9 * (size_t)ldk * (size_t)(col0 + ncol), (hipStream_t)stream, &gs)) return rc;
-  return tgx_launch_blktri3_f64(p, q, r, f, x, (double *)gs, ldk, nrow, col0, ncol, (hipStream_t)stream);
+extern "C" int tgx_blktri2_dev_f64_scheme(const double *a, const double *b, const double *c, const double *f, double *x,
+                                          int ldk, int nrow, int col0, int ncol, int scheme, void *stream) {
+  return run_blocks(2, "tgx_blktri2_dev_f64", a, b, c, f, x, ldk, nrow, col0, ncol, scheme, (hipStream_t)stream);
+}
+extern "C" int tgx_blktri2_dev_f64(const double *a, const double *b, const double *c, const double *f, double *x,
+                                   int ldk, int nrow, int col0, int ncol, void *stream) {
+  return tgx_blktri2_dev_f64_scheme(a, b, c, f, x, ldk, nrow, col0, ncol, TGX_SCHEME_AUTO, stream);
+}
+extern "C" int tgx_blktri3_dev_f64_scheme(const double *p, const double *q, const double *r, const double *f, double *x,
+                                          int ldk, int nrow, int col0, int ncol, int scheme, void *stream) {
+  return run_blocks(3, "tgx_blktri3_dev_f64", p, q, r, f, x, ldk, nrow, col0, ncol, scheme, (hipStream_t)stream);
+}
+extern "C" int tgx_blktri3_dev_f64(const double *p, const double *q, const double *r, const double *f, double *x,
+                                   int ldk, int nrow, int col0, int ncol, void *stream) {
+  return tgx_blktri3_dev_f64_scheme(p, q, r, f, x, ldk, nrow, col0, ncol, TGX_SCHEME_AUTO, stream);
 }
 
 // ---- host drop-ins ------------------------------------------------------------

@@ -37,7 +37,9 @@ _SIGS = {
     "tgx_autotune_choice": ([_I] * 4, _I),
     "tgx_trsolv_dev_mixed": ([_D] * 5 + [_I] * 6 + [_D], _I),
     "tgx_blktri2_dev_f64": ([_D] * 5 + [_I] * 4 + [_D], _I),
+    "tgx_blktri2_dev_f64_scheme": ([_D] * 5 + [_I] * 5 + [_D], _I),
     "tgx_blktri3_dev_f64": ([_D] * 5 + [_I] * 4 + [_D], _I),
+    "tgx_blktri3_dev_f64_scheme": ([_D] * 5 + [_I] * 5 + [_D], _I),
     "tgx_ringfilter_f64": ([_D, _I, _I, _I, C.c_char_p, _I, _I, _I, C.c_double, _I, _D], None),
     "tgx_ringfilter_dev": ([_D] + [_I] * 6 + [C.c_double, _I, _D, _D], _I),
     "tgx_ng_pack_levels": ([_D, _D] + [_I] * 4 + [_D], _I),
@@ -194,10 +196,10 @@ def autotune_choice(ldk, k1, k2, ncol):
     return lib().tgx_autotune_choice(ldk, k1, k2, ncol)
 
 
-def blktri2_dev(a, b, c, f, x, nrow, stream=None):
+def blktri2_dev(a, b, c, f, x, nrow, stream=None, scheme=SCHEME_AUTO):
     ncol, ldk = a.shape[0], a.shape[1]
-    _check(lib().tgx_blktri2_dev_f64(_dp(a), _dp(b), _dp(c), _dp(f), _dp(x), ldk, nrow, 0, ncol,
-                                     _stream(stream)))
+    _check(lib().tgx_blktri2_dev_f64_scheme(_dp(a), _dp(b), _dp(c), _dp(f), _dp(x), ldk, nrow, 0, ncol,
+                                            scheme, _stream(stream)))
     return x
 
 
@@ -305,8 +307,8 @@ def ringfilter_dev(f, nlon, nlat, order, oplus, dlamda, chunk, stream=None):
     return f
 
 
-def blktri3_dev(p, q, r, f, x, nrow, stream=None):
+def blktri3_dev(p, q, r, f, x, nrow, stream=None, scheme=SCHEME_AUTO):
     ncol, ldk = p.shape[0], p.shape[1]
-    _check(lib().tgx_blktri3_dev_f64(_dp(p), _dp(q), _dp(r), _dp(f), _dp(x), ldk, nrow, 0, ncol,
-                                     _stream(stream)))
+    _check(lib().tgx_blktri3_dev_f64_scheme(_dp(p), _dp(q), _dp(r), _dp(f), _dp(x), ldk, nrow, 0, ncol,
+                                            scheme, _stream(stream)))
     return x
