@@ -135,14 +135,18 @@ int tgx_ng_step(const tgx_ng_grid *g, const tgx_ng_fields *in, const tgx_ng_out 
 /* Autotuner of TGX_SCHEME_AUTO: times each routine on `stream`
  * (host-synchronising; not for graph capture) under the Thomas scheme and
  * under the wavefront-per-column scheme with 1, 2 and 4 columns per block, and
- * keeps the fastest per device, shape and routine.  tgx_ng_step calls it on
- * the first AUTO step of a shape.  tgx_ng_scheme_choice reports the scheme a
- * routine (0..4 = oplus, minors, dt, duv, comp) runs with for this grid, and
- * tgx_ng_wave_columns_choice its columns per block when that is
+ * keeps the fastest per device, shape and routine for calls of that routine; in
+ * a step (tgx_ng_step, tgx_ng_step_serial) Thomas stays on small grids unless the
+ * other is clearly faster, because it leaves more room to the routines that run
+ * beside it.  tgx_ng_step calls it on the first AUTO step of a shape.
+ * tgx_ng_scheme_choice reports the scheme a routine (0..4 = oplus, minors, dt,
+ * duv, comp) runs with in a step for this grid, tgx_ng_scheme_choice_alone on its
+ * own, and tgx_ng_wave_columns_choice the columns per block where that is
  * TGX_SCHEME_PCR (4 unless tuned).  No reference counterpart. */
 int tgx_ng_autotune(const tgx_ng_grid *g, const tgx_ng_fields *in, const tgx_ng_out *out, void *work,
                     void *stream);
 int tgx_ng_scheme_choice(const tgx_ng_grid *g, int routine);
+int tgx_ng_scheme_choice_alone(const tgx_ng_grid *g, int routine);
 int tgx_ng_wave_columns_choice(const tgx_ng_grid *g, int routine);
 /* Columns per block (1, 2 or 4) of the wavefront-per-column kernels launched
  * from the calling host thread, in place of the autotuner's choice; 0 returns

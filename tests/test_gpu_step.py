@@ -523,3 +523,36 @@ def test_block_kernels_equal_thread_per_column(pkg, monkeypatch, shape, glb):
             for n in a:
                 rows = slice(2, nlat + 2) if glb and n not in ("op", "op_nm") else slice(None)
                 assert torch.equal(a[n][..., rows, :], b[n][..., rows, :]), n
+
+
+def test_autotuner_keeps_the_fastest_for_a_routine_on_its_own(pkg, monkeypatch):
+    """The block kernels are favoured in a step only, and only where they run: a
+    routine called on its own takes what was fastest alone, a favoured routine
+    Thomas in the step, and with the large-grid forms selected nothing is
+    favoured.  Each call's results show which scheme ran."""
+    import torch
+    outs = {"oplus": ("op", "Fe", "Fn"), "minors": ("n2d", "ar", "no", "n4s"), "dt": ("tn",), "duv": ("un", "vn"),
+            "comp": ("o2", "o1", "he")}
+    for n, (shape, large) in enumerate((((60, 40, 57), "0"), ((104, 54, 30), "0"), ((56, 40, 57), "1"))):
+        name = "tune%d" % n
+        monkeypatch.setitem(pkg.synth.CONFIGS, name, shape + (14. / (shape[2] - 1), 10., 10., None))
+        monkeypatch.setenv("TGX_LARGE_GRID_FORMS", large)
+        g = pkg.synth.make_grid(name, nstep_sub=1)
+        F = pkg.synth.make_state(g)
+        st = pkg.step.NestState(g, F, scheme="auto")
+        st.autotune()
+        alone, step = st.schemes(alone=True), st.schemes()
+        print("case %s large=%s alone %s step %s" % (shape, large, alone, step), flush=True)
+        assert all(step[r] == alone[r] or (large == "0" and step[r] == "thomas") for r in alone)
+        forced = {s: pkg.step.NestState(g, F, scheme=s) for s in ("thomas", "pcr")}
+        for s in forced.values():
+            s.step_serial()
+        st.step_serial()
+        for r in ("oplus", "minors", "dt", "comp"):
+            for f in outs[r]:
+                assert torch.equal(st.out[f], forced[step[r]].out[f]), (r, f)
+        for r in ("oplus", "minors", "dt", "comp"):
+            for s in (st, *forced.values()):
+                getattr(s, r)()
+            for f in outs[r]:
+                assert torch.equal(st.out[f], forced[alone[r]].out[f]), (r, f)

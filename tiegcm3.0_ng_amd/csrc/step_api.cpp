@@ -283,23 +283,32 @@ int comp_post(const tgx_ng_grid *g, const tgx_ng_fields *in, const tgx_ng_out *o
 namespace {
 // Solve scheme of each routine.  The wavefront-per-column cyclic reduction
 // holds at most 128 levels.  TGX_SCHEME_AUTO uses the choice timed by
-// tgx_ng_autotune for this device and shape (PCR until then).
+// tgx_ng_autotune for this device and shape (PCR until then): the fastest alone
+// for a routine called on its own, and in a step what leaves room for the
+// routines beside it (BLOCK_FAVOUR).
 typedef std::tuple<int, int, int, int, int, int, int> TuneKey;  // dev nk nlon nlat ld nsub routine
 std::mutex g_tune_mu;
-std::map<TuneKey, int> g_tune;
+struct TuneChoice { int alone, step; };  // schemes
+std::map<TuneKey, TuneChoice> g_tune;
 std::map<TuneKey, int> g_tune_cols;  // columns per block of the wavefront-per-column kernels
 thread_local int t_forced = -1;       // scheme forced while the autotuner times a routine
 thread_local int t_forced_cols = 0;   // and its columns per block (PCR)
+thread_local bool t_in_step = false;  // a whole step runs on this host thread
+struct StepScope {
+  bool prev = t_in_step;
+  StepScope() { t_in_step = true; }
+  ~StepScope() { t_in_step = prev; }
+};
 
 TuneKey tune_key(const tgx_ng_grid *g, int routine) {
   int dev = 0;
   (void)hipGetDevice(&dev);
   return TuneKey(dev, g->nk, g->nlon, g->nlat, g->ld, g->nstep_sub, routine);
 }
-int tuned_choice(const tgx_ng_grid *g, int routine) {
+int tuned_choice(const tgx_ng_grid *g, int routine, bool step) {
   std::lock_guard<std::mutex> lk(g_tune_mu);
   auto it = g_tune.find(tune_key(g, routine));
-  return it == g_tune.end() ? TGX_SCHEME_AUTO : it->second;
+  return it == g_tune.end() ? TGX_SCHEME_AUTO : step ? it->second.step : it->second.alone;
 }
 // Whether the routine runs the wavefront-per-column scheme; if so, its
 // columns per block (the autotuner's choice, else 4) are set for the launches
@@ -309,7 +318,7 @@ bool use_pcr(const tgx_ng_grid *g, int routine) {
   if (g->nk > 128 || t_glb) pcr = false;
   else if (t_forced >= 0) pcr = t_forced == TGX_SCHEME_PCR;
   else if (g->scheme != TGX_SCHEME_AUTO) pcr = g->scheme == TGX_SCHEME_PCR;
-  else pcr = tuned_choice(g, routine) != TGX_SCHEME_THOMAS;
+  else pcr = tuned_choice(g, routine, t_in_step) != TGX_SCHEME_THOMAS;
   if (pcr) {
     int cols = 4;
     if (t_forced_cols > 0) {
@@ -674,15 +683,17 @@ typedef int (*RoutineFn)(const tgx_ng_grid *, const tgx_ng_fields *, const tgx_n
 
 // In the step a routine runs beside the others, where the block kernels (16
 // threads per column) leave more room than a wavefront per column does, so
-// Thomas is kept unless the other scheme is this much faster alone.  104x54x57
-// columns, alone, block and wavefront: minor species 129 and 111 us, dt 40 and
-// 38; the nested outer step 4.03 ms with the block forms, 4.21 with what is
-// faster alone.  (60x40: minor species 88 and 66, left to the wavefront.)
+// their Thomas is kept there unless the other scheme is this much faster alone
+// (104x54x57 columns: minor species 129 us and 111, dt 40 and 38).  Steps with
+// and without it: nests of 60x40 to 150x100, 29 to 113 levels, one to five O+
+// sub-cycles, 0.96 to 1.13 times as fast, 1.03 on average over eight; nested outer
+// steps of four kinds 0.99 to 1.11, the largest 3.96 ms against 4.39.
 constexpr float BLOCK_FAVOUR = 0.83f;
 
 // Times every routine under both schemes on `stream` (reference order, so
-// duv sees this step's dt and oplus outputs) and keeps the faster scheme per
-// routine for this device and shape, the block kernels favoured.  The outputs are left as a full step
+// duv sees this step's dt and oplus outputs) and keeps per routine, for this
+// device and shape, the faster scheme for calls on its own and the scheme of a
+// step, the block kernels favoured.  The outputs are left as a full step
 // computed with the last scheme timed; the caller runs its step afterwards.
 extern "C" int tgx_ng_autotune(const tgx_ng_grid *g, const tgx_ng_fields *in, const tgx_ng_out *out,
                                void *work, void *stream) {
@@ -724,9 +735,10 @@ extern "C" int tgx_ng_autotune(const tgx_ng_grid *g, const tgx_ng_fields *in, co
     if (rc == 0) {
       int q = 0;
       for (int c = 1; c < nsch; ++c)
-        if (best[c] < (q == 0 && block_grid(g, r) ? BLOCK_FAVOUR : 1.f) * best[q]) q = c;
+        if (best[c] < best[q]) q = c;
+      const bool keep = q > 0 && use_block(g, r) && !(best[q] < BLOCK_FAVOUR * best[0]);
       std::lock_guard<std::mutex> lk(g_tune_mu);
-      g_tune[tune_key(g, r)] = schemes[q];
+      g_tune[tune_key(g, r)] = {schemes[q], keep ? TGX_SCHEME_THOMAS : schemes[q]};
       if (q > 0) g_tune_cols[tune_key(g, r)] = cols[q];
     }
   }
@@ -746,13 +758,17 @@ extern "C" int tgx_ng_wave_columns_choice(const tgx_ng_grid *g, int routine) {
   return it == g_tune_cols.end() ? 4 : it->second;
 }
 
-extern "C" int tgx_ng_scheme_choice(const tgx_ng_grid *g, int routine) {
+namespace {
+int scheme_choice(const tgx_ng_grid *g, int routine, bool step) {
   if (!g || routine < 0 || routine >= R_N) return tgx_set_error(1, "tgx_ng_scheme_choice: bad arguments");
   if (g->scheme != TGX_SCHEME_AUTO) return g->scheme;
   if (g->nk > 128) return TGX_SCHEME_THOMAS;
-  int c = tuned_choice(g, routine);
+  int c = tuned_choice(g, routine, step);
   return c == TGX_SCHEME_AUTO ? TGX_SCHEME_PCR : c;
 }
+}  // namespace
+extern "C" int tgx_ng_scheme_choice(const tgx_ng_grid *g, int routine) { return scheme_choice(g, routine, true); }
+extern "C" int tgx_ng_scheme_choice_alone(const tgx_ng_grid *g, int routine) { return scheme_choice(g, routine, false); }
 
 // Small grids outside a graph run comp on the minor species' stream and, with
 // one O+ sub-cycle, O+ on the caller's.  There the step is bound by the host: a
@@ -773,8 +789,9 @@ extern "C" int tgx_ng_step(const tgx_ng_grid *g, const tgx_ng_fields *in, const 
   // dynamics_ng.F90 order: oplus (:99-121), minors (:147-165), dt (:203),
   // duv (:210), comp_o2o + comp (:221-233)
   if (int rc = check(g, work)) return rc;
-  if (!t_glb && g->scheme == TGX_SCHEME_AUTO && g->nk <= 128 && tuned_choice(g, R_OPLUS) == TGX_SCHEME_AUTO)
+  if (!t_glb && g->scheme == TGX_SCHEME_AUTO && g->nk <= 128 && tuned_choice(g, R_OPLUS, true) == TGX_SCHEME_AUTO)
     if (int rc = tgx_ng_autotune(g, in, out, work, stream)) return rc;
+  StepScope in_step;
   Fork *F = nullptr;
   if (int rc = get_fork(&F)) return rc;
   const bool few = few_streams(g, (hipStream_t)stream), two = few && g->nstep_sub == 1;
@@ -851,8 +868,9 @@ extern "C" int tgx_ng_step(const tgx_ng_grid *g, const tgx_ng_fields *in, const 
 extern "C" int tgx_ng_step_serial(const tgx_ng_grid *g, const tgx_ng_fields *in,
                                   const tgx_ng_out *out, void *work, void *stream) {
   if (int rc = check(g, work)) return rc;
-  if (!t_glb && g->scheme == TGX_SCHEME_AUTO && g->nk <= 128 && tuned_choice(g, R_OPLUS) == TGX_SCHEME_AUTO)
+  if (!t_glb && g->scheme == TGX_SCHEME_AUTO && g->nk <= 128 && tuned_choice(g, R_OPLUS, true) == TGX_SCHEME_AUTO)
     if (int rc = tgx_ng_autotune(g, in, out, work, stream)) return rc;
+  StepScope in_step;
   if (int rc = run_chem(g, in, out, work, (hipStream_t)stream)) return rc;
   if (int rc = run_oplus(g, in, out, work, stream, true, g->nstep_sub)) return rc;
   if (int rc = run_minors(g, in, out, work, stream, true)) return rc;

@@ -76,6 +76,7 @@ _SIGS = {
     "tgx_ng_profile_begin": ([C.c_int], C.c_int),
     "tgx_ng_autotune": ([_P] * 5, C.c_int),
     "tgx_ng_scheme_choice": ([_P, C.c_int], C.c_int),
+    "tgx_ng_scheme_choice_alone": ([_P, C.c_int], C.c_int),
     "tgx_ng_wave_columns_choice": ([_P, C.c_int], C.c_int),
     "tgx_ng_force_wave_columns": ([C.c_int], None),
     "tgx_ng_set_tile_dma": ([C.c_int], None),
@@ -313,10 +314,12 @@ class NestState:
     def autotune(self, stream=None):
         self._call("tgx_ng_autotune", stream)
 
-    def schemes(self):
-        """The column-solve scheme each routine runs with ("thomas" / "pcr")."""
+    def schemes(self, alone=False):
+        """The column-solve scheme each routine runs with ("thomas" / "pcr") in a
+        step or, with alone, called on its own."""
         names = {1: "thomas", 2: "pcr"}
-        return {r: names.get(_lib().tgx_ng_scheme_choice(C.byref(self.g), n), "?")
+        choice = _lib().tgx_ng_scheme_choice_alone if alone else _lib().tgx_ng_scheme_choice
+        return {r: names.get(choice(C.byref(self.g), n), "?")
                 for n, r in enumerate(ROUTINES)}
 
     def wave_columns(self):
