@@ -556,3 +556,42 @@ def test_autotuner_keeps_the_fastest_for_a_routine_on_its_own(pkg, monkeypatch):
                 getattr(s, r)()
             for f in outs[r]:
                 assert torch.equal(st.out[f], forced[alone[r]].out[f]), (r, f)
+
+
+@pytest.mark.parametrize("mode", [1, 2], ids=["thread_local", "relaxed"])
+def test_step_on_the_default_stream_beside_a_capture(pkg, mode):
+    """A step on the default stream while another host thread captures a blocking
+    stream of its own: the runtime refuses questions about the default stream
+    then, the step does not depend on one."""
+    import ctypes
+    import threading
+    import torch
+    g = pkg.synth.make_grid("small")
+    F = pkg.synth.make_state(g)
+    a, b = pkg.step.NestState(g, F, scheme="thomas"), pkg.step.NestState(g, F, scheme="thomas")
+    a.step()
+    torch.cuda.synchronize()
+    hip = ctypes.CDLL("libamdhip64.so")
+    stream, graph = ctypes.c_void_p(), ctypes.c_void_p()
+    assert hip.hipStreamCreate(ctypes.byref(stream)) == 0
+    begun, stepped, rc = threading.Event(), threading.Event(), []
+
+    def capture():
+        rc.append(hip.hipStreamBeginCapture(stream, mode))
+        begun.set()
+        stepped.wait(60)
+        rc.append(hip.hipStreamEndCapture(stream, ctypes.byref(graph)))
+
+    t = threading.Thread(target=capture)
+    t.start()
+    try:
+        assert begun.wait(60)
+        b.step(stream=0)
+    finally:
+        stepped.set()
+        t.join()
+    assert rc == [0, 0]
+    assert hip.hipGraphDestroy(graph) == 0 and hip.hipStreamDestroy(stream) == 0
+    torch.cuda.synchronize()
+    for n in a.out:
+        assert torch.equal(a.out[n], b.out[n]), n

@@ -780,6 +780,9 @@ extern "C" int tgx_ng_scheme_choice_alone(const tgx_ng_grid *g, int routine) { r
 // in a graph, where waits cost the host nothing, four are faster at any size.
 static bool few_streams(const tgx_ng_grid *g, hipStream_t s) {
   if ((long)(g->nlon + 4) * (g->nlat + 4) * g->nk > 450000) return false;
+  // the default stream is never captured, and asking about it is an error, which
+  // the next launch's check would report, while any blocking stream is
+  if (!s || s == hipStreamLegacy) return true;
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
   return hipStreamIsCapturing(s, &st) == hipSuccess && st == hipStreamCaptureStatusNone;
 }
