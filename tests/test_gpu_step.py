@@ -595,3 +595,25 @@ def test_step_on_the_default_stream_beside_a_capture(pkg, mode):
     torch.cuda.synchronize()
     for n in a.out:
         assert torch.equal(a.out[n], b.out[n]), n
+
+
+@pytest.mark.parametrize("glb", [False, True], ids=["nest", "global"])
+@pytest.mark.parametrize("nk,nsub", [(29, 1), (80, 1), (29, 3), (81, 1)], ids=["two", "two_limit", "three", "four"])
+def test_forked_step_equals_serial_for_every_number_of_streams(pkg, monkeypatch, nk, nsub, glb):
+    """Outside a graph small grids fork fewer streams, by levels and O+
+    sub-cycles; each schedule gives the serial step bit for bit, three in a row."""
+    import torch
+    name = "fork%d" % nk
+    monkeypatch.setitem(pkg.synth.CONFIGS, name, (24, 12, nk, 14. / (nk - 1), 10., 10., None))
+    monkeypatch.setitem(pkg.tgx.RING_CHUNKS, (24, 12), [3, 6, 12])
+    g = pkg.synth.make_grid(name, nstep_sub=nsub, glb=glb)
+    F = (pkg.synth.make_global_state if glb else pkg.synth.make_state)(g)
+    new = (lambda: pkg.step.GlobalState(g, F)) if glb else (lambda: pkg.step.NestState(g, F, scheme="thomas"))
+    a, b = new(), new()
+    a.step_serial()
+    for _ in range(3):
+        b.step()
+    torch.cuda.synchronize()
+    rows = slice(2, 14) if glb else slice(None)
+    for n in a.out:
+        assert torch.equal(a.out[n][..., rows, :], b.out[n][..., rows, :]), n

@@ -773,13 +773,20 @@ extern "C" int tgx_ng_scheme_choice_alone(const tgx_ng_grid *g, int routine) { r
 // Small grids outside a graph run comp on the minor species' stream and, with
 // one O+ sub-cycle, O+ on the caller's.  There the step is bound by the host: a
 // launch costs it 3 us, but a wait for another stream's event 8-10 us, and two
-// streams take three waits where four take eight.  72x36x29: 235 us per step
-// with two streams, 290 with four, 270 on one.  100x50x57 nest with five
-// sub-cycles, whose O+ chain is the longest: 461 us with three streams, 478 with
-// two, 510 with four; 144x72x57 with ten: 1185 us with two and 1140 with four, and
-// in a graph, where waits cost the host nothing, four are faster at any size.
+// streams take three waits where four take eight.  With one sub-cycle that pays
+// while the kernels' own chain, which grows with the levels as well as with the
+// points, is shorter than the host's work (steps, four streams and two, us):
+// 72x36x29 global 268 and 228, 48x24x57 285 and 255, 96x48x29 (151,000 points) 288
+// and 244, 36x18x72 280 and 252; 50x30x57 nest 224 and 169; but 60x40x57 (160,000) 211 and 216, 72x36x57
+// global 266 and 278, 120x60x29 273 and 297, and 48x24x100 (146,000) 278 and 346.
+// With several sub-cycles, whose O+ chain is the longest and has a stream of its
+// own, three streams are as fast as four or faster up to 450,000 points: 72x36x29
+// with five 344 and 329, 100x50x57 nest 471 and 459, 120x60x50 nest 528 and 511;
+// 60x30x113 global with three 423 and 429; 144x72x57 with ten loses 4%.  In a
+// graph, where waits cost the host nothing, four are faster at any size.
 static bool few_streams(const tgx_ng_grid *g, hipStream_t s) {
-  if ((long)(g->nlon + 4) * (g->nlat + 4) * g->nk > 450000) return false;
+  const long points = (long)(g->nlon + 4) * (g->nlat + 4) * g->nk;
+  if (g->nstep_sub == 1 ? points > 155000 || g->nk > 80 : points > 450000) return false;
   // the default stream is never captured, and asking about it is an error, which
   // the next launch's check would report, while any blocking stream is
   if (!s || s == hipStreamLegacy) return true;
