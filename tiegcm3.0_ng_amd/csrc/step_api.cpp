@@ -178,14 +178,20 @@ size_t tile_elems(const tgx_ng_grid *g) {
 // levels 0.36 and 0.21; 11,248 x 57 0.86 and 0.55 (ten O+ sub-cycles 2.96 and
 // 1.31); 11,248 x 113 1.63 and 1.23; 17,296 x 57 0.96 and 0.79; 24,640 x 57
 // 1.11 and 1.13, x 113 2.17 and 2.48.  dt and O+ alone gain further up
-// (43,216 x 113: dt 0.58 and 0.37; the step at five O+ sub-cycles 6.36 and
-// 5.86, at one 3.34 and 3.35; 66,976 x 57 loses 3%).  comp's block form moves
+// (43,216 x 113: dt 0.58 and 0.37; the step at five O+ sub-cycles 6.25 and
+// 5.21; 66,976 x 57 loses 3%), in a global step with one sub-cycle, whose other
+// routines fill the chip, only as far as kBlockColsStep (24,640 x 57 1.08 and 1.03, x
+// 113 2.15 and 2.04; 33,280 x 57 1.325 and 1.333, x 113 2.65 and 2.61; 43,216 x 57
+// 1.66 and 1.69, x 113 3.29 and 3.33; a nest's step gains there too, 46,816 x 90 3.08
+// and 3.00).  comp's block form moves
 // its rows through the workspace and only pays on the smallest grids (5,200 x
 // 57: step 0.36 and 0.34; 11,248 x 57: 0.55 and 0.65).
 constexpr long kBlockCols[5] = {49152, 20480, 49152, 20480, 5400};
+constexpr long kBlockColsStep = 38000;
 // (their LDS holds up to 128 levels)
-bool block_grid(const tgx_ng_grid *g, int routine) {
-  return g->nk <= 128 && (long)(g->nlon + 4) * (g->nlat + 4) < kBlockCols[routine];
+bool block_grid(const tgx_ng_grid *g, int routine, bool step = false) {
+  const long cols = (long)(g->nlon + 4) * (g->nlat + 4);
+  return g->nk <= 128 && cols < kBlockCols[routine] && !(step && t_glb && g->nstep_sub == 1 && cols >= kBlockColsStep);
 }
 
 double *tiles(void *work, const tgx_ng_grid *g, int idx) {
@@ -341,7 +347,7 @@ namespace {
 // thread-per-column kernels on every grid.
 bool use_block(const tgx_ng_grid *g, int routine) {
   const char *large = getenv("TGX_LARGE_GRID_FORMS");
-  return !g->capture && block_grid(g, routine) && !(large && large[0] == '1' && large[1] == 0);
+  return !g->capture && block_grid(g, routine, t_in_step) && !(large && large[0] == '1' && large[1] == 0);
 }
 }  // namespace
 
