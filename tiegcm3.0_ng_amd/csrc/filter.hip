@@ -357,11 +357,11 @@ ringfilter_kernel(Fields P, long plane, Rows R, int nlon, int nkp, int order, in
 // With the table in device memory: one wavefront per block, at most 128
 // VGPRs, so that four wavefronts of it fit on a SIMD beside the column
 // kernels of the routines running at the same time.
-template <int NPL, int MO>
+template <int NPL>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(NPL <= 9 ? 4 : NPL <= 18 ? 3 : 2)))
 ringfilter_gtab_kernel(Fields P, long plane, Rows R, int nlon, int nkp, int order, int oplus, double dlamda, int wl,
                        const double *__restrict__ gtab, int tord) {
-  ringfilter_body<NPL, true, MO>(P, plane, R, nlon, nkp, order, oplus, dlamda, wl, gtab, tord);
+  ringfilter_body<NPL, true, TGX_GLB_RING_ORDER>(P, plane, R, nlon, nkp, order, oplus, dlamda, wl, gtab, tord);
 }
 
 // The table of ringfilter_gtab_kernel: cos(m ang) and sin(m ang) of
@@ -478,12 +478,8 @@ int launch(const Fields &P, int nkp, long plane, int nrows, const Rows &R, int n
     // routines running at the same time
     const size_t lds = sizeof(double) * wl;
     const unsigned ny = (unsigned)((long)P.nf * nkp);
-    if (order <= 3)
-      hipLaunchKernelGGL((ringfilter_gtab_kernel<NPL, 3>), dim3((unsigned)nrows, ny), dim3(64), lds, s, P, plane, R,
-                         nlon, nkp, order, oplus, dlamda, wl, gtab, tord);
-    else
-      hipLaunchKernelGGL((ringfilter_gtab_kernel<NPL, kMaxOrder>), dim3((unsigned)nrows, ny), dim3(64), lds, s, P,
-                         plane, R, nlon, nkp, order, oplus, dlamda, wl, gtab, tord);
+    hipLaunchKernelGGL((ringfilter_gtab_kernel<NPL>), dim3((unsigned)nrows, ny), dim3(64), lds, s, P, plane, R, nlon,
+                       nkp, order, oplus, dlamda, wl, gtab, tord);
   } else if (!table_fits(nlon, order, wl, &W)) {
     if (P.nf != 1 || P.kind != POST_NONE || nkp != P.nlev)
       return tgx_set_error(TGX_ERR_ARG, "ring filter: fused post pass needs the LDS table (nlon %d, order %d)",
@@ -535,7 +531,7 @@ int launch_rows(const tgx::ring::Fields &P, int nkp, long plane, int nrows, cons
     R.off[r] = rowoff[r];
     R.n[r] = nchnk[r];
   }
-  if (gtab && order > tord)
+  if (gtab && (order > tord || order > TGX_GLB_RING_ORDER))
     return tgx_set_error(TGX_ERR_ARG, "ring filter: order %d beyond the table's %d", order, tord);
   return tgx::ring::launch_any(P, nkp, plane, nrows, R, nlon, order, oplus, dlamda, gtab, tord, s);
 }

@@ -6364,18 +6364,22 @@ extern "C" int tgx_ng_launch(int which, const tgx_ng_grid *gp, const tgx_ng_fiel
     jb.kind = kind; jb.f = f; jb.out = o; jb.s = sh;
     return jb;
   };
-  // a block kernel whose columns hold `vals` LDS doubles per level, 16 columns
-  // per block or, where those take more than 64 KB, 8
-#define LAUNCH_BLOCK(kern, vals, ...)                                                                              \
-  do {                                                                                                             \
-    const size_t per = sizeof(double) * (vals) * (size_t)G.nk;                                                     \
-    const unsigned rows = (unsigned)G.nlatd;                                                                       \
-    if (16 * per <= BLOCK_LDS)                                                                                     \
-      hipLaunchKernelGGL((kern<16>), dim3((unsigned)((G.nlond + 15) / 16) * rows), dim3(16 * BSEG), 16 * per, s, g, G, \
-                         in, out, __VA_ARGS__);                                                                    \
-    else                                                                                                           \
-      hipLaunchKernelGGL((kern<8>), dim3((unsigned)((G.nlond + 7) / 8) * rows), dim3(8 * BSEG), 8 * per, s, g, G, in, \
-                         out, __VA_ARGS__);                                                                        \
+  // a block kernel whose columns hold `vals` LDS doubles per level: 16 columns per
+  // block (of up to 4 values at 128 levels) or, where those take more than 64 KB, 8
+#define LAUNCH_BLOCK_N(kern, cols, vals, ...)                                                                       \
+  hipLaunchKernelGGL((kern<cols>), dim3((unsigned)((G.nlond + (cols) - 1) / (cols)) * (unsigned)G.nlatd),             \
+                     dim3((cols) * BSEG), (cols) * sizeof(double) * (vals) * (size_t)G.nk, s, g, G, in, out, __VA_ARGS__)
+#define LAUNCH_BLOCK(kern, vals, ...)                                                            \
+  do {                                                                                           \
+    static_assert(16 * sizeof(double) * (vals) * 128 <= BLOCK_LDS, "8 columns from some level on"); \
+    LAUNCH_BLOCK_N(kern, 16, vals, __VA_ARGS__);                                                 \
+  } while (0)
+#define LAUNCH_BLOCK_8(kern, vals, ...)                              \
+  do {                                                               \
+    if (16 * sizeof(double) * (vals) * (size_t)G.nk <= BLOCK_LDS)    \
+      LAUNCH_BLOCK_N(kern, 16, vals, __VA_ARGS__);                   \
+    else                                                             \
+      LAUNCH_BLOCK_N(kern, 8, vals, __VA_ARGS__);                    \
   } while (0)
   switch (which) {
     case 20:
@@ -6394,7 +6398,7 @@ extern "C" int tgx_ng_launch(int which, const tgx_ng_grid *gp, const tgx_ng_fiel
       break;
     case 40: {  // duv stage 2: bufs = {ztmp, (unused), divx_ztmp, divy_z, unms, vnms, advu, advv}
       UvTerms UT{D(2), D(3), D(4), D(5), D(6), D(7)};
-      LAUNCH_BLOCK(duv_block_kernel, 8, UT);
+      LAUNCH_BLOCK_8(duv_block_kernel, 8, UT);
       break;
     }
     case 25: {  // bufs = {comp input tiles, fs(:,1,0), fs(:,2,0), (unused x3), minor source tiles,
@@ -6460,11 +6464,11 @@ extern "C" int tgx_ng_launch(int which, const tgx_ng_grid *gp, const tgx_ng_fiel
         MT.n2d = out.n2d;
       }
       if (which == 44)  // a block per 16 columns, as 1, 2 and 27
-        LAUNCH_BLOCK(minor_block_a_kernel, 8, MT);
+        LAUNCH_BLOCK_8(minor_block_a_kernel, 8, MT);
       else if (which == 45)
-        LAUNCH_BLOCK(minor_block_b_kernel, 8, MT);
+        LAUNCH_BLOCK_8(minor_block_b_kernel, 8, MT);
       else if (which == 46)
-        LAUNCH_BLOCK(minor_block_b_lin_kernel, 8, MT);
+        LAUNCH_BLOCK_8(minor_block_b_lin_kernel, 8, MT);
       else if (which == 1 && g.capture)
         hipLaunchKernelGGL((minor_kernel<2, 3, true>), grid, block, 0, s, g, G, in, out, D(0), MT);
       else if (which == 1)
