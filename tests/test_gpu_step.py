@@ -617,3 +617,20 @@ def test_forked_step_equals_serial_for_every_number_of_streams(pkg, monkeypatch,
     rows = slice(2, 14) if glb else slice(None)
     for n in a.out:
         assert torch.equal(a.out[n][..., rows, :], b.out[n][..., rows, :]), n
+
+
+@pytest.mark.parametrize("fn", ["step", "step_serial"])
+def test_profile_hooks_time_each_routine_once_per_step(pkg, fn):
+    """One call per routine and step, the minor species' too where the step
+    queues their prelude apart; as many O+ column kernels as sub-cycles."""
+    import torch
+    g = pkg.synth.make_grid("small", nstep_sub=2)
+    ns = pkg.step.NestState(g, pkg.synth.make_state(g), scheme="thomas")
+    getattr(ns, fn)()
+    pkg.step.profile_begin(20)
+    for _ in range(3):
+        getattr(ns, fn)()
+    torch.cuda.synchronize()
+    prof, kern = pkg.step.profile_end()
+    assert {r: n for r, (_, n) in prof.items()} == {r: 3 for r in pkg.step.ROUTINES}
+    assert {r: n for r, (_, n) in kern.items()} == {r: 6 if r == "oplus" else 3 for r in pkg.step.ROUTINES}

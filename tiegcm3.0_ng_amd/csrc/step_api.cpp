@@ -5,6 +5,7 @@
 #include <cstdlib>
 #include <map>
 #include <mutex>
+#include <optional>
 #include <tuple>
 #include <vector>
 
@@ -429,12 +430,13 @@ extern "C" int tgx_ng_comp(const tgx_ng_grid *g, const tgx_ng_fields *in, const 
 
 namespace {
 // The stencil prelude reads no output of the chemistry pass; the column
-// kernels do.
+// kernels do.  Queued in parts, the caller times the routine.
 int run_minors(const tgx_ng_grid *g, const tgx_ng_fields *in, const tgx_ng_out *out, void *work,
                void *stream, bool chem_done, int parts) {
   if (int rc = check(g, work)) return rc;
   hipStream_t s = (hipStream_t)stream;
-  ProfScope prof(R_MINORS, s);
+  std::optional<ProfScope> prof;
+  if (parts == PART_ALL) prof.emplace(R_MINORS, s);
   void *b[14];
   b[0] = tiles(work, g, T_MW);
   b[1] = tiles(work, g, T_MR);
@@ -851,6 +853,7 @@ extern "C" int tgx_ng_step(const tgx_ng_grid *g, const tgx_ng_fields *in, const 
   // and comp before the minor species, 3.91.  Some 40 orders were tried; steps
   // outside a graph hardly depend on it.
   const bool early = !few && !t_glb;
+  std::optional<ProfScope> minors(std::in_place, R_MINORS, sb);
   if (int rc = run_minors(g, in, out, work, sb, true, PART_PRELUDE)) return rc;
   if (early) {
     TGX_HIP(join.fork(2, 5));
@@ -869,6 +872,7 @@ extern "C" int tgx_ng_step(const tgx_ng_grid *g, const tgx_ng_fields *in, const 
   }
   TGX_HIP(hipStreamWaitEvent(sb, F->ev[0], 0));
   if (int rc = run_minors(g, in, out, work, sb, true, PART_COLUMNS)) return rc;
+  minors.reset();
   if (!early) {
     if (!few) TGX_HIP(join.fork(2, 0));
     if (int rc = run_comp(g, in, out, work, sc, true)) return rc;
