@@ -108,11 +108,13 @@ int tgx_ringfilter_dev(double *f, int nk, int nlon, int nlat, int ld, int order,
 /* Column j of the batch starts at ptr + (col0+j)*ldk (scalars) and rows
  * k1..k2 (0-based, inclusive) are solved. */
 
-/* scheme: TGX_SCHEME_THOMAS (thread per column, reference operation order),
- * TGX_SCHEME_PCR (4 to 32 lanes per column, each lane eliminating its rows in
+/* scheme: TGX_SCHEME_THOMAS (one lane per column eliminating in the reference's
+ * operation order, from LDS up to 511 rows, beyond from HBM),
+ * TGX_SCHEME_PCR (8 to 32 lanes per column, each lane eliminating its rows in
  * registers, cyclic reduction across the lanes; at most 256 rows; a column
- * whose segments are badly pivoted on their own is solved in the reference
- * order), TGX_SCHEME_AUTO (timed once per shape, cached). */
+ * whose segments are badly pivoted on their own is refined from its residual,
+ * or solved in the reference's order where nothing finite came out),
+ * TGX_SCHEME_AUTO (timed once per shape, cached). */
 int tgx_trsolv_dev_f64(const double *a, const double *b, const double *c, const double *f,
                        double *x, int ldk, int k1, int k2, int col0, int ncol, int scheme,
                        void *stream);
@@ -123,13 +125,14 @@ int tgx_autotune_choice(int ldk, int k1, int k2, int ncol);
  * for callers that cannot allocate device memory (code under HIP graph
  * capture, tight serving loops, hosts that forbid hipMalloc).  Same arguments
  * and results as tgx_trsolv_dev_f64; it calls no hipMalloc, hipFree or other
- * allocating routine.  The Thomas scheme keeps its ratios in a fixed device
- * array of TGX_NOALLOC_SCRATCH_DOUBLES doubles (64 MiB) that the library holds
- * on every GPU it runs on until the process ends, so ldk*ncol must not exceed
- * TGX_NOALLOC_SCRATCH_DOUBLES (TGX_ERR_ARG otherwise; PCR needs no scratch).
- * Every call on one GPU shares that GPU's array: calls that overlap in time
+ * allocating routine.  The Thomas scheme keeps the ratios of columns beyond 511
+ * rows in a fixed device array of TGX_NOALLOC_SCRATCH_DOUBLES doubles (64 MiB)
+ * that the library holds on every GPU it runs on until the process ends; at
+ * every row count ldk*ncol must not exceed TGX_NOALLOC_SCRATCH_DOUBLES under
+ * Thomas (TGX_ERR_ARG otherwise; PCR has no such limit).
+ * Thomas calls beyond 511 rows share the GPU's array: those that overlap in time
  * on one GPU (other streams, other host threads) race and must be ordered by
- * the caller.  TGX_SCHEME_AUTO takes the autotuner's cached choice for the
+ * the caller; all others may overlap.  TGX_SCHEME_AUTO takes the autotuner's cached choice for the
  * shape if tgx_trsolv_dev_f64 made one, else Thomas; it never times. */
 #define TGX_NOALLOC_SCRATCH_DOUBLES (8u * 1024u * 1024u)
 int tgx_trsolv_dev_f64_noalloc(const double *a, const double *b, const double *c, const double *f,
@@ -145,7 +148,8 @@ int tgx_trsolv_dev_mixed(const double *a, const double *b, const double *c, cons
 
 /* 2x2 block rows (duv.F:830-906): a,b,c (2,2,ldk,·), f,x (2,ldk,·);
  * rows 0..nrow-1.  Up to 256 rows by the partitioned elimination of
- * TGX_SCHEME_PCR, block form; beyond, thread per column in reference order. */
+ * TGX_SCHEME_PCR, block form (16 to 64 lanes per column); beyond, thread per
+ * column in reference order. */
 int tgx_blktri2_dev_f64(const double *a, const double *b, const double *c, const double *f,
                         double *x, int ldk, int nrow, int col0, int ncol, void *stream);
 

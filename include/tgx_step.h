@@ -32,8 +32,9 @@ typedef struct {
   int nk, nlon, nlat, ld;
   int nstep_sub;      /* O+ sub-cycles per step (input namelist NSTEP_SUB) */
   int calc_helium;
-  int scheme;         /* column solve: TGX_SCHEME_THOMAS (thread per column, the
-                         reference's operation order), TGX_SCHEME_PCR (one
+  int scheme;         /* column solve: TGX_SCHEME_THOMAS (the reference's operation
+                         order; a thread per column, or on small grids 16
+                         threads with the same results), TGX_SCHEME_PCR (one
                          wavefront per column, cyclic reduction, nk <= 128) or
                          TGX_SCHEME_AUTO (the faster one, timed once per shape) */
   double dz;          /* dz(i_ng) = dlev_ng */
@@ -96,7 +97,9 @@ typedef struct {
 } tgx_ng_out;
 
 /* Bytes of device workspace the step needs for this grid (Thomas ratios,
- * block gammas, O+ and wind intermediates). */
+ * block gammas, O+ and wind intermediates).  A buffer that several grids share
+ * takes the largest of their bytes, which need not be the largest grid's: grids
+ * of fewer than 5,400 columns keep comp's rows in it too. */
 unsigned long long tgx_ng_workspace_bytes(const tgx_ng_grid *g);
 
 /* The routines, each on its own; work is a device buffer of

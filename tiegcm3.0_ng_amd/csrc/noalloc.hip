@@ -1,7 +1,8 @@
 // Allocation-free form of tgx_trsolv_dev_f64 for callers that cannot allocate
 // device memory (code under HIP graph capture, tight serving loops, hosts that
-// forbid hipMalloc).  The Thomas ratios live in a file-scope device array of
-// fixed size instead of a library-allocated buffer; see include/tgx.h.
+// forbid hipMalloc).  The Thomas ratios of columns beyond 511 rows (shorter ones
+// stay in LDS) live in a file-scope device array of fixed size instead of a
+// library-allocated buffer; the size limits every Thomas batch; see include/tgx.h.
 #include <hip/hip_runtime.h>
 
 #include <mutex>

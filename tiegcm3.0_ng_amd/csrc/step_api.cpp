@@ -640,9 +640,9 @@ int run_comp(const tgx_ng_grid *g, const tgx_ng_fields *in, const tgx_ng_out *ou
 
 // Concurrency of the step: oplus, the minor species, dt and comp read only
 // the step's inputs and write disjoint outputs and workspace planes, so they
-// run on streams forked from the caller's (three, or on small grids one:
-// two_streams); duv needs dt's TN and oplus' Fe/Fn and joins both.  All streams
-// have the default priority.
+// run on streams forked from the caller's (three; on small grids outside a graph
+// two, or with one O+ sub-cycle one: few_streams); duv needs dt's TN and oplus'
+// Fe/Fn and joins both.  All streams have the default priority.
 namespace {
 // The fork streams and events belong to the calling host thread (one set per
 // thread and device): calls from several threads never share an event, and
