@@ -3480,13 +3480,14 @@ struct OpTerms {  // prelude planes of one sub-step
 // FULL = false (the middle sub-steps of a sub-cycled step): only the values
 // that depend on O+ (bvel, tp_op, diffj, op/bmod2**2); dj, bdotu and dj*bz
 // stay those of the first sub-step, and Fe, Fn are left to the last one.
-// keep_vni: Fe receives the collision frequency, from which the last
-// sub-step's oplus_sub_prelude forms Fe and Fn.
-template <bool RUNS, bool FULL>  // RUNS false: nrun == 1, the whole column (a fixed loop)
+// KEEP: Fe receives the collision frequency, from which the last sub-step's
+// oplus_sub_prelude forms Fe and Fn (decided at run time, the branch cost the
+// 0.625 deg grid's columns 10%: 812 us and 898).
+template <bool RUNS, bool FULL, bool KEEP>  // RUNS false: nrun == 1, the whole column (a fixed loop)
 __global__ void __launch_bounds__(256) oplus_stage1(tgx_ng_grid g, Geo G, tgx_ng_fields in,
                                                     const double *__restrict__ op, OpWork W,
                                                     double *__restrict__ Fe, double *__restrict__ Fn,
-                                                    int nrun, int keep_vni) {
+                                                    int nrun) {
   const int nb = gridDim.x;
   const long tid = (long)tgx_xcd_block(nb) * blockDim.x + threadIdx.x;
   const int nk = G.nk;
@@ -3535,7 +3536,7 @@ __global__ void __launch_bounds__(256) oplus_stage1(tgx_ng_grid g, Geo G, tgx_ng
       dj = dj < cap ? dj : cap;
     }
     double bdotu = bx * in.un[p] + by * in.vn[p] + hj * bz * wni;
-    if (keep_vni) {
+    if (KEEP) {
       Fe[p] = vni;
     } else {
       double wd = vni * diffj * dj;
@@ -6542,15 +6543,19 @@ extern "C" int tgx_ng_launch(int which, const tgx_ng_grid *gp, const tgx_ng_fiel
       } else if (which == 3 || which == 49 || which == 31) {  // 31: the O+-dependent values only; 49: keeps vni in Fe
         const int nrun = oplus_runs(ncol, G.nk, 1);
         dim3 grid1((unsigned)((ncol * nrun + 255) / 256));
-        if (which == 31) {
-          if (nrun > 1)
-            hipLaunchKernelGGL((oplus_stage1<true, false>), grid1, block, 0, s, g, G, in, op, W, out.Fe, out.Fn, nrun, which == 49);
-          else
-            hipLaunchKernelGGL((oplus_stage1<false, false>), grid1, block, 0, s, g, G, in, op, W, out.Fe, out.Fn, 1, which == 49);
-        } else if (nrun > 1)
-          hipLaunchKernelGGL((oplus_stage1<true, true>), grid1, block, 0, s, g, G, in, op, W, out.Fe, out.Fn, nrun, which == 49);
+        auto stage1 = [&](auto kernel) {
+          hipLaunchKernelGGL(kernel, grid1, block, 0, s, g, G, in, op, W, out.Fe, out.Fn, nrun);
+        };
+        if (which == 49)  // grids with the block form, whose runs are two levels
+          stage1(oplus_stage1<true, true, true>);
+        else if (which == 31 && nrun > 1)
+          stage1(oplus_stage1<true, false, false>);
+        else if (which == 31)
+          stage1(oplus_stage1<false, false, false>);
+        else if (nrun > 1)
+          stage1(oplus_stage1<true, true, false>);
         else
-          hipLaunchKernelGGL((oplus_stage1<false, true>), grid1, block, 0, s, g, G, in, op, W, out.Fe, out.Fn, 1, which == 49);
+          stage1(oplus_stage1<false, true, false>);
       } else if (which == 4) {
         const int nrun = oplus_runs(ncol, G.nk, 2);
         dim3 grid2((unsigned)((ncol * nrun + 255) / 256));
