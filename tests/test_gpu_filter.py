@@ -113,3 +113,10 @@ def test_ringfilter_forms_at_their_limits(pkg, oracle, nlon, order, nk, oplus):
         oracle.ringfilter_row(row, nlon, order, oplus, nc, dlam)
         scale = np.abs(row).max(axis=1, keepdims=True)
         assert float((np.abs(got[:, j, :nlon + 4] - row) / scale).max()) <= TOL, (lat, nc)
+
+
+@pytest.mark.parametrize("nlon,order,nk", [(1024, 3, 5), (1026, 3, 5), (1152, 3, 4), (1536, 2, 3)])
+def test_ringfilter_rows_too_long_for_two_wavefronts_and_a_table(pkg, oracle, nlon, order, nk):
+    """The last row that takes the table (two wavefronts beside it) and rows
+    beyond, where the sincos are formed as they are used."""
+    test_ringfilter_forms_at_their_limits(pkg, oracle, nlon, order, nk, 0)

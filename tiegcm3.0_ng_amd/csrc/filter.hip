@@ -456,12 +456,16 @@ __global__ void __launch_bounds__(64) ringfilter_direct_kernel(double *__restric
   if (lane == 3) row[nlon + 3] = wm[1];
 }
 
-// Whether the table and the rows of up to kWaves wavefronts fit in a block's LDS; if not,
-// the launcher filters with ringfilter_direct_kernel (one field, no post pass).
+// Whether the table and the rows of 2 to kWaves wavefronts fit in a block's LDS;
+// if not, the launcher filters with ringfilter_direct_kernel (one field, no post
+// pass).  A table for one wavefront's level takes as many sincos as that filter
+// and leaves one wavefront per block: 1152 longitudes, order 3, 113 levels 325 us
+// direct and 429, 1536, order 2, 397 and 468.  With two wavefronts the table wins
+// (1024, order 3, 113 levels 176 us; 355 for a table per three levels of one).
 inline bool table_fits(int nlon, int order, int wl, int *waves) {
   const size_t tab = sizeof(double) * 2 * (size_t)order * nlon, per = sizeof(double) * wl;
   int W = kWaves;
-  while (W > 1 && tab + W * per > kLdsMax) W >>= 1;
+  while (W > 2 && tab + W * per > kLdsMax) W >>= 1;
   if (waves) *waves = W;
   return tab + W * per <= kLdsMax;
 }
@@ -469,7 +473,7 @@ inline bool table_fits(int nlon, int order, int wl, int *waves) {
 template <int NPL>
 int launch(const Fields &P, int nkp, long plane, int nrows, const Rows &R, int nlon, int order, int oplus,
            double dlamda, const double *gtab, int tord, hipStream_t s) {
-  int W, maxc = 1;
+  int W = 1, maxc = 1;
   for (int r = 0; r < nrows; ++r) maxc = R.n[r] > maxc ? R.n[r] : maxc;
   const int wl = wave_doubles(nlon, maxc);
   if (gtab) {
