@@ -850,9 +850,12 @@ extern "C" int tgx_ng_step(const tgx_ng_grid *g, const tgx_ng_fields *in, const 
   // end of each step, and a nested outer step (one 144x72x57, two 120x60x57 and ten
   // 100x50x57 steps) took 4.99 ms; prelude, O+, dt, minor species, comp: 4.38 (4.00
   // with the block kernels favoured); with a nest's dt first on its own stream
-  // and comp before the minor species, 3.91.  Some 40 orders were tried; steps
-  // outside a graph hardly depend on it.
-  const bool early = !few && !t_glb;
+  // and comp before the minor species, 3.91.  Some 40 orders were tried.
+  // On nests that fill the chip for long a dt beside the chemistry pass only takes
+  // bandwidth from it (eager steps with it and without, us: 150x100x57 733 and 775,
+  // 250x150x40 1,169 and 1,240, 300x200x57 (3.5 million points) 2,387 and 2,418;
+  // 300x150x113 (5.4 million) 3,728 and 3,603, 400x300x57 4,476 and 4,411).
+  const bool early = !few && !t_glb && (long)(g->nlon + 4) * (g->nlat + 4) * g->nk < 3600000;
   std::optional<ProfScope> minors(std::in_place, R_MINORS, sb);
   if (int rc = run_minors(g, in, out, work, sb, true, PART_PRELUDE)) return rc;
   if (early) {
