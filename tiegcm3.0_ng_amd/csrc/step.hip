@@ -4677,9 +4677,14 @@ __global__ void __launch_bounds__(256) duv_tile_kernel(tgx_ng_grid g, Geo G, tgx
 }
 
 // duv_ng stage 2 with one wavefront per column: the 2x2 block rows 0..nk-2 by
-// block cyclic reduction, the top level extrapolated (:250).
+// block cyclic reduction, the top level extrapolated (:250).  Two rows per lane are
+// held to three wavefronts per SIMD: the registers leave room for a fourth, whose
+// loads of 8 bytes of each of 64 lines push the others' lines out of L2 (PCR,
+// 154x104x113 columns 393 us with four and 365 with three, 204x124x100 502 and 462,
+// 254x154x113 877 and 782; 104x54x113 143 and 148).
 template <int NH>
-__global__ void __launch_bounds__(256) duv_wave_stage2(tgx_ng_grid g, Geo G, tgx_ng_fields in,
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NH == 2 ? 3 : 4, NH == 2 ? 3 : 8)))
+duv_wave_stage2(tgx_ng_grid g, Geo G, tgx_ng_fields in,
                                                        tgx_ng_out out, UvTerms UT) {
   int i, j;
   if (!wave_column_of(G, i, j)) return;
