@@ -135,8 +135,8 @@ inline int wave_doubles(int nlon, int maxc) {
 // next level's loads in flight let the compiler hold each longitude's chunk
 // geometry across levels, 247 VGPRs, two wavefronts per SIMD).  One component
 // at 0.625 deg, order 3: 83.9 us, 1.0 TB/s of its rows, before (LDS shuffles
-// for the sums, a block barrier per level, four divisions by 12 per point); 44.4
-// us, 1.9 TB/s, now.  2.5 deg 21.9 -> 10.7 us, 5 deg 20.4 -> 10.6 us.
+// for the sums, a block barrier per level, four divisions by 12 per point); 44.0
+// us by the profiler, 1.9 TB/s, now (40 per launch in a row of launches).  2.5 deg 21.9 -> 10.7 us, 5 deg 20.4 -> 10.6 us.
 template <int NPL, bool GTAB, int MO>
 __device__ __forceinline__ void ringfilter_body(const Fields &P, long plane, const Rows &R, int nlon, int nkp,
                                                 int order, int oplus, double dlamda, int wl,

@@ -7,8 +7,9 @@
 // which leaves one row per lane; the S of them are solved by cyclic reduction
 // across the lanes, and the lane's other rows follow by substitution.
 //
-// What bounds it: HBM for scalar rows; for block rows the FP64 arithmetic of
-// the one or two wavefronts per SIMD that their registers leave room for.
+// What bounds it: HBM for scalar rows; for block rows chains of dependent FP64
+// instructions in the one or two wavefronts per SIMD that their registers leave
+// room for (the VALU busy 42% of the time on 2x2 rows, 27% on 3x3).
 // Every coefficient is read once and every unknown written once.  A thread per
 // column, or a wavefront per column reduced row by row (the solvers before),
 // kept ratios or block gammas in HBM between two sweeps, read each array with
@@ -17,9 +18,9 @@
 // loads in flight at once, and turns each array round through LDS to the lanes
 // that own the rows (one padding double per lane makes the stride odd: no bank
 // conflicts).  Measured, before and after (a plain copy moves 4.9 TB/s):
-//   scalar, 165,888 columns x 112 rows   359 ->  149 us (5.0 TB/s)
-//   2x2,     41,472 columns x 112 rows   755 ->  168 us (3.5 TB/s)
-//   3x3,     10,368 columns x  56 rows   475 ->   78 us (2.0 TB/s)
+//   scalar, 165,888 columns x 112 rows   359 ->  148 us (5.0 TB/s)
+//   2x2,     41,472 columns x 112 rows   755 ->  146 us (4.1 TB/s)
+//   3x3,     10,368 columns x  56 rows   475 ->   76 us (2.0 TB/s)
 // Staging whole columns in LDS instead of registers: 206, 418 and 149 us (two
 // to five wavefronts per CU).
 //
@@ -30,7 +31,8 @@
 // and 165,888 columns: 5.3, 6.4 and 32 us against 7.6, 8.4 and 40 with M = 8; 56
 // rows, 2,592 and 41,472: 4.5 and 17 us against 6.1 and 19), beyond that M = 8,
 // where DPP no longer reaches across a column of M = 4.  2x2 rows at M = 4 just fit two
-// wavefronts per SIMD (113 levels: 168 us, 190 with M = 2); up to 32 rows
+// wavefronts per SIMD (113 levels, before the limits on multipliers were one
+// comparison each: 168 us, 190 with M = 2); up to 32 rows
 // M = 2 fits three (43 us against 48, 41,472 x 28).  3x3 rows at M = 4 use
 // every register of a SIMD (56 rows: 78 us, 118 with M = 2), up to 32 rows
 // M = 2 is as fast (41 and 48 us) and faster on few columns (14 and 23).
