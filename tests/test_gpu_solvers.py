@@ -467,6 +467,29 @@ def test_partitioned_solver_growing_segments(pkg, oracle, nblk, n):
     assert err[0].max() <= 8. * err[1].max(), (what[worst], err[0].max(), err[1].max())
 
 
+@pytest.mark.parametrize("n", [56, 65, 112, 128, 200, 256])
+def test_partitioned_solver_slowly_refined_columns(pkg, oracle, n):
+    """One pivot of 1e-2.5 to 1 in eight rows: multipliers compound to 1e10 and
+    more, so that a correction tells little of the next.  The last one is within
+    1e-13 of the unknowns, and what the reference's order solves has its error."""
+    k, nc = np.arange(n) % 8, 256
+    g = np.logspace(0., 2.5, nc)[:, None]
+    A = np.where((k == 0) | (k == 7), 1., 1. / g)
+    B = np.where(k == 0, 1. / g, np.where(k == 7, 2.5, 1. + 1. / g))
+    C, F = np.ones((nc, n)), np.random.default_rng(n).standard_normal((nc, n))
+    B[:, 0] = 2.
+    A[:, 0] = C[:, -1] = 0.
+    A, B, C, F = (v.reshape(nc, n, 1, 1) for v in (A, B, C, F))
+    F = F[..., 0]
+    exact = _refined(A, B, C, F)
+    scale = np.abs(exact).max(axis=(1, 2))
+    y = np.zeros((nc, n))
+    oracle.trsolv_ng(*(np.ascontiguousarray(v[..., 0, 0]) for v in (A, B, C)), np.ascontiguousarray(F[..., 0]), y, n, nc, n)
+    err = [(np.abs(v - exact).max(axis=(1, 2)) / scale).astype(np.float64)
+           for v in (_device_segments(pkg, 1, A, B, C, F), y[..., None])]
+    assert err[0].max() <= 1e-13 + err[1].max(), (g[int(np.argmax(err[0])), 0], err[0].max(), err[1].max())
+
+
 @pytest.mark.parametrize("nblk", [1, 2, 3])
 @pytest.mark.parametrize("n", [28, 56, 112, 200])
 def test_partitioned_solver_in_place(pkg, nblk, n):

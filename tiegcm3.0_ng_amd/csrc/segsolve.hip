@@ -284,18 +284,23 @@ __device__ __noinline__ void serial_column(const double *A, const double *B, con
 // by a decade per row; 1e-11 where a segment lost five digits.
 constexpr double CORRECTION = 1e-12;
 // A badly pivoted column is refined: the same elimination solves for the
-// residual, which is computed in 64 bits from the rows themselves, until a
-// correction is within REFINED of the unknowns, so that what it leaves
-// (its own relative error squared) is below rounding.  At most REFINEMENTS
+// residual, which is computed in 64 bits from the rows themselves.  A first
+// correction within REFINED of the unknowns shows that the elimination keeps
+// eight digits, so that what it leaves is below rounding.  A later one shows
+// less (each correction is an elimination's error further down, and where
+// products of multipliers pass 1e10 that error stops falling as rounding itself is
+// multiplied), so it has to be within SETTLED.  With 1e-8 for those too, pivots of
+// 1e-2 in segments of eight rows kept errors of 3e-12; now 6e-14 at most (reduced
+// row by row 8e-14, the reference's order 2e-14).  At most REFINEMENTS
 // times, then in the reference's order by one lane, as where a pivot
 // vanished and nothing finite came out.  Emulated on the families above, one
 // pass suffices but for multipliers of 20 and more over eight rows (two) and 1
 // in 100 random 3x3 columns (three); the error is 0.2 to 0.9 times that of the
 // reference's order.  One lane per column for all of them instead: scalar
 // 165,888 x 112, every column bad, 1,280 us; 2x2 41,472 x 112 1,660; 3x3 10,368 x
-// 56 520; refined 361, 259 and 137 (a wavefront per column reduced row by row, or a
+// 56 520; refined 361, 257 to 285 and 136 (a wavefront per column reduced row by row, or a
 // thread per column, took 355, 577 and 337).
-constexpr double REFINED = 1e-8;
+constexpr double REFINED = 1e-8, SETTLED = 1e-13;
 constexpr int REFINEMENTS = 3;
 
 // The rows of a block's nc columns, column c0 the first: 64 consecutive doubles
@@ -448,7 +453,7 @@ __device__ __forceinline__ void refine_columns(const double *a, const double *b,
       const double big = largest(solved(e - 1), here, solved(e + 1));
 #pragma unroll
       for (int q = 0; q < N; ++q) {
-        bad |= !(fabs(d[e].v[q]) <= REFINED * big);
+        bad |= !(fabs(d[e].v[q]) <= (pass ? SETTLED : REFINED) * big);
         d[e].v[q] = here.v[q] + d[e].v[q];
         lost |= !(fabs(d[e].v[q]) <= 1.e300);
       }
